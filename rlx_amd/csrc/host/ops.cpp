@@ -1088,7 +1088,8 @@ struct TopkArgs {  // mirrors kernels/topk.hip
     uint32_t *out_idx;
     float *out_val;
 };
-constexpr int64_t TOPK_GROUP = 1024;  // candidates one wave reduces to `cap`
+constexpr int64_t TOPK_GROUP = 1024;   // candidates one wave of rlx_topk_select reduces to `cap`
+constexpr int64_t TOPK_FINISH = 8192;  // candidates rlx_topk_finish takes
 constexpr int TOPK_MAX_CAP = 64;
 static int64_t topk_groups(int64_t n) { return (n + TOPK_GROUP - 1) / TOPK_GROUP; }
 }  // namespace rlx
@@ -1127,20 +1128,20 @@ static int tied_lm_topk(const char *who, const void *hidden_dev, int xk, const r
     const rlx_qweight *ws[1] = {embed};
     float *outs[1] = {logits};
     RLX_TRY(launch_gemv(xs, xk, ws, outs, 1, 1, (hipStream_t)stream, nullptr, nullptr, nullptr, norm));
-    // every pass: one wave per 1024 candidates keeps its cap best; the pass with a single wave writes the answer
+    // One workgroup orders up to TOPK_FINISH candidates; more than that first lose all but the cap best of every 1024.
     int64_t count = n;
     int side = 0;
-    for (bool first = true;; first = false) {
+    bool first = true;
+    for (; count > TOPK_FINISH; first = false, side ^= 1) {
         const int64_t groups = topk_groups(count);
-        const bool last = groups == 1;
-        TopkArgs p{first ? logits : nullptr, first ? nullptr : keys[side ^ 1], (int)count, cap, last ? nullptr : keys[side],
-                   last ? out_idx_dev : nullptr, last ? out_val_dev : nullptr};
+        TopkArgs p{first ? logits : nullptr, first ? nullptr : keys[side ^ 1], (int)count, cap, keys[side], nullptr, nullptr};
         void *params[] = {&p};
         RLX_TRY(launch(K_TOPK_SELECT, (unsigned)groups, 1, 64, 0, (hipStream_t)stream, params));
-        if (last) break;
         count = groups * cap;
-        side ^= 1;
     }
+    TopkArgs p{first ? logits : nullptr, first ? nullptr : keys[side ^ 1], (int)count, cap, nullptr, out_idx_dev, out_val_dev};
+    void *params[] = {&p};
+    RLX_TRY(launch(K_TOPK_FINISH, 1, 1, 1024, 0, (hipStream_t)stream, params));
     return RLX_OK;
 }
 

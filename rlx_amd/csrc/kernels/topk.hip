@@ -1,18 +1,23 @@
 // Top-k over the logits of the tied LM head: rlx_cpu::lm_head::gguf_tied_lm_topk (rlx-cpu/src/lm_head.rs:172-198) and
 // topk_from_scores (:130-141) keep the `cap` largest (token, logit) pairs, largest first. The reference visits the
-// rows one after another against a rising floor; here the decode kernel writes all logits and a few selection passes
-// follow, all the same kernel: one wave holds up to 1024 candidates as (value, row) keys in registers, sixteen per lane,
-// sorted once per lane; it takes the wave-wide maximum of the lanes' heads `cap` times and the lane that held the winner
-// moves its list up by one - no LDS, no barrier. The wave-wide maximum of the 64-bit keys is two 32-bit reductions (the
-// value, then the row among the lanes that hold that value), each four row-local DPP steps and four lane reads. The first
-// pass turns every 1024 logits into their `cap` best, each further pass does the same to 1024 of the survivors, until
-// one wave is left; that one writes rows and values. Keys order as in the argmax: larger value first, among equal
-// values the smaller row; a NaN logit is no candidate.
+// rows one after another against a rising floor; here the decode kernel writes all logits and a selection over
+// (value, row) keys follows. Keys order as in the argmax: larger value first, among equal values the smaller row; a NaN
+// logit is no candidate; every key is unique, so "the cap-th largest" is one key.
+//
+// Neither kernel takes the winners one by one (cap rounds of a wave-wide maximum, each waiting for the one before, were
+// 12 - 17 us a launch): both find a threshold by bisection over the bits of the key, a count per step, and only the last
+// kernel puts the few survivors in order, every survivor counting the keys above its own.
+//   rlx_topk_select  one wave per 1024 candidates, sixteen per lane, leaves their `cap` best in any order. No LDS, no barrier.
+//   rlx_topk_finish  one workgroup, up to 8192 candidates, eight per thread: writes rows and values, largest first.
+// Both are bound by latency (launch, one load, the chain of counts), not by bandwidth: 128256 logits are 0.5 MB. The whole
+// LM-head call at [128256, 4096] Q4_K, cap 40: 93.3 -> 71.6 us, 57 of it the matmul.
 #include "common.h"
 
 namespace rlx {
 
-constexpr int TOPK_PER_LANE = 16, TOPK_GROUP = 64 * TOPK_PER_LANE;  // candidates per wave
+constexpr int TOPK_PER_LANE = 16, TOPK_GROUP = 64 * TOPK_PER_LANE;       // candidates per wave of rlx_topk_select
+constexpr int TOPK_PER_THREAD = 8, TOPK_FINISH = 1024 * TOPK_PER_THREAD;  // candidates rlx_topk_finish takes
+constexpr int TOPK_SURVIVORS = 128;                                       // keys it puts in order (cap <= 64)
 
 __device__ __forceinline__ unsigned long long topk_key_of(float v, uint32_t row) {
     const uint32_t b = __builtin_bit_cast(uint32_t, v + 0.0f);  // -0 and +0 compare equal
@@ -20,27 +25,41 @@ __device__ __forceinline__ unsigned long long topk_key_of(float v, uint32_t row)
     return ((unsigned long long)ordered << 32) | (uint32_t)~row;
 }
 
-// Maximum over the 64 lanes, returned in a scalar register: four DPP steps leave every row of 16 lanes with its maximum, four
-// lane reads and three scalar maxima finish it.
-__device__ __forceinline__ uint32_t wave_max_u32(uint32_t v) {
-    v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0xB1, 0xF, 0xF, true));   // quad_perm [1,0,3,2]
-    v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x4E, 0xF, 0xF, true));   // quad_perm [2,3,0,1]
-    v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x141, 0xF, 0xF, true));  // row_half_mirror
-    v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x140, 0xF, 0xF, true));  // row_mirror
+// Reduction over the 64 lanes, returned in a scalar register: four DPP steps leave every row of 16 lanes with its result,
+// four lane reads and three scalar operations finish it.
+template <typename Op>
+__device__ __forceinline__ uint32_t wave_reduce_u32(uint32_t v, Op op) {
+    v = op(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0xB1, 0xF, 0xF, true));   // quad_perm [1,0,3,2]
+    v = op(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x4E, 0xF, 0xF, true));   // quad_perm [2,3,0,1]
+    v = op(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x141, 0xF, 0xF, true));  // row_half_mirror
+    v = op(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x140, 0xF, 0xF, true));  // row_mirror
     const uint32_t r0 = (uint32_t)__builtin_amdgcn_readlane((int)v, 0), r1 = (uint32_t)__builtin_amdgcn_readlane((int)v, 16);
     const uint32_t r2 = (uint32_t)__builtin_amdgcn_readlane((int)v, 32), r3 = (uint32_t)__builtin_amdgcn_readlane((int)v, 48);
-    return max(max(r0, r1), max(r2, r3));
+    return op(op(r0, r1), op(r2, r3));
+}
+__device__ __forceinline__ uint32_t wave_max_u32(uint32_t v) {
+    return wave_reduce_u32(v, [](uint32_t x, uint32_t y) { return max(x, y); });
+}
+__device__ __forceinline__ uint32_t wave_min_u32(uint32_t v) {
+    return wave_reduce_u32(v, [](uint32_t x, uint32_t y) { return min(x, y); });
 }
 
 struct TopkArgs {
     const float *vals;                  // first pass: [n] logits; null afterwards
     const unsigned long long *keys_in;  // later passes: [n] keys, zero = no candidate
-    int n;                              // candidates in all; workgroup g takes [g * TOPK_GROUP, (g + 1) * TOPK_GROUP)
+    int n;                              // candidates in all; wave g of rlx_topk_select takes [g * TOPK_GROUP, (g + 1) * TOPK_GROUP)
     int cap;
-    unsigned long long *keys_out;       // all but the last pass: [workgroups][cap] keys
-    uint32_t *out_idx;                  // last pass (one workgroup): [cap] rows and values; (0, -inf) where no candidate is left
+    unsigned long long *keys_out;       // rlx_topk_select: [waves][cap] keys
+    uint32_t *out_idx;                  // rlx_topk_finish: [cap] rows and values; (0, -inf) where no candidate is left
     float *out_val;
 };
+
+__device__ __forceinline__ unsigned long long topk_load(const TopkArgs &a, long long i) {
+    if (i >= a.n) return 0;
+    if (!a.vals) return a.keys_in[i];
+    const float v = a.vals[i];
+    return v == v ? topk_key_of(v, (uint32_t)i) : 0;
+}
 
 }  // namespace rlx
 
@@ -48,57 +67,129 @@ extern "C" __global__ __launch_bounds__(64) void rlx_topk_select(rlx::TopkArgs a
     using namespace rlx;
     const int lane = threadIdx.x;
     const long long base = (long long)blockIdx.x * TOPK_GROUP;
-    const int count = (int)min((long long)TOPK_GROUP, (long long)a.n - base);
     unsigned long long mine[TOPK_PER_LANE];
 #pragma unroll
-    for (int e = 0; e < TOPK_PER_LANE; e++) {
-        const int i = lane + e * 64;
-        unsigned long long k = 0;
-        if (i < count) {
-            if (a.vals) {
-                const float v = a.vals[base + i];
-                if (v == v) k = topk_key_of(v, (uint32_t)(base + i));
-            } else {
-                k = a.keys_in[base + i];
-            }
-        }
-        mine[e] = k;
+    for (int e = 0; e < TOPK_PER_LANE; e++) mine[e] = topk_load(a, base + lane + e * 64);
+    uint32_t best = 0;
+#pragma unroll
+    for (int e = 0; e < TOPK_PER_LANE; e++) best = max(best, (uint32_t)(mine[e] >> 32));
+    // The lanes' own maxima bound the threshold: at least 64 >= cap keys reach the smallest of them, none passes the
+    // largest, so the bits the two share are decided.
+    const uint32_t top = wave_max_u32(best), low = wave_min_u32(best);
+    unsigned long long t = 0;  // the largest value with at least cap keys >= t (0: fewer than cap candidates, take them all)
+    const int bits = top == low ? 32 : 64 - __builtin_clz(top ^ low);  // undecided low bits of t
+    if (bits < 64) t = (unsigned long long)top << 32 >> bits << bits;
+    for (int bit = bits - 1; bit >= 0; bit--) {
+        const unsigned long long trial = t | (1ull << bit);
+        int count = 0;
+#pragma unroll
+        for (int e = 0; e < TOPK_PER_LANE; e++) count += __builtin_popcountll(__ballot(mine[e] >= trial));
+        if (count >= a.cap) t = trial;
+        if (count == a.cap) break;
     }
-    // this lane's candidates in descending order (bitonic network over registers: every index is a constant)
+    if (t == 0) t = 1;  // an absent candidate is key 0
+    int at = 0;
 #pragma unroll
-    for (int k = 2; k <= TOPK_PER_LANE; k <<= 1)
+    for (int e = 0; e < TOPK_PER_LANE; e++) {
+        const bool take = mine[e] >= t;
+        const unsigned long long who = __ballot(take);
+        const int pos = at + __builtin_popcountll(who & ((1ull << lane) - 1ull));
+        if (take) a.keys_out[(long long)blockIdx.x * a.cap + pos] = mine[e];
+        at += __builtin_popcountll(who);
+    }
+    if (at + lane < a.cap) a.keys_out[(long long)blockIdx.x * a.cap + at + lane] = 0;
+}
+
+extern "C" __global__ __launch_bounds__(1024) void rlx_topk_finish(rlx::TopkArgs a) {
+    using namespace rlx;
+    __shared__ uint32_t wave_hi[16], wave_lo[16];
+    __shared__ uint32_t counts[2][3][16];                      // [step parity][trial][wave]
+    __shared__ unsigned long long survivors[TOPK_SURVIVORS];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    unsigned long long mine[TOPK_PER_THREAD];
 #pragma unroll
-        for (int j = k >> 1; j > 0; j >>= 1)
+    for (int e = 0; e < TOPK_PER_THREAD; e++) mine[e] = topk_load(a, tid + e * 1024);
+    uint32_t best = 0;
 #pragma unroll
-            for (int i = 0; i < TOPK_PER_LANE; i++) {
-                const int l = i ^ j;
-                if (l > i) {
-                    const unsigned long long x = mine[i], y = mine[l];
-                    const bool desc = (i & k) == 0;  // descending runs first, so the last merge leaves the whole list descending
-                    const bool swap = desc ? (x < y) : (x > y);
-                    mine[i] = swap ? y : x;
-                    mine[l] = swap ? x : y;
-                }
-            }
-    for (int r = 0; r < a.cap; r++) {
-        const uint32_t hi = (uint32_t)(mine[0] >> 32), lo = (uint32_t)mine[0];
-        const uint32_t whi = wave_max_u32(hi);
-        const uint32_t wlo = wave_max_u32(hi == whi ? lo : 0u);  // keys are unique (they carry the row): one lane matches both
-        const unsigned long long win = ((unsigned long long)whi << 32) | wlo;
-        if (win != 0 && mine[0] == win) {  // the lane that held the winner moves its list up
+    for (int e = 0; e < TOPK_PER_THREAD; e++) best = max(best, (uint32_t)(mine[e] >> 32));
+    if (tid < TOPK_SURVIVORS) survivors[tid] = 0;
+    // As above, with the maxima of the 64 rows of 16 lanes: every one of them is a key, so 64 >= cap keys reach the smallest.
+    uint32_t rowbest = best;
+    rowbest = max(rowbest, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)rowbest, 0xB1, 0xF, 0xF, true));
+    rowbest = max(rowbest, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)rowbest, 0x4E, 0xF, 0xF, true));
+    rowbest = max(rowbest, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)rowbest, 0x141, 0xF, 0xF, true));
+    rowbest = max(rowbest, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)rowbest, 0x140, 0xF, 0xF, true));
+    const uint32_t wtop = wave_max_u32(best), wlow = wave_min_u32(rowbest);
+    if (lane == 0) {
+        wave_hi[wave] = wtop;
+        wave_lo[wave] = wlow;
+    }
+    __syncthreads();
+    const uint32_t top = wave_max_u32(wave_hi[lane & 15]), low = wave_min_u32(wave_lo[lane & 15]);
+    // t: at least cap keys are >= t; two bits a step, until no more than TOPK_SURVIVORS keys are left. Keys are unique,
+    // so the end of the bits is the end of the search at the latest.
+    int bits = top == low ? 32 : 64 - __builtin_clz(top ^ low);  // undecided low bits of t
+    bits = (bits + 1) & ~1;
+    unsigned long long t = bits >= 64 ? 0 : (unsigned long long)top << 32 >> bits << bits;
+    bool done = false;
+    for (int step = 0; bits > 0 && !done; step++) {
+        bits -= 2;
 #pragma unroll
-            for (int e = 0; e + 1 < TOPK_PER_LANE; e++) mine[e] = mine[e + 1];
-            mine[TOPK_PER_LANE - 1] = 0;
+        for (int q = 1; q <= 3; q++) {
+            const unsigned long long trial = t | ((unsigned long long)q << bits);
+            int c = 0;
+#pragma unroll
+            for (int e = 0; e < TOPK_PER_THREAD; e++) c += __builtin_popcountll(__ballot(mine[e] >= trial));
+            if (lane == 0) counts[step & 1][q - 1][wave] = (uint32_t)c;
         }
-        if (lane == 0) {
-            if (a.keys_out) {
-                a.keys_out[(long long)blockIdx.x * a.cap + r] = win;
-            } else {
-                const uint32_t ordered = (uint32_t)(win >> 32);
-                const uint32_t b = (ordered & 0x80000000u) ? (ordered & 0x7FFFFFFFu) : ~ordered;
-                a.out_idx[r] = win ? ~(uint32_t)win : 0u;
-                a.out_val[r] = win ? __builtin_bit_cast(float, b) : -__builtin_inff();
+        __syncthreads();  // the other parity is written next: a wave still reading this one is not overtaken
+        const unsigned long long t0 = t;
+#pragma unroll
+        for (int q = 1; q <= 3; q++) {  // counts fall with q
+            const uint32_t c = wave_reduce_u32(lane < 16 ? counts[step & 1][q - 1][lane] : 0u, [](uint32_t x, uint32_t y) { return x + y; });
+            if (c >= (uint32_t)a.cap) {
+                t = t0 | ((unsigned long long)q << bits);
+                done = c <= (uint32_t)TOPK_SURVIVORS;
             }
         }
+    }
+    if (t == 0) t = 1;
+    // survivors, in any order: every wave counts its own, takes its place among the waves, writes
+    int c = 0;
+#pragma unroll
+    for (int e = 0; e < TOPK_PER_THREAD; e++) c += __builtin_popcountll(__ballot(mine[e] >= t));
+    __syncthreads();
+    if (lane == 0) wave_hi[wave] = (uint32_t)c;
+    __syncthreads();
+    int at = (int)wave_reduce_u32(lane < wave ? wave_hi[lane & 15] : 0u, [](uint32_t x, uint32_t y) { return x + y; });
+#pragma unroll
+    for (int e = 0; e < TOPK_PER_THREAD; e++) {
+        const bool take = mine[e] >= t;
+        const unsigned long long who = __ballot(take);
+        const int pos = at + __builtin_popcountll(who & ((1ull << lane) - 1ull));
+        if (take && pos < TOPK_SURVIVORS) survivors[pos] = mine[e];
+        at += __builtin_popcountll(who);
+    }
+    __syncthreads();
+    // rank = keys above; eight neighbouring threads share a survivor, sixteen comparisons each
+    const unsigned long long key = survivors[tid >> 3];
+    uint32_t above = 0;
+#pragma unroll
+    for (int i = 0; i < TOPK_SURVIVORS / 8; i++) above += survivors[i * 8 + (tid & 7)] > key ? 1u : 0u;
+    above += (uint32_t)__shfl_xor((int)above, 1);
+    above += (uint32_t)__shfl_xor((int)above, 2);
+    above += (uint32_t)__shfl_xor((int)above, 4);
+    if ((tid & 7) == 0 && key != 0 && above < (uint32_t)a.cap) {
+        const uint32_t ordered = (uint32_t)(key >> 32);
+        const uint32_t b = (ordered & 0x80000000u) ? (ordered & 0x7FFFFFFFu) : ~ordered;
+        a.out_idx[above] = ~(uint32_t)key;
+        a.out_val[above] = __builtin_bit_cast(float, b);
+    }
+    // fewer candidates than cap: the rest of the list
+    const int total = (int)wave_reduce_u32(lane < 16 ? wave_hi[lane] : 0u, [](uint32_t x, uint32_t y) { return x + y; });
+    if (tid >= total && tid < a.cap) {
+        a.out_idx[tid] = 0u;
+        a.out_val[tid] = -__builtin_inff();
     }
 }

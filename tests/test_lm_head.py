@@ -254,3 +254,21 @@ def test_topk_and_argmax_at_llama3_vocabulary_size():
         assert np.array_equal(idx, want_idx) and np.array_equal(val.view(np.uint32), want_val.view(np.uint32)), cap
     assert ops.gguf_tied_lm_argmax(hidden, w) == (int(want_idx[0]), float(want_val[0]))
     w.free()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,cap", [(1, 1), (63, 63), (1025, 64), (8192, 40), (8193, 1), (8193, 64), (140000, 64)])
+@pytest.mark.parametrize("distinct", [False, True])
+def test_topk_selection_edges_on_device(n, cap, distinct):
+    # Both sides of what the finishing workgroup takes in one go (8192 candidates), a second selection pass (140000 rows leave
+    # 137 x 64 keys), and bulk ties: with three different rows in all, every cut goes through equal values.
+    rng = np.random.default_rng(n + cap)
+    rows = ops.quantize(QuantScheme.GgufQ4_0, rng.standard_normal((n if distinct else 3, 32)).astype(np.float32)).reshape(-1, 18)
+    packed = rows if distinct else rows[rng.integers(0, 3, n)]
+    w = ops.QWeight(QuantScheme.GgufQ4_0, np.ascontiguousarray(packed).reshape(-1), n, 32)
+    hidden = rng.standard_normal(32).astype(np.float32)
+    logits = ops.gguf_matmul_bt(hidden.reshape(1, 32), w, 1)[0]
+    idx, val = ops.gguf_tied_lm_topk(hidden, w, cap)
+    want_idx, want_val = full_sort_topk(logits, cap)
+    assert np.array_equal(idx, want_idx) and np.array_equal(val.view(np.uint32), want_val.view(np.uint32))
+    w.free()
