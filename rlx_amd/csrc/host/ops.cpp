@@ -102,12 +102,18 @@ struct GemmArgs {
     const int *perm;
     long long slab_bytes;
 };
-struct GemmBigArgs {  // mirrors kernels/gemm_big.hip
-    const void *a_img;
-    const void *b_img;
+struct GemmBigSeg {  // mirrors kernels/gemm_big.hip
+    const void *w;
     float *out;
+    int n, row_tiles, tile_begin;
+};
+struct GemmBigArgs {
+    GemmBigSeg seg[GEMM_MAX_SEG];
+    int nseg;
+    const void *a_img;
     const float *rowfac;
-    int m_out, n, steps;
+    float *part;
+    int m_out, tiles_m, tiles_n, a_steps, quads, pair_rows;
 };
 constexpr int GEMVW_MAX_SEG = 8;
 struct GemvWSeg {  // mirrors kernels/gemv_wide.hip
@@ -411,6 +417,44 @@ static GemmSplit wide_split(const Layout &L, const WeightDims &D, int64_t m, siz
     units_per_split = (units_per_split + 1) / 2 * 2;
     return GemmSplit{(int)((D.units + units_per_split - 1) / units_per_split), units_per_split};
 }
+// The 256 x 256 tiles of kernels/gemm_big.hip (Q4_0, Q8_0, code images) against the 256 x 128 tiles of kernels/gemm.hip, and how the
+// former are handed out: a tile per workgroup, or the whole line of (tile, 128 columns of K) items in equal runs, one per CU, with
+// the pieces of shared tiles added by a launch of their own. `groups` = 0: the 256 x 128 tiles. Estimated times decide, in us, with what
+// was measured on 2222 image rows of f32 activations in Q4_0: 128 columns of a tile cost BIG_QUAD with one workgroup per CU (28672 x
+// 4096: 1008 tiles in four rounds, 480 - 520 us in all) or SMALL_QUAD for half a tile (the same matrix 526); partial results travel
+// at 5 MB / us each way and the launch that adds them costs 4 us. 144 tiles of 4096 x 14336 (386 us as 288 half tiles in two rounds)
+// take 256 us shared out + 16 us for the sum, of 4096 x 4096 96 + 16 against 117.
+struct BigPlan {
+    int groups;
+    size_t part_bytes;
+};
+constexpr double BIG_QUAD = 3.8, BIG_START = 4, SMALL_QUAD = 2.0, PART_BYTES_US = 5e6, REDUCE_US = 4;
+static BigPlan big_plan(int scheme, int xk, int64_t m, int64_t m_rows, int64_t tiles_n, int64_t small_tiles_n, int64_t n_sum, int64_t quads, size_t part_room) {
+    BigPlan none{0, 0};
+    if (scheme != SCHEME_Q4_0 && scheme != SCHEME_Q8_0) return none;
+    const long long cus = device_props().cu_count > 0 ? device_props().cu_count : 256;
+    const long long tiles_m = m_rows / 256, tiles = tiles_m * tiles_n;
+    auto rounds = [&](long long t) { return (double)((t + cus - 1) / cus); };
+    // the 256 x 128 tiles, with the split of K gemm_split gives them
+    const long long small = tiles_m * small_tiles_n;
+    double t_small = rounds(small) * (double)quads * SMALL_QUAD;
+    if (small * 5 < cus * 4) {
+        const long long split = std::min<long long>(quads, cus / small);
+        t_small = t_small / (double)split + 2.0 * 4.0 * (double)split * (double)m * (double)n_sum / PART_BYTES_US + REDUCE_US;
+    }
+    const double t_whole = BIG_START + rounds(tiles) * (double)quads * BIG_QUAD;
+    const size_t tile_bytes = (size_t)(xk == 0 ? 128 : 256) * 1024;
+    const size_t part = (size_t)cus * 2 * tile_bytes;
+    double t_shared = 1e30;
+    if (part <= part_room && tiles * quads >= cus) {
+        // a workgroup leaves at most two pieces; a tile that is not shared leaves none
+        const double pieces = (double)std::min<long long>(2 * cus, cus + tiles);
+        t_shared = BIG_START + (double)((tiles * quads + cus - 1) / cus) * BIG_QUAD + 2.0 * pieces * (double)tile_bytes / PART_BYTES_US + REDUCE_US;
+    }
+    if (std::min(t_whole, t_shared) >= t_small) return none;
+    if (t_shared < t_whole) return BigPlan{(int)cus, part};
+    return BigPlan{(int)tiles, 0};
+}
 static GemmPlan gemm_plan(int scheme, int xk, int64_t m, int64_t k, int64_t n = 0) {
     GemmPlan p;
     const int64_t rv = xk == 0 ? 2 * m : m;
@@ -434,6 +478,7 @@ static GemmPlan gemm_plan(int scheme, int xk, int64_t m, int64_t k, int64_t n = 
         const int64_t k_units = xk == XK_CODES ? p.k_pad / 64 : (k + L.unit_k - 1) / L.unit_k;
         const GemmSplit sp = gemm_split((n + 127) / 128, skinny ? (rv + 63) / 64 : p.m_rows / 256, k_units, spu, skinny);
         if (sp.split > 1) p.part_bytes = (size_t)sp.split * (size_t)m * (size_t)n * 4;
+        if (!skinny) p.part_bytes = std::max(p.part_bytes, big_plan(scheme, xk, m, p.m_rows, (n + 255) / 256, (n + 127) / 128, n, xk == XK_CODES ? p.k_pad / 128 : k_units, SIZE_MAX).part_bytes);
     }
     return p;
 }
@@ -495,14 +540,6 @@ static int launch_gemm(const void *x, int xk, const rlx_qweight *const *ws, floa
         void *wparams[] = {&wa};
         const KernelId wid = w->scheme == SCHEME_Q4_0 ? K_WSCALE_Q4_0 : K_WSCALE_Q8_0;
         RLX_TRY(launch(wid, (unsigned)(p.k_pad / w->layout.unit_k), (unsigned)((w->dims.n + 255) / 256 * 16), 64, 0, stream, wparams));
-        // Many rows: the 256 x 256 tile kernel for ready operands (two rounds of workgroups or more, so that its larger
-        // tile does not leave the chip half empty)
-        const long long big_tiles = (p.m_rows / 256) * ((w->dims.n + 255) / 256);
-        if (big_tiles >= 2LL * std::max(1, device_props().cu_count)) {
-            GemmBigArgs ba{xh, wimg, outs[0], fac, (int)m, (int)w->dims.n, (int)(p.k_pad / 64)};
-            void *bparams[] = {&ba};
-            return launch3(K_GEMM_BIG_F16W, (unsigned)((w->dims.n + 255) / 256), (unsigned)(p.m_rows / 256), 1, 512, 2 * 65536, stream, bparams);
-        }
     } else if (!prepared) {
         RLX_TRY(launch_xprep(x, xk, m, w->dims.k, p, workspace, stream));
     }
@@ -551,6 +588,36 @@ static int launch_gemm(const void *x, int xk, const rlx_qweight *const *ws, floa
                 ra.split[nred++] = sps[i].split;
             }
         return launch_split_reduce(ra, nred, stream);
+    }
+
+    if (!gemm_skinny(xk, m)) {
+        RLX_TRY(runtime_init());
+        GemmBigArgs ba{};
+        int64_t small_n = 0, n_sum = 0;
+        for (int i = 0; i < count; i++) {
+            ba.seg[i] = GemmBigSeg{codes ? (const void *)wimg : ws[i]->dev, outs[i], (int)ws[i]->dims.n, (int)ws[i]->dims.row_tiles, ba.tiles_n};
+            ba.tiles_n += (int)((ws[i]->dims.n + 255) / 256);
+            small_n += (ws[i]->dims.n + 127) / 128;
+            n_sum += ws[i]->dims.n;
+        }
+        ba.quads = codes ? (int)(p.k_pad / 128) : (int)w->dims.units;
+        const BigPlan bp = big_plan(w->scheme, xk, m, p.m_rows, ba.tiles_n, small_n, n_sum, ba.quads, workspace_bytes - ops_end);
+        if (bp.groups) {
+            ba.nseg = count;
+            ba.a_img = xh;
+            ba.rowfac = fac;
+            ba.part = (float *)((uint8_t *)workspace + ops_end);
+            ba.m_out = (int)m;
+            ba.tiles_m = (int)(p.m_rows / 256);
+            ba.a_steps = (int)(p.k_pad / 64);
+            ba.pair_rows = xk == 0 ? 1 : 0;
+            int groups = bp.groups;
+            void *bparams[] = {&ba, &groups};
+            const KernelId bid = codes ? K_GEMM_BIG_F16W : w->scheme == SCHEME_Q4_0 ? K_GEMM_BIG_Q4_0 : K_GEMM_BIG_Q8_0;
+            RLX_TRY(launch(bid, (unsigned)groups, 1, 256, 5 * 32768, stream, bparams));
+            if (!bp.part_bytes) return RLX_OK;
+            return launch(K_GEMM_BIG_REDUCE, (unsigned)(ba.tiles_m * ba.tiles_n), ba.pair_rows ? 8 : 16, 256, 0, stream, bparams);
+        }
     }
 
     const int steps_per_unit = L.unit_k / 64;

@@ -45,20 +45,26 @@ __device__ __forceinline__ uint32_t and_or(uint32_t a, uint32_t mask, uint32_t m
 
 // 4-bit granule word -> four half2 registers holding (q - OFF) for the 8 weights, fragment order.
 // OFF = 8 for Q4_0 (signed codes), 0 for Q4_K. All results are exact integers.
+// q4_magic takes weights 0 - 3 out of the word (4 - 7 out of the word shifted right by 8) as 1024 + q and 1024 + 16 q,
+// q4_signed turns those into q - OFF; kernels that interleave their decode with matrix instructions call them apart.
+__device__ __forceinline__ void q4_magic(uint32_t w, half2_t v[2]) {
+    v[0] = as_half2(and_or(w, 0x000F000Fu, MAGIC));
+    v[1] = as_half2(and_or(w, 0x00F000F0u, MAGIC));
+}
 template <int OFF>
-__device__ __forceinline__ void unpack_q4(uint32_t w, Frag &f) {
+__device__ __forceinline__ void q4_signed(half2_t v[2]) {
     const half2_t sub_lo = {(half_t)(-(1024 + OFF)), (half_t)(-(1024 + OFF))};
     const half2_t mul_hi = {(half_t)0.0625f, (half_t)0.0625f};
     const half2_t sub_hi = {(half_t)(-(64 + OFF)), (half_t)(-(64 + OFF))};
-    uint32_t w2 = w >> 8;
-    half2_t a0 = as_half2(and_or(w, 0x000F000Fu, MAGIC));   // 1024 + q
-    half2_t a1 = as_half2(and_or(w, 0x00F000F0u, MAGIC));   // 1024 + 16 q
-    half2_t a2 = as_half2(and_or(w2, 0x000F000Fu, MAGIC));
-    half2_t a3 = as_half2(and_or(w2, 0x00F000F0u, MAGIC));
-    f.h2[0] = a0 + sub_lo;
-    f.h2[1] = __builtin_elementwise_fma(a1, mul_hi, sub_hi);  // (1024+16q)/16 - 64 - OFF, single rounding of an exact value
-    f.h2[2] = a2 + sub_lo;
-    f.h2[3] = __builtin_elementwise_fma(a3, mul_hi, sub_hi);
+    v[0] = v[0] + sub_lo;
+    v[1] = __builtin_elementwise_fma(v[1], mul_hi, sub_hi);  // (1024+16q)/16 - 64 - OFF, single rounding of an exact value
+}
+template <int OFF>
+__device__ __forceinline__ void unpack_q4(uint32_t w, Frag &f) {
+    q4_magic(w, f.h2);
+    q4_magic(w >> 8, f.h2 + 2);
+    q4_signed<OFF>(f.h2);
+    q4_signed<OFF>(f.h2 + 2);
 }
 
 // Q4_K granule word -> sc * q (exact integers <= 945) given sc as a half2 splat.
@@ -114,18 +120,22 @@ __device__ __forceinline__ void unpack_q5_scaled(uint32_t w, uint32_t hx, half2_
 }
 
 // Q8_0 granule (two words of offset-binary bytes) -> signed codes as halfs, fragment order.
-__device__ __forceinline__ void unpack_q8(uint32_t w0, uint32_t w1, Frag &f) {
-    const half2_t sub = {(half_t)(-1152.0f), (half_t)(-1152.0f)};  // 1024 + 128
+__device__ __forceinline__ void q8_magic(uint32_t w, half2_t v[2]) {  // four bytes -> 1024 + u
     const uint32_t c64 = 0x64646464u;
     // v_perm_b32: selector byte 0..3 picks from the second source, 4..7 from the first.
-    half2_t a0 = as_half2(__builtin_amdgcn_perm(c64, w0, 0x04010400u));  // bytes 0,1
-    half2_t a1 = as_half2(__builtin_amdgcn_perm(c64, w0, 0x04030402u));  // bytes 2,3
-    half2_t a2 = as_half2(__builtin_amdgcn_perm(c64, w1, 0x04010400u));
-    half2_t a3 = as_half2(__builtin_amdgcn_perm(c64, w1, 0x04030402u));
-    f.h2[0] = a0 + sub;
-    f.h2[1] = a1 + sub;
-    f.h2[2] = a2 + sub;
-    f.h2[3] = a3 + sub;
+    v[0] = as_half2(__builtin_amdgcn_perm(c64, w, 0x04010400u));  // bytes 0,1
+    v[1] = as_half2(__builtin_amdgcn_perm(c64, w, 0x04030402u));  // bytes 2,3
+}
+__device__ __forceinline__ void q8_signed(half2_t v[2]) {
+    const half2_t sub = {(half_t)(-1152.0f), (half_t)(-1152.0f)};  // 1024 + 128
+    v[0] = v[0] + sub;
+    v[1] = v[1] + sub;
+}
+__device__ __forceinline__ void unpack_q8(uint32_t w0, uint32_t w1, Frag &f) {
+    q8_magic(w0, f.h2);
+    q8_magic(w1, f.h2 + 2);
+    q8_signed(f.h2);
+    q8_signed(f.h2 + 2);
 }
 
 // Q4_K: the eight 6-bit (scale, min) pairs of a super-block from its 12 packed bytes held in three words,

@@ -1,0 +1,71 @@
+"""The 256 x 256 tile prefill kernel (csrc/kernels/gemm_big.hip): tiles handed out whole and shared between workgroups, ragged rows, columns
+and K, f32 and 16-bit activations, several matrices in one launch. Sizes are the smallest at which the dispatch takes it."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+import rlx_amd
+from helpers import Q4_0, Q8_0, f32_to_bf16_bits, rel_err
+from rlx_amd import DType, QuantScheme, ops
+from test_bench_launches import tiled_packed
+
+pytestmark = pytest.mark.gpu
+TOL = 2e-3  # the matmul's bound: one rounding of d * code to binary16 per weight
+
+
+def run(scheme, m, ns, k, x_dtype, seed, lean=False, offset=0):
+    rng = np.random.default_rng(seed)
+    x = rng.standard_normal((m, k)).astype(np.float32)
+    x[3] *= 3e4  # a row whose values are carried with a power of two
+    bits = f32_to_bf16_bits(x)
+    if x_dtype == DType.BF16:
+        x = (bits.astype(np.uint32) << 16).view(np.float32)
+    packs = [tiled_packed(scheme, n, k, seed + i, 0.02).reshape(-1) for i, n in enumerate(ns)]
+    ws = [ops.QWeight(QuantScheme(scheme), p, n, k) for p, n in zip(packs, ns)]
+    L = rlx_amd._lib.lib()
+    need = sum(L.rlx_mi355x_gguf_matmul_workspace(scheme, int(x_dtype), m, k, 0 if lean else n) for n in ns)
+    wsb, xd = ops.DeviceBuffer(need), ops.DeviceBuffer.from_numpy(bits if x_dtype == DType.BF16 else x)
+    outs = [ops.DeviceBuffer(m * n * 4 + 16) for n in ns]
+    xp = (C.c_void_p * len(ns))(*[xd.ptr] * len(ns))
+    wp = (C.c_void_p * len(ns))(*[w.ptr for w in ws])
+    op = (C.c_void_p * len(ns))(*[o.ptr + offset for o in outs])
+    got = []
+    for _ in range(2):
+        rlx_amd._lib.check(L.rlx_mi355x_gguf_matmul_bt_batch(xp, int(x_dtype), wp, op, len(ns), m, wsb.ptr, need, None))
+        ops.sync()
+        got.append([o.to_numpy(np.float32)[offset // 4:offset // 4 + m * n].reshape(m, n) for o, n in zip(outs, ns)])
+    for a, b in zip(*got):
+        assert np.array_equal(a.view(np.uint32), b.view(np.uint32))
+    for w in ws:
+        w.free()
+    return x, packs, got[0]
+
+
+@pytest.mark.parametrize("scheme,m,ns,k,x_dtype,offset", [
+    (Q4_0, 1111, [4100], 4096, DType.F32, 0),          # shared tiles, ragged rows and columns
+    (Q8_0, 1100, [4093], 4128, DType.F32, 0),          # odd columns: no 16-byte stores; K ends inside a 128-column unit of the image
+    (Q4_0, 1111, [4096], 4096, DType.F32, 4),          # an output that is only 4-byte aligned
+    (Q8_0, 2050, [6143], 4064, DType.BF16, 0),         # a tile per workgroup, 16-bit rows
+    (Q4_0, 1090, [4096, 1030, 1024], 4096, DType.F32, 0),  # three matrices side by side
+    (Q8_0, 2050, [3900], 8192, DType.BF16, 0),         # shared tiles, 16-bit rows
+])
+def test_large_tiles_match_the_oracle(oracle, scheme, m, ns, k, x_dtype, offset):
+    x, packs, got = run(scheme, m, ns, k, x_dtype, m + k, offset=offset)
+    rows = [0, 1, 2, 127, 128, 255, 256, m // 2, m - 2, m - 1]
+    for p, n, y in zip(packs, ns, got):
+        assert rel_err(y[rows], oracle.gguf_matmul_f64(x[rows], p, len(rows), k, n, scheme)) <= TOL
+        # the scaled row, and every other row through the sum of them all: a weight's rounding is 2^-12 of it at most
+        rest = np.delete(x.astype(np.float64), 3, 0).sum(0, keepdims=True)
+        for part, mine in ((x[3:4], y[3].astype(np.float64)), (rest.astype(np.float32), np.delete(y.astype(np.float64), 3, 0).sum(0))):
+            want = oracle.gguf_matmul_f64(part, p, 1, k, n, scheme)[0]
+            assert np.linalg.norm(mine - want) <= 2.0 ** -11 * np.linalg.norm(want)
+
+
+def test_shared_tiles_need_room_for_their_pieces(oracle):
+    # without room for partial results the tiles are not shared: the same numbers up to the order of the sums
+    m, n, k = 1111, 4100, 4096
+    _, _, full = run(Q4_0, m, [n], k, DType.F32, 5)
+    _, _, lean = run(Q4_0, m, [n], k, DType.F32, 5, lean=True)
+    keep = np.arange(m) != 3
+    assert rel_err(lean[0][keep], full[0][keep].astype(np.float64)) <= 1e-5
