@@ -241,13 +241,13 @@ static int launch_gemv(const void *const *xs, int xk, const rlx_qweight *const *
     const size_t slot_bytes = (size_t)ng * 256;
     auto stage_bytes = [&](int kcu) {
         size_t b = ((size_t)rv * ((size_t)kcu * L.unit_k + 8) * 2 + 15) & ~(size_t)15;
-        if (scheme == SCHEME_Q4K || scheme == SCHEME_Q5K) b += (size_t)kcu * (L.unit_k / 32) * 16 * rg * 4;  // block sums
+        if (r2 && (scheme == SCHEME_Q4K || scheme == SCHEME_Q5K)) b += (size_t)kcu * (L.unit_k / 32) * 16 * 4;  // block sums
         return b;
     };
     // A launch shape: `wgs_per_cu` workgroups of `waves` waves per CU, every one resident at once, each with the same
     // number of (tile, unit) items (a segment with a longer K gets fewer row tiles per workgroup), LDS split between
-    // the per-(tile, wave) partial sums and the staged activation chunk (rv rows of halfs, 16 B row padding, plus the
-    // Q4_K block sums).
+    // the per-(tile, wave) partial sums and the staged activation chunk (rv rows of halfs, 16 B row padding, with one
+    // row plus the Q4_K / Q5_K block sums).
     struct Shape {
         GemvArgs a;
         int nwaves, wg, kcu;

@@ -205,14 +205,14 @@ __device__ __forceinline__ void load_afrags(const half_t *xrow, bool live, int c
 
 // One K unit of one 16-row weight tile against RG groups of 16 activation rows: the fragments are decoded once and
 // every group runs its own matrix instructions on them. xrow[rg] / live[rg]: the lane's row of group rg in LDS and
-// whether that row exists; acc[rg]: the four output rows 4 g + r of group rg this lane holds. SXS: row stride of the
-// Q4_K / Q5_K block-sum table (16 RG).
+// whether that row exists; acc[rg]: the four output rows 4 g + r of group rg this lane holds. sxs: the Q4_K / Q5_K
+// block-sum table of the one-row kernels, [block][16].
 template <int SCHEME, int NREG, int RG>
 __device__ __forceinline__ void compute_unit(const UnitRegs<SCHEME> &w, const half_t *const (&xrow)[RG], const bool (&live)[RG],
                                              Frag (&a)[4], const float *sxs, int g, int ucol, int ublk, float (&acc)[RG][4],
                                              half2_t sc_bias) {
     const float4_t zero = {0.f, 0.f, 0.f, 0.f};
-    constexpr int SXS = 16 * RG;
+    static_assert(RG == 1 || NREG == 4, "two groups hold more than two rows");
     if constexpr (SCHEME == SCHEME_Q4_0 || SCHEME == SCHEME_Q8_0) {
         Frag b[4];
         if constexpr (RG == 1) load_afrags<4>(xrow[0], live[0], ucol, a);  // before the decode, so the reads are in flight under it
@@ -342,6 +342,22 @@ __device__ __forceinline__ void compute_unit(const UnitRegs<SCHEME> &w, const ha
         uint32_t sc[2], mn[2];
         q4k_scales(w.meta[1], w.meta[2], w.meta[3], sc, mn);
         float psum[4] = {0.f, 0.f, 0.f, 0.f}, msum[4] = {0.f, 0.f, 0.f, 0.f};  // RG == 1: the super-block's two sums per output row
+        // The min term, sum over the blocks of mn * (sum of x over the block). With one activation row (NREG == 2) a table of block sums in
+        // LDS and one multiply-add per block and row. With more rows it is a matrix product of its own on the same activation
+        // fragments: B = mn in every place, exact, eight instructions chained in smin; no table to make between two barriers, no
+        // reads of it, four multiply-adds per block less. 4096 x 14336 at six f32 rows 26.3 -> 22.4 us; on the 128256-row LM head at one
+        // row the other way round, 61.5 against 54.4.
+        constexpr bool MIN_MFMA = NREG == 4;
+        float4_t smin[RG];
+        auto splat_min = [&](int h, int t) {
+            const half2_t m2 = splat_code_half(mn[h], t);
+            Frag f;
+#pragma unroll
+            for (int e = 0; e < 4; e++) f.h2[e] = m2;
+            return f;
+        };
+#pragma unroll
+        for (int rg = 0; rg < RG; rg++) smin[rg] = zero;
 #pragma unroll
         for (int h = 0; h < 2; h++) {
             Frag b[4];
@@ -356,6 +372,10 @@ __device__ __forceinline__ void compute_unit(const UnitRegs<SCHEME> &w, const ha
                 float4_t blk[4];
 #pragma unroll
                 for (int t = 0; t < 4; t++) blk[t] = mfma16(a[t], b[t], zero);
+                if constexpr (MIN_MFMA) {
+#pragma unroll
+                    for (int t = 0; t < 4; t++) smin[0] = mfma16(a[t], splat_min(h, t), smin[0]);
+                }
                 // Q4_K: the super-block's d and dmin are applied once, to the sums of sc * (block product) and of m * (block's
                 // activation sum) over its eight blocks: one conversion and one multiply-add per block, row and term
                 // (12.7 against 13.1 us on a 4096 -> 14336 projection). Q5_K keeps them per block: its kernels have no
@@ -364,15 +384,16 @@ __device__ __forceinline__ void compute_unit(const UnitRegs<SCHEME> &w, const ha
                 for (int t = 0; t < 4; t++) {
                     const float scf = ubyte_to_float(sc[h], t), mnf = ubyte_to_float(mn[h], t);
                     // sum of the activations of this 32-column block for the four output rows this lane holds
-                    float4_t sx = *(const float4_t *)(sxs + (ublk + 4 * h + t) * SXS + 4 * g);
+                    float4_t sx = zero;
+                    if constexpr (!MIN_MFMA) sx = *(const float4_t *)(sxs + (ublk + 4 * h + t) * 16 + 4 * g);
 #pragma unroll
                     for (int r = 0; r < NREG; r++) {
                         if constexpr (SCHEME == SCHEME_Q4K) {
                             psum[r] = __builtin_fmaf(scf, blk[t][r], psum[r]);
-                            msum[r] = __builtin_fmaf(mnf, sx[r], msum[r]);
+                            if constexpr (!MIN_MFMA) msum[r] = __builtin_fmaf(mnf, sx[r], msum[r]);
                         } else {
                             acc[0][r] = __builtin_fmaf(d * scf, blk[t][r], acc[0][r]);
-                            acc[0][r] = __builtin_fmaf(-(dmin * mnf), sx[r], acc[0][r]);
+                            if constexpr (!MIN_MFMA) acc[0][r] = __builtin_fmaf(-(dmin * mnf), sx[r], acc[0][r]);
                         }
                     }
                 }
@@ -380,7 +401,7 @@ __device__ __forceinline__ void compute_unit(const UnitRegs<SCHEME> &w, const ha
 #pragma unroll
                     for (int r = 0; r < NREG; r++) {
                         acc[0][r] = __builtin_fmaf(d, psum[r], acc[0][r]);
-                        acc[0][r] = __builtin_fmaf(-dmin, msum[r], acc[0][r]);
+                        if constexpr (!MIN_MFMA) acc[0][r] = __builtin_fmaf(-dmin, msum[r], acc[0][r]);
                     }
                 }
             } else {
@@ -389,25 +410,28 @@ __device__ __forceinline__ void compute_unit(const UnitRegs<SCHEME> &w, const ha
 #pragma unroll
                 for (int t = 0; t < 4; t++) {
                     const float dj = d * ubyte_to_float(sc[h], t);
-                    const float mj = dmin * ubyte_to_float(mn[h], t);
-                    float4_t blk[RG], sx[RG];
+                    const Frag fm = splat_min(h, t);
+                    float4_t blk[RG];
 #pragma unroll
                     for (int rg = 0; rg < RG; rg++) {
                         Frag af;
                         af.u4 = *(const uint4_t *)(xrow[rg] + ucol + h * 128 + t * 32);
                         blk[rg] = mfma16(af, b[t], zero);
-                        sx[rg] = *(const float4_t *)(sxs + (ublk + 4 * h + t) * SXS + 16 * rg + 4 * g);
+                        smin[rg] = mfma16(af, fm, smin[rg]);
                     }
 #pragma unroll
                     for (int rg = 0; rg < RG; rg++)
 #pragma unroll
-                        for (int r = 0; r < NREG; r++) {
-                            acc[rg][r] = __builtin_fmaf(dj, blk[rg][r], acc[rg][r]);
-                            acc[rg][r] = __builtin_fmaf(-mj, sx[rg][r], acc[rg][r]);
-                        }
+                        for (int r = 0; r < NREG; r++) acc[rg][r] = __builtin_fmaf(dj, blk[rg][r], acc[rg][r]);
                     __builtin_amdgcn_sched_barrier(0);
                 }
             }
+        }
+        if constexpr (MIN_MFMA) {
+#pragma unroll
+            for (int rg = 0; rg < RG; rg++)
+#pragma unroll
+                for (int r = 0; r < NREG; r++) acc[rg][r] = __builtin_fmaf(-dmin, smin[rg][r], acc[rg][r]);
         }
     }
 }
@@ -686,7 +710,7 @@ __device__ __forceinline__ bool gemv_pass(const GemvArgs &a) {
 
     const int kc = kc_units * L.unit_k;
     const int row_stride = kc + XS_PAD_HALFS;
-    // LDS: [partial sums: tiles_per_wg x nwaves x (4 ng) x 16 f32][staged activations: rv rows][Q4_K block sums]
+    // LDS: [partial sums: tiles_per_wg x nwaves x (4 ng) x 16 f32][staged activations: rv rows][Q4_K / Q5_K block sums of the one-row kernels]
     const int slot_floats = ng * 64;
     float *part = (float *)smem;
     // kw waves split the K units of one tile, tw = nwaves / kw tiles are walked side by side (kw = nwaves: every wave
@@ -786,9 +810,9 @@ __device__ __forceinline__ bool gemv_pass(const GemvArgs &a) {
                 atomicOr(notes + 1, wm[1]);
             }
         }
-        if constexpr (SCHEME == SCHEME_Q4K || SCHEME == SCHEME_Q5K) {
+        if constexpr ((SCHEME == SCHEME_Q4K || SCHEME == SCHEME_Q5K) && NREG == 2) {
             const int nblk = nu * BLK_PER_UNIT;
-            // rows >= rv of the [blk][16 RG] table are never read: compute_unit only uses the rows its lane group owns
+            // rows >= rv of the [blk][16] table are never read: compute_unit only uses the rows its lane group owns
             for (int idx = tid; idx < nblk * rv; idx += blockDim.x) {
                 const int blk = idx / rv, i = idx - blk * rv;
                 float sum = 0.f;
@@ -799,7 +823,7 @@ __device__ __forceinline__ bool gemv_pass(const GemvArgs &a) {
 #pragma unroll
                     for (int e = 0; e < 8; e++) sum += (float)f.h8[e];
                 }
-                sxs[blk * (16 * RG) + i] = sum;
+                sxs[blk * 16 + i] = sum;
             }
             __syncthreads();
         }
