@@ -153,6 +153,7 @@ struct XPrepArgs {
     float *rowfac;
     const int *perm;
     int perm_len;
+    int row_group, subs;
     int sums16;
 };
 constexpr int MOE_MAX_EXPERTS = 256;
@@ -490,10 +491,16 @@ static int launch_xprep(const void *x, int xk, int64_t m, int64_t k, const GemmP
     float *fac = (float *)workspace;
     void *xh = (uint8_t *)workspace + p.fac_bytes;
     void *sxh = p.sxh_bytes ? (uint8_t *)workspace + p.fac_bytes + p.cs_bytes + p.xh_bytes : nullptr;
-    XPrepArgs xa{x, xh, sxh, (int)m, (int)k, (int)p.k_pad, (int)p.m_rows, xk, fac, perm, perm_len, p.sums_kind == 2};
+    // Up to 128 image rows every kernel that reads the image does so 64 rows at a pass (rlx_gemvw_*, rlx_gemm64_*): the rest of the
+    // 256-row tile is not written. 64 bf16 rows of 28672: 7.1 -> 5.0 us.
+    const int64_t rv = xk == 0 ? 2 * m : m;
+    const int subs = !perm && rv <= 128 ? (int)((rv + 63) / 64 * 2) : 8;
+    // A workgroup per row of the scan until there are waves enough with one each (four to a workgroup, two workgroups per CU)
+    const int row_group = m < 2048;
+    XPrepArgs xa{x, xh, sxh, (int)m, (int)k, (int)p.k_pad, (int)p.m_rows, xk, fac, perm, perm_len, row_group, subs, p.sums_kind == 2};
     void *xparams[] = {&xa};
-    RLX_TRY(launch(K_XROWSCALE, (unsigned)((m + 3) / 4), 1, 256, 0, stream, xparams));
-    const long long xblocks = (p.m_rows / 256) * (p.k_pad / 64) * 8;  // (tile, step, 32-row sub-tile)
+    RLX_TRY(launch(K_XROWSCALE, (unsigned)(row_group ? m : (m + 3) / 4), 1, 256, 0, stream, xparams));
+    const long long xblocks = (p.m_rows / 256) * (p.k_pad / 64) * subs;  // (tile, step, 32-row sub-tile)
     return launch(K_XPREP, (unsigned)xblocks, 1, 256, 0, stream, xparams);
 }
 

@@ -752,6 +752,8 @@ struct XPrepArgs {
     float *rowfac;  // [m][2] (forward factor, its inverse), written by rlx_xrowscale before rlx_xprep runs
     const int *perm;  // expert-sorted image: row i of the image is row perm[i] of x (-1: a padding row of zeros); else null
     int perm_len;
+    int row_group;    // rlx_xrowscale: a workgroup per row (grid = m) instead of a wave
+    int subs;         // rlx_xprep: 32-row sub-tiles of every 256-row tile that are written (8, or as many as the 64-row passes of a small batch read)
     int sums16;       // sxh holds the sums of 16-column sub-blocks (Q2_K): sxh[row][k_pad / 256][32], leading halves then residuals
 };
 
@@ -760,11 +762,14 @@ struct XPrepArgs {
 // puts its largest value in [2^9, 2^10) (a sum of 32 such values stays below 2^15); every other row gets 1.
 // rlx_xprep multiplies by it while converting and the GEMM epilogue multiplies the finished sums by its inverse, both
 // exact, so the f32 range the reference computes in (rlx-cpu/src/gguf_matmul.rs:65-94) is kept. binary16 inputs are
-// carried as they are. One wave per row.
+// carried as they are. One wave per row, or with few rows (row_group: 256 threads a row) the whole workgroup, so that a long row is
+// a memory latency or two instead of one per 8 KB of it (64 bf16 rows of 28672: 7.0 -> 4.4 us).
 __device__ __forceinline__ void xrowscale_body(const XPrepArgs &a) {
+    __shared__ float wave_max[4];
     const int lane = threadIdx.x & 63;
-    const long long row = (long long)blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
-    if (row >= a.m) return;
+    const int span = a.row_group ? 256 : 64, at = a.row_group ? threadIdx.x : lane;  // threads that share a row, this one's place
+    const long long row = a.row_group ? (long long)blockIdx.x : (long long)blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
+    if (row >= a.m) return;  // with row_group no workgroup gets here: its threads meet at a barrier below
     // Eight 16-byte loads per lane are issued before the first is looked at: a row costs one memory latency per 8 KB, not
     // one per KB (the kernel is a launch of its own in front of every prefill matmul, and nothing but latency).
     float amax = 0.f;
@@ -772,12 +777,12 @@ __device__ __forceinline__ void xrowscale_body(const XPrepArgs &a) {
         const int esz = decltype(as_f32)::esz;
         const int chunks = a.k * esz / 16;  // 16-byte chunks of the row (k is a multiple of 32)
         const uint4_t *p = (const uint4_t *)((const uint8_t *)a.x + row * a.k * esz);
-        for (int c0 = lane; c0 < chunks; c0 += 64 * 8) {
+        for (int c0 = at; c0 < chunks; c0 += span * 8) {
             uint4_t raw[8];
 #pragma unroll
             for (int u = 0; u < 8; u++) {
                 raw[u] = uint4_t{0, 0, 0, 0};
-                if (c0 + 64 * u < chunks) raw[u] = p[c0 + 64 * u];
+                if (c0 + span * u < chunks) raw[u] = p[c0 + span * u];
             }
 #pragma unroll
             for (int u = 0; u < 8; u++)
@@ -800,7 +805,12 @@ __device__ __forceinline__ void xrowscale_body(const XPrepArgs &a) {
     else if (a.x_dtype == 1) scan(Bf16Word{});  // binary16 rows are not looked at: they are carried as they are
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) amax = __builtin_fmaxf(amax, __shfl_xor(amax, off));
-    if (lane == 0) {
+    if (a.row_group) {
+        if (lane == 0) wave_max[threadIdx.x >> 6] = amax;
+        __syncthreads();
+        amax = __builtin_fmaxf(__builtin_fmaxf(wave_max[0], wave_max[1]), __builtin_fmaxf(wave_max[2], wave_max[3]));
+    }
+    if (at == 0) {
         float fwd = 1.f, back = 1.f;
         const uint32_t mb = __builtin_bit_cast(uint32_t, amax);
         if (a.x_dtype != 2 && mb != 0 && mb < 0x7F800000u && (amax >= 1024.0f || amax < 0.00390625f)) {
@@ -819,9 +829,9 @@ __device__ __forceinline__ void xprep_body(const XPrepArgs &a) {
     __shared__ float part[4][32];
     const int lane = threadIdx.x & 63, ks = threadIdx.x >> 6;
     const int steps = a.k_pad / GEMM_KS;
-    const int sub = blockIdx.x & 7;
-    const int step = (blockIdx.x >> 3) % steps;
-    const int tile = (blockIdx.x >> 3) / steps;
+    const int sub = blockIdx.x % a.subs;
+    const int step = (blockIdx.x / a.subs) % steps;
+    const int tile = (blockIdx.x / a.subs) / steps;
     const int h = lane >> 5, c = 2 * ks + h;
     const int r = (lane & 31) ^ c;  // the slot's row within the sub-tile (frag_offset's swizzle is its own inverse)
     const long long vrow = (long long)tile * GEMM_MT + sub * 32 + r;
