@@ -153,7 +153,7 @@ struct XPrepArgs {
     float *rowfac;
     const int *perm;
     int perm_len;
-    int row_group, subs;
+    int row_group, subs_log2;
     int sums16;
 };
 constexpr int MOE_MAX_EXPERTS = 256;
@@ -421,15 +421,17 @@ static GemmSplit wide_split(const Layout &L, const WeightDims &D, int64_t m, siz
 // The 256 x 256 tiles of kernels/gemm_big.hip (Q4_0, Q8_0, code images) against the 256 x 128 tiles of kernels/gemm.hip, and how the
 // former are handed out: a tile per workgroup, or the whole line of (tile, 128 columns of K) items in equal runs, one per CU, with
 // the pieces of shared tiles added by a launch of their own. `groups` = 0: the 256 x 128 tiles. Estimated times decide, in us, with what
-// was measured on 2222 image rows of f32 activations in Q4_0: 128 columns of a tile cost BIG_QUAD with one workgroup per CU (28672 x
-// 4096: 1008 tiles in four rounds, 480 - 520 us in all) or SMALL_QUAD for half a tile (the same matrix 526); partial results travel
-// at 5 MB / us each way and the launch that adds them costs 4 us. 144 tiles of 4096 x 14336 (386 us as 288 half tiles in two rounds)
-// take 256 us shared out + 16 us for the sum, of 4096 x 4096 96 + 16 against 117.
+// was measured on 2222 image rows of f32 activations in Q4_0: a round of whole tiles costs BIG_ROUND and BIG_QUAD per 128 columns
+// (28672 x 4096: 1008 tiles in four rounds, 480 - 520 us in all), half tiles SMALL_QUAD (the same matrix 526); shared tiles cost
+// SHARE_START more than a round (two epilogues and a second prologue per workgroup), their pieces travel at 5 MB / us each way and the
+// launch that adds them costs 4 us. 144 tiles of 4096 x 14336 (386 us as 288 half tiles in two rounds) take 256 us shared + 16 us for the
+// sum, of 4096 x 4096 96 + 16 against 117; of 3072 x 2048 (1500 rows) 75 against 62, which the estimate leaves to the half tiles.
+// Code images run whole tiles from two rounds on in any case ([8192, 4096] x [4096, 4096] 310 -> 282 us; half tiles 14 % slower at K = 1024).
 struct BigPlan {
     int groups;
     size_t part_bytes;
 };
-constexpr double BIG_QUAD = 3.8, BIG_START = 4, SMALL_QUAD = 2.0, PART_BYTES_US = 5e6, REDUCE_US = 4;
+constexpr double BIG_QUAD = 3.65, BIG_ROUND = 6, SHARE_START = 20, SMALL_QUAD = 2.0, PART_BYTES_US = 5e6, REDUCE_US = 4;
 static BigPlan big_plan(int scheme, int xk, int64_t m, int64_t m_rows, int64_t tiles_n, int64_t small_tiles_n, int64_t n_sum, int64_t quads, size_t part_room) {
     BigPlan none{0, 0};
     if (scheme != SCHEME_Q4_0 && scheme != SCHEME_Q8_0) return none;
@@ -438,21 +440,23 @@ static BigPlan big_plan(int scheme, int xk, int64_t m, int64_t m_rows, int64_t t
     auto rounds = [&](long long t) { return (double)((t + cus - 1) / cus); };
     // the 256 x 128 tiles, with the split of K gemm_split gives them
     const long long small = tiles_m * small_tiles_n;
-    double t_small = rounds(small) * (double)quads * SMALL_QUAD;
+    // A single round that leaves CUs idle runs at a higher clock: 1.5 us on 160 half tiles, 1.65 on 192, 2.0 on a full chip
+    double t_small = rounds(small) * (double)quads * SMALL_QUAD * (small < cus ? 0.35 + 0.65 * (double)small / (double)cus : 1.0);
     if (small * 5 < cus * 4) {
         const long long split = std::min<long long>(quads, cus / small);
         t_small = t_small / (double)split + 2.0 * 4.0 * (double)split * (double)m * (double)n_sum / PART_BYTES_US + REDUCE_US;
     }
-    const double t_whole = BIG_START + rounds(tiles) * (double)quads * BIG_QUAD;
+    const double t_whole = rounds(tiles) * (BIG_ROUND + (double)quads * BIG_QUAD);
     const size_t tile_bytes = (size_t)(xk == 0 ? 128 : 256) * 1024;
     const size_t part = (size_t)cus * 2 * tile_bytes;
     double t_shared = 1e30;
     if (part <= part_room && tiles * quads >= cus) {
         // a workgroup leaves at most two pieces; a tile that is not shared leaves none
         const double pieces = (double)std::min<long long>(2 * cus, cus + tiles);
-        t_shared = BIG_START + (double)((tiles * quads + cus - 1) / cus) * BIG_QUAD + 2.0 * pieces * (double)tile_bytes / PART_BYTES_US + REDUCE_US;
+        t_shared = SHARE_START + (double)((tiles * quads + cus - 1) / cus) * BIG_QUAD + 2.0 * pieces * (double)tile_bytes / PART_BYTES_US + REDUCE_US;
     }
-    if (std::min(t_whole, t_shared) >= t_small) return none;
+    if (xk == XK_CODES && tiles >= 2 * cus) return BigPlan{(int)tiles, 0};
+    if (std::min(t_whole, t_shared) > 0.97 * t_small) return none;  // within the error of the estimate: the smaller tile
     if (t_shared < t_whole) return BigPlan{(int)cus, part};
     return BigPlan{(int)tiles, 0};
 }
@@ -484,7 +488,8 @@ static GemmPlan gemm_plan(int scheme, int xk, int64_t m, int64_t k, int64_t n = 
     return p;
 }
 
-// The conversion of x [m, k] into the workspace: one look at every row for its prescale factor, then the image.
+// The conversion of x [m, k] into the workspace: one look at every row for its prescale factor (none for binary16: a launch of
+// 5 us less), then the image.
 // With `perm` the image's row i is row perm[i] of x (tokens sorted by expert, padding rows -1), m still counting the rows of x.
 static int launch_xprep(const void *x, int xk, int64_t m, int64_t k, const GemmPlan &p, void *workspace, hipStream_t stream,
                         const int *perm = nullptr, int perm_len = 0) {
@@ -494,13 +499,14 @@ static int launch_xprep(const void *x, int xk, int64_t m, int64_t k, const GemmP
     // Up to 128 image rows every kernel that reads the image does so 64 rows at a pass (rlx_gemvw_*, rlx_gemm64_*): the rest of the
     // 256-row tile is not written. 64 bf16 rows of 28672: 7.1 -> 5.0 us.
     const int64_t rv = xk == 0 ? 2 * m : m;
-    const int subs = !perm && rv <= 128 ? (int)((rv + 63) / 64 * 2) : 8;
-    // A workgroup per row of the scan until there are waves enough with one each (four to a workgroup, two workgroups per CU)
-    const int row_group = m < 2048;
-    XPrepArgs xa{x, xh, sxh, (int)m, (int)k, (int)p.k_pad, (int)p.m_rows, xk, fac, perm, perm_len, row_group, subs, p.sums_kind == 2};
+    const int subs_log2 = perm || rv > 128 ? 3 : rv > 64 ? 2 : 1;
+    // A workgroup per row of the scan where a row is two or more memory latencies long for a wave (8 KB each) and one wave per row would
+    // leave CUs short of waves: 1111 f32 rows of 14336 15.5 -> 13.1 us; on 1500 bf16 rows of 2048 it would lose 1 us.
+    const int row_group = m < 2048 && k * (xk == 0 ? 4 : 2) >= 16384;
+    XPrepArgs xa{x, xh, sxh, (int)m, (int)k, (int)p.k_pad, (int)p.m_rows, xk, fac, perm, perm_len, row_group, subs_log2, p.sums_kind == 2};
     void *xparams[] = {&xa};
-    RLX_TRY(launch(K_XROWSCALE, (unsigned)(row_group ? m : (m + 3) / 4), 1, 256, 0, stream, xparams));
-    const long long xblocks = (p.m_rows / 256) * (p.k_pad / 64) * subs;  // (tile, step, 32-row sub-tile)
+    if (xk != 2) RLX_TRY(launch(K_XROWSCALE, (unsigned)(row_group ? m : (m + 3) / 4), 1, 256, 0, stream, xparams));
+    const long long xblocks = (p.m_rows / 256) * (p.k_pad / 64) << subs_log2;  // (tile, step, 32-row sub-tile)
     return launch(K_XPREP, (unsigned)xblocks, 1, 256, 0, stream, xparams);
 }
 

@@ -749,11 +749,11 @@ struct XPrepArgs {
     half_t *sxh;  // may be null
     int m, k, k_pad, m_rows;
     int x_dtype;  // 0 f32 (rows become hi / lo*2048 pairs), 1 bf16, 2 f16
-    float *rowfac;  // [m][2] (forward factor, its inverse), written by rlx_xrowscale before rlx_xprep runs
+    float *rowfac;  // [m][2] (forward factor, its inverse), written by rlx_xrowscale before rlx_xprep runs (binary16: by rlx_xprep)
     const int *perm;  // expert-sorted image: row i of the image is row perm[i] of x (-1: a padding row of zeros); else null
     int perm_len;
     int row_group;    // rlx_xrowscale: a workgroup per row (grid = m) instead of a wave
-    int subs;         // rlx_xprep: 32-row sub-tiles of every 256-row tile that are written (8, or as many as the 64-row passes of a small batch read)
+    int subs_log2;    // rlx_xprep: 1 << subs_log2 32-row sub-tiles of every 256-row tile are written (8, or as many as the 64-row passes of a small batch read)
     int sums16;       // sxh holds the sums of 16-column sub-blocks (Q2_K): sxh[row][k_pad / 256][32], leading halves then residuals
 };
 
@@ -762,7 +762,7 @@ struct XPrepArgs {
 // puts its largest value in [2^9, 2^10) (a sum of 32 such values stays below 2^15); every other row gets 1.
 // rlx_xprep multiplies by it while converting and the GEMM epilogue multiplies the finished sums by its inverse, both
 // exact, so the f32 range the reference computes in (rlx-cpu/src/gguf_matmul.rs:65-94) is kept. binary16 inputs are
-// carried as they are. One wave per row, or with few rows (row_group: 256 threads a row) the whole workgroup, so that a long row is
+// carried as they are and not scanned (rlx_xprep writes their factors, 1). One wave per row, or with few rows (row_group: 256 threads a row) the whole workgroup, so that a long row is
 // a memory latency or two instead of one per 8 KB of it (64 bf16 rows of 28672: 7.0 -> 4.4 us).
 __device__ __forceinline__ void xrowscale_body(const XPrepArgs &a) {
     __shared__ float wave_max[4];
@@ -802,7 +802,7 @@ __device__ __forceinline__ void xrowscale_body(const XPrepArgs &a) {
         }
     };
     if (a.x_dtype == 0) scan(F32Word{});
-    else if (a.x_dtype == 1) scan(Bf16Word{});  // binary16 rows are not looked at: they are carried as they are
+    else scan(Bf16Word{});
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) amax = __builtin_fmaxf(amax, __shfl_xor(amax, off));
     if (a.row_group) {
@@ -813,7 +813,7 @@ __device__ __forceinline__ void xrowscale_body(const XPrepArgs &a) {
     if (at == 0) {
         float fwd = 1.f, back = 1.f;
         const uint32_t mb = __builtin_bit_cast(uint32_t, amax);
-        if (a.x_dtype != 2 && mb != 0 && mb < 0x7F800000u && (amax >= 1024.0f || amax < 0.00390625f)) {
+        if (mb != 0 && mb < 0x7F800000u && (amax >= 1024.0f || amax < 0.00390625f)) {
             int e = (int)(mb >> 23) - 127;
             e = e < -100 ? -100 : e;
             fwd = __builtin_bit_cast(float, (uint32_t)(9 - e + 127) << 23);
@@ -829,9 +829,9 @@ __device__ __forceinline__ void xprep_body(const XPrepArgs &a) {
     __shared__ float part[4][32];
     const int lane = threadIdx.x & 63, ks = threadIdx.x >> 6;
     const int steps = a.k_pad / GEMM_KS;
-    const int sub = blockIdx.x % a.subs;
-    const int step = (blockIdx.x / a.subs) % steps;
-    const int tile = (blockIdx.x / a.subs) / steps;
+    const int sub = blockIdx.x & ((1 << a.subs_log2) - 1);
+    const int step = (blockIdx.x >> a.subs_log2) % steps;
+    const int tile = (blockIdx.x >> a.subs_log2) / steps;
     const int h = lane >> 5, c = 2 * ks + h;
     const int r = (lane & 31) ^ c;  // the slot's row within the sub-tile (frag_offset's swizzle is its own inverse)
     const long long vrow = (long long)tile * GEMM_MT + sub * 32 + r;
@@ -843,7 +843,12 @@ __device__ __forceinline__ void xprep_body(const XPrepArgs &a) {
 #pragma unroll
     for (int e = 0; e < 8; e++) v[e] = 0.f;
     const bool live_row = src_row >= 0 && src_row < a.m;
-    const float fwd = live_row ? a.rowfac[2 * src_row] : 1.f;
+    float fwd = 1.f;
+    if (a.x_dtype == 2) {  // binary16 rows are carried as they are: there is no scan before this launch, the factors are written here
+        if (live_row && step == 0 && threadIdx.x < 32) a.rowfac[2 * src_row] = a.rowfac[2 * src_row + 1] = 1.f;
+    } else if (live_row) {
+        fwd = a.rowfac[2 * src_row];
+    }
     if (live_row && col < a.k) {  // k is a multiple of 32, so a chunk of 8 is inside or outside as a whole
         if (a.x_dtype == 0) {
             const float4_t *p = (const float4_t *)((const float *)a.x + src_row * a.k + col);

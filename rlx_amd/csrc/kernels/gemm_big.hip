@@ -261,7 +261,7 @@ __device__ __forceinline__ void gemm_big_body(const GemmBigArgs &a) {
         // at a time around in LDS of its own, so that a store instruction covers 512 contiguous bytes of two rows; the rows'
         // factors come through LDS too.
         const int rows = a.pair_rows ? 128 : 256;
-        float *fac_s = (float *)smem, *turn_s = (float *)(smem + 1024 + wave * 16 * 132 * 4);
+        float *fac_s = (float *)smem, *turn_w = (float *)(smem + 1024 + wave * 2 * 16 * 132 * 4);  // two buffers: rows are written while the 16 before are read
         if (tid < rows) {
             const int row = by * rows + tid;
             fac_s[tid] = row < a.m_out ? a.rowfac[2 * row + 1] : 0.f;
@@ -274,23 +274,29 @@ __device__ __forceinline__ void gemm_big_body(const GemmBigArgs &a) {
         const bool wide = (ld & 3) == 0 && ((uintptr_t)dst & 15) == 0;
         const int scol = wn * 128 + (lane & 31) * 4;
 #pragma unroll
-        for (int i = 0; i < 8; i++) {
+        for (int ii = 0; ii < 9; ii++) {
             __builtin_amdgcn_sched_barrier(0);
             asm volatile("" ::: "memory");
-            const int t0 = wm * 128 + i * 16;  // image row
-            if (a.pair_rows) {
+            const int i = ii;
+            int t0 = wm * 128 + i * 16;  // image row
+            float *turn_s = turn_w + (i & 1) * 16 * 132;
+            if (ii == 8) {
+            } else if (a.pair_rows) {
 #pragma unroll
                 for (int r = 0; r < 4; r += 2)
 #pragma unroll
                     for (int j = 0; j < 8; j++)
-                        turn_s[(2 * lg + (r >> 1)) * 132 + j * 16 + lr] = (acc[i][j][r] + acc[i][j][r + 1] * (1.0f / BIG_LO_SCALE)) * fac_s[t0 / 2 + 2 * lg + (r >> 1)];
+                        turn_s[(2 * lg + (r >> 1)) * 132 + j * 16 + lr] = (acc[i & 7][j][r] + acc[i & 7][j][r + 1] * (1.0f / BIG_LO_SCALE)) * fac_s[t0 / 2 + 2 * lg + (r >> 1)];
             } else {
 #pragma unroll
                 for (int r = 0; r < 4; r++)
 #pragma unroll
-                    for (int j = 0; j < 8; j++) turn_s[(4 * lg + r) * 132 + j * 16 + lr] = acc[i][j][r] * fac_s[t0 + 4 * lg + r];
+                    for (int j = 0; j < 8; j++) turn_s[(4 * lg + r) * 132 + j * 16 + lr] = acc[i & 7][j][r] * fac_s[t0 + 4 * lg + r];
             }
             asm volatile("" ::: "memory");
+            if (ii == 0) continue;
+            t0 -= 16;
+            turn_s = turn_w + ((i & 1) ^ 1) * 16 * 132;
             const int r0 = a.pair_rows ? t0 / 2 : t0;
             for (int g = 0; g < (a.pair_rows ? 4 : 8); g++) {
                 const int tr = 2 * g + (lane >> 5), row = r0 + tr;

@@ -46,8 +46,8 @@ def run(scheme, m, ns, k, x_dtype, seed, lean=False, offset=0):
     (Q4_0, 1111, [4100], 4096, DType.F32, 0),          # shared tiles, ragged rows and columns
     (Q8_0, 1100, [4093], 4128, DType.F32, 0),          # odd columns: no 16-byte stores; K ends inside a 128-column unit of the image
     (Q4_0, 1111, [4096], 4096, DType.F32, 4),          # an output that is only 4-byte aligned
-    (Q8_0, 2050, [6143], 4064, DType.BF16, 0),         # a tile per workgroup, 16-bit rows
-    (Q4_0, 1090, [4096, 1030, 1024], 4096, DType.F32, 0),  # three matrices side by side
+    (Q8_0, 2050, [6143], 8992, DType.BF16, 0),         # a tile per workgroup, 16-bit rows
+    (Q4_0, 1090, [4096, 1030, 1024], 8992, DType.F32, 0),  # three matrices side by side
     (Q8_0, 2050, [3900], 8192, DType.BF16, 0),         # shared tiles, 16-bit rows
 ])
 def test_large_tiles_match_the_oracle(oracle, scheme, m, ns, k, x_dtype, offset):

@@ -18,7 +18,7 @@ def test_no_image_row_is_read_that_was_not_written(oracle, scheme, m, x_dtype):
     check(oracle, scheme, n, k, m, x_dtype)
 
 
-@pytest.mark.parametrize("m,k", [(2047, 64), (2048, 64), (2049, 32), (70, 16416)])
+@pytest.mark.parametrize("m,k", [(2047, 64), (2049, 32), (70, 4064), (70, 4096), (70, 16416)])
 def test_row_scan_by_waves_and_by_workgroups(oracle, m, k):
     check(oracle, Q4_0, 48, k, m, DType.F32, rows=[0, 3, 5, m // 2, m - 1])
 
