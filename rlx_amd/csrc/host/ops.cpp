@@ -115,6 +115,13 @@ struct GemmBigArgs {
     float *part;
     int m_out, tiles_m, tiles_n, a_steps, quads, pair_rows;
 };
+struct GemmImgArgs {  // mirrors kernels/gemm.hip
+    const void *a_img;
+    const void *b_img;
+    float *out;
+    const float *rowfac;
+    int m_out, n, steps;
+};
 constexpr int GEMVW_MAX_SEG = 8;
 struct GemvWSeg {  // mirrors kernels/gemv_wide.hip
     const void *w;
@@ -624,6 +631,11 @@ static int launch_gemm(const void *x, int xk, const rlx_qweight *const *ws, floa
             ba.tiles_m = (int)(p.m_rows / 256);
             ba.a_steps = (int)(p.k_pad / 64);
             ba.pair_rows = xk == 0 ? 1 : 0;
+            if (codes && !bp.part_bytes && p.k_pad < 2048) {  // short K: the kernel with the shorter way in and out of a tile
+                GemmImgArgs ia{xh, wimg, outs[0], fac, (int)m, (int)w->dims.n, (int)(p.k_pad / 64)};
+                void *iparams[] = {&ia};
+                return launch3(K_GEMM_IMG_F16W, (unsigned)ba.tiles_n, (unsigned)ba.tiles_m, 1, 512, 2 * 65536, stream, iparams);
+            }
             int groups = bp.groups;
             void *bparams[] = {&ba, &groups};
             const KernelId bid = codes ? K_GEMM_BIG_F16W : w->scheme == SCHEME_Q4_0 ? K_GEMM_BIG_Q4_0 : K_GEMM_BIG_Q8_0;

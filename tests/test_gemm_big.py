@@ -69,3 +69,22 @@ def test_shared_tiles_need_room_for_their_pieces(oracle):
     _, _, lean = run(Q4_0, m, [n], k, DType.F32, 5, lean=True)
     keep = np.arange(m) != 3
     assert rel_err(lean[0][keep], full[0][keep].astype(np.float64)) <= 1e-5
+
+
+@pytest.mark.parametrize("m,k,n", [(8192, 512, 3900), (8000, 2048, 4001)])  # code images: short K, and the first K of the four-wave kernel
+def test_code_images_of_many_rows(oracle, m, k, n):
+    from rlx_amd import Graph, Op, Session, Shape
+    rng = np.random.default_rng(k)
+    x = rng.standard_normal((m, k)).astype(np.float32)
+    packed = tiled_packed(Q8_0, n, k, 7, 0.02).reshape(-1)
+    g = Graph.new("chain")
+    w = g.param("w", Shape.new([len(packed)], DType.U8))
+    q = g.fake_quantize(g.input("x", Shape.new([m, k], DType.F32)), 8, 1)
+    g.set_outputs([g.add_node(Op.DequantMatMul(QuantScheme.GgufQ8_0), [q, w], Shape.new([m, n], DType.F32))])
+    c = Session.new().compile(g)
+    c.set_param_typed("w", packed, DType.U8)
+    got = np.asarray(c.run([("x", x)])[0]).reshape(m, n)
+    s = np.maximum(np.abs(x).max(0) / np.float32(127), np.float32(1e-12)).astype(np.float32)
+    xq = np.clip(np.round(x / s), -127, 127).astype(np.float32) * s
+    rows = [0, 1, 255, 256, m // 2, m - 1]
+    assert rel_err(got[rows], oracle.gguf_matmul_f64(xq[rows], packed, len(rows), k, n, Q8_0)) <= TOL
