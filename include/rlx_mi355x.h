@@ -262,8 +262,9 @@ int rlx_mi355x_qweight_rows(const rlx_qweight *w, int64_t row0, int64_t rows, rl
  * (its thunk converts nothing). ..._prepare writes the binary16 image of x[m, k] (and, for Q4_K / Q5_K, its block
  * sums) into `workspace` (rlx_mi355x_gguf_matmul_workspace(scheme, x_dtype, m, k, 0) bytes); ..._bt_prepared multiplies
  * that image by `count` matrices, all with the k the image was made for: outs_dev[i][m, n_i]. An image made for Q4_K / Q5_K also
- * serves the other schemes, not the other way round. x_dtype = RLX_I8 names the code image rlx_mi355x_fake_quantize_image
- * leaves (see there). */
+ * serves the schemes without block sums (all but Q2_K), not the other way round, and stays whole through such calls. A workspace
+ * larger than the image (the size call with n > 0) takes partial results behind every scheme's image, so calls on one workspace
+ * must be ordered on one stream. x_dtype = RLX_I8 names the code image rlx_mi355x_fake_quantize_image leaves (see there). */
 int rlx_mi355x_gguf_matmul_prepare(const void *x_dev, int x_dtype, int scheme, int64_t m, int64_t k, void *workspace,
                                    size_t workspace_bytes, void *stream);
 int rlx_mi355x_gguf_matmul_bt_prepared(const void *workspace, size_t workspace_bytes, int x_dtype, const rlx_qweight *const *ws,

@@ -393,14 +393,17 @@ static GemmSplit gemm_split(long long tiles_x, long long tiles_y, int64_t k_unit
 // Workspace of a prefill matmul: [per-row factors][column scales][image of x][block sums][image of the scaled weights]
 // [partial results of a split K]. The second and the fifth exist only for a FakeQuantize code image (XK_CODES), whose
 // matmul runs on ready binary16 weights W * diag(s) (n is the widest matrix multiplied from the image, one at a time).
+// The image may have been made for another scheme than the one that multiplies it (rlx_mi355x_gguf_matmul_prepare), and that
+// scheme's matmul may follow: partial results begin past the widest block sums any scheme's image has, whatever the scheme.
 struct GemmPlan {
     int64_t m_rows, k_pad;
     size_t xh_bytes, sxh_bytes, fac_bytes;  // the image, the block sums (Q4_K / Q5_K per 32 columns, Q2_K per 16), the per-row prescale factors
     size_t cs_bytes, wimg_bytes;
+    size_t part_off;                        // where partial results begin
     size_t part_bytes;                      // split K of one [m, n] matmul on its own: split x m x n floats (0: no split)
     int sums_kind;                          // act_sums_kind of the scheme the plan was made for
     size_t image_end() const { return fac_bytes + cs_bytes + xh_bytes + sxh_bytes; }
-    size_t total() const { return image_end() + wimg_bytes + part_bytes; }
+    size_t total() const { return part_bytes ? part_off + part_bytes : image_end() + wimg_bytes; }
 };
 static bool gemm_skinny(int xk, int64_t m) { return (xk == 0 ? 2 * m : m) <= 128; }
 // Up to 192 image rows of Q4_0 / Q8_0 run rlx_gemvw_* (kernels/gemv_wide.hip): weights decoded in registers by the wave
@@ -478,6 +481,8 @@ static GemmPlan gemm_plan(int scheme, int xk, int64_t m, int64_t k, int64_t n = 
     p.fac_bytes = ((size_t)m * 8 + 255) & ~(size_t)255;
     p.cs_bytes = xk == XK_CODES ? (size_t)p.k_pad * 4 : 0;
     p.wimg_bytes = xk == XK_CODES ? (size_t)((n + 255) / 256 * 256) * p.k_pad * 2 : 0;  // whole 256-row tiles of the large-m kernel
+    p.part_off = xk == XK_CODES ? p.image_end() + p.wimg_bytes
+                                : p.fac_bytes + p.xh_bytes + (size_t)p.m_rows * (p.k_pad / 256) * 32 * ACT_SUMS_KIND_MAX;
     p.part_bytes = 0;
     if (n > 0 && gemm_wide(scheme, xk, m)) {
         const WeightDims D = weight_dims(scheme, n, k);
@@ -540,7 +545,7 @@ static int launch_gemm(const void *x, int xk, const rlx_qweight *const *ws, floa
             set_error("gguf_matmul_bt: matrices of one prefill launch differ in scheme or K");
             return RLX_ERR_INVALID;
         }
-    const size_t ops_end = p.image_end() + p.wimg_bytes;  // the operands; partial results of a split K follow
+    const size_t ops_end = p.image_end() + p.wimg_bytes;  // the operands
     if (!workspace || workspace_bytes < ops_end) {
         set_error("gguf_matmul_bt: m=%lld needs a %zu-byte workspace, got %zu", (long long)m, ops_end, workspace_bytes);
         return RLX_ERR_INVALID;
@@ -555,6 +560,8 @@ static int launch_gemm(const void *x, int xk, const rlx_qweight *const *ws, floa
     void *xh = (uint8_t *)workspace + p.fac_bytes + p.cs_bytes;
     void *sxh = p.sxh_bytes ? (uint8_t *)workspace + p.fac_bytes + p.cs_bytes + p.xh_bytes : nullptr;
     uint8_t *wimg = (uint8_t *)workspace + p.image_end();
+    uint8_t *part_base = (uint8_t *)workspace + p.part_off;  // partial results; every part of the workspace is a multiple of 256 bytes
+    const size_t part_room = workspace_bytes > p.part_off ? workspace_bytes - p.part_off : 0;
     if (codes) {  // B = fl16(W * diag(s) / S) as stage images; fac holds (1 / S, S) for every row
         WScaleArgs wa{w->dev, wimg, (const float *)((uint8_t *)workspace + p.fac_bytes), fac, w->dims.row_tiles, w->dims.units, (int)p.k_pad, w->sc_off()};
         void *wparams[] = {&wa};
@@ -575,7 +582,7 @@ static int launch_gemm(const void *x, int xk, const rlx_qweight *const *ws, floa
             sps[i] = wide_split(ws[i]->layout, ws[i]->dims, m, launch_bytes);
             if (sps[i].split > 1) part_need += (size_t)sps[i].split * (size_t)m * (size_t)ws[i]->dims.n * 4;
         }
-        if (part_need > workspace_bytes - ops_end)  // a workspace without room for the slices: every matrix in one piece
+        if (part_need > part_room)  // a workspace without room for the slices: every matrix in one piece
             for (int i = 0; i < count; i++) sps[i] = GemmSplit{1, (int)((ws[i]->dims.units + 1) / 2 * 2)};
         GemvWArgs wa{};
         long long wgs = 0;
@@ -583,7 +590,7 @@ static int launch_gemm(const void *x, int xk, const rlx_qweight *const *ws, floa
         for (int i = 0; i < count; i++) {
             float *dst = outs[i];
             if (sps[i].split > 1) {
-                dst = (float *)((uint8_t *)workspace + ops_end + off);
+                dst = (float *)(part_base + off);
                 off += (size_t)sps[i].split * (size_t)m * (size_t)ws[i]->dims.n * 4;
             }
             wa.seg[i] = GemvWSeg{ws[i]->dev, dst, (int)ws[i]->dims.n, (int)ws[i]->dims.row_tiles, (int)wgs, sps[i].split, sps[i].units_per_split};
@@ -621,12 +628,12 @@ static int launch_gemm(const void *x, int xk, const rlx_qweight *const *ws, floa
             n_sum += ws[i]->dims.n;
         }
         ba.quads = codes ? (int)(p.k_pad / 128) : (int)w->dims.units;
-        const BigPlan bp = big_plan(w->scheme, xk, m, p.m_rows, ba.tiles_n, small_n, n_sum, ba.quads, workspace_bytes - ops_end);
+        const BigPlan bp = big_plan(w->scheme, xk, m, p.m_rows, ba.tiles_n, small_n, n_sum, ba.quads, part_room);
         if (bp.groups) {
             ba.nseg = count;
             ba.a_img = xh;
             ba.rowfac = fac;
-            ba.part = (float *)((uint8_t *)workspace + ops_end);
+            ba.part = (float *)part_base;
             ba.m_out = (int)m;
             ba.tiles_m = (int)(p.m_rows / 256);
             ba.a_steps = (int)(p.k_pad / 64);
@@ -658,13 +665,11 @@ static int launch_gemm(const void *x, int xk, const rlx_qweight *const *ws, floa
     }
     a.nseg = count;
     const int gy = skinny ? (int)((rv + 63) / 64) : (int)(p.m_rows / 256);
-    // Split K: every slice writes its partial result behind the operands in the workspace, then one reduce launch per
+    // Split K: every slice writes its partial result behind the images in the workspace, then one reduce launch per
     // matrix adds the slices in ascending K into the output. A workspace sized for fewer slices gets fewer.
     size_t n_sum = 0;
     for (int i = 0; i < count; i++) n_sum += (size_t)ws[i]->dims.n;
     GemmSplit sp = gemm_split(gx, gy, k_units, steps_per_unit, skinny);
-    const size_t part_room = workspace_bytes - ops_end;
-    uint8_t *part_base = (uint8_t *)workspace + ops_end;  // every part of the workspace is a multiple of 256 bytes
     if (sp.split > 1 && (size_t)sp.split * (size_t)m * n_sum * 4 > part_room)
         sp = gemm_split(gx, gy, k_units, steps_per_unit, skinny, (int)std::max<size_t>(1, part_room / ((size_t)m * n_sum * 4)));
     if (sp.split > 1 && (size_t)sp.split * (size_t)m * n_sum * 4 > part_room) sp = gemm_split(gx, gy, k_units, steps_per_unit, skinny, 1);
@@ -953,7 +958,7 @@ int rlx_mi355x_gguf_matmul_bt_prepared(const void *workspace, size_t workspace_b
         while (i + c < count && c < GEMM_MAX_SEG && ws[i + c]->scheme == ws[i]->scheme && ws[i + c]->dims.k == ws[i]->dims.k &&
                ws[i + c]->sc_off() == ws[i]->sc_off())
             c++;
-        // `workspace` is only read; the x pointer is not looked at when the image is already there
+        // of `workspace` only what lies past every scheme's image is written; the x pointer is not looked at when the image is already there
         RLX_TRY(launch_gemm(workspace, xk, ws + i, outs_dev + i, c, m, const_cast<void *>(workspace), workspace_bytes, (hipStream_t)stream, true));
         i += c;
     }

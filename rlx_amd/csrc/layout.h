@@ -100,6 +100,7 @@ RLX_HD constexpr int kernel_scheme(int scheme) { return scheme == SCHEME_Q3K ? S
 // What a scheme's prefill kernel needs next to the activation image: 0 nothing, 1 the sums of every 32-column block
 // (Q4_K / Q5_K: the dmin term), 2 the sums of every 16-column sub-block (Q2_K).
 RLX_HD constexpr int act_sums_kind(int scheme) { return (scheme == SCHEME_Q4K || scheme == SCHEME_Q5K) ? 1 : scheme == SCHEME_Q2K ? 2 : 0; }
+constexpr int ACT_SUMS_KIND_MAX = 2;  // sums take 32 bytes of every row and 256 columns per kind
 
 // nibble position of fragment element e inside a granule word
 RLX_HD constexpr int nib_pos(int e) { return ((e & 1) << 2) | (e >> 1); }

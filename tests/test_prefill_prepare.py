@@ -1,10 +1,13 @@
 """Activation preparation of the prefill path (rlx_xrowscale, rlx_xprep): a workspace that holds NaN everywhere, so that an image row read
-without having been written shows, around the 64-row passes of small batches; and both ways of scanning the rows."""
+without having been written shows, around the 64-row passes of small batches; both ways of scanning the rows; and an image made once for
+matmuls of two schemes."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
 import rlx_amd
-from helpers import Q2K, Q4_0, Q4K, f32_to_bf16_bits, make_weights, random_blocks, rel_err
+from helpers import Q2K, Q4_0, Q4K, Q5K, Q6K, Q8_0, f32_to_bf16_bits, make_weights, random_blocks, rel_err
 from rlx_amd import DType, QuantScheme, ops
 
 pytestmark = pytest.mark.gpu
@@ -21,6 +24,37 @@ def test_no_image_row_is_read_that_was_not_written(oracle, scheme, m, x_dtype):
 @pytest.mark.parametrize("m,k", [(2047, 64), (2049, 32), (70, 4064), (70, 4096), (70, 16416)])
 def test_row_scan_by_waves_and_by_workgroups(oracle, m, k):
     check(oracle, Q4_0, 48, k, m, DType.F32, rows=[0, 3, 5, m // 2, m - 1])
+
+
+@pytest.mark.parametrize("first,second,m,n,k,x_dtype", [
+    (Q4K, Q4_0, 1111, 4100, 4096, DType.F32),   # shared 256 x 256 tiles leave pieces
+    (Q4K, Q8_0, 40, 1100, 4096, DType.F32),     # K slices of the 64-rows-a-pass kernel
+    (Q2K, Q6K, 40, 200, 2048, DType.BF16),      # split K of the 64-row tiles
+    (Q5K, Q6K, 300, 200, 2048, DType.F32),      # split K of the 256-row tiles
+])
+def test_an_image_stays_whole_through_matmuls_of_other_schemes(first, second, m, n, k, x_dtype):
+    # prepared once for a scheme with block sums; between two matmuls of that scheme another scheme's partial results go into the
+    # same workspace, which holds what either scheme asks for
+    rng = np.random.default_rng(m + n)
+    x = rng.standard_normal((m, k)).astype(np.float32)
+    xd = ops.DeviceBuffer.from_numpy(f32_to_bf16_bits(x) if x_dtype == DType.BF16 else x)
+    L = rlx_amd._lib.lib()
+    ws = [ops.QWeight(QuantScheme(s), random_blocks(s, n, k, seed=i, d_std=2e-3, dmin_std=2e-3) if s in (Q2K, Q5K, Q6K) else make_weights(s, n, k, seed=i)[0], n, k)
+          for i, s in enumerate((first, second))]
+    need = max(L.rlx_mi355x_gguf_matmul_workspace(s, int(x_dtype), m, k, n) for s in (first, second))
+    wsb, od = ops.DeviceBuffer(need), ops.DeviceBuffer(m * n * 4)
+    rlx_amd._lib.check(L.rlx_mi355x_gguf_matmul_prepare(xd.ptr, int(x_dtype), first, m, k, wsb.ptr, need, None))
+
+    def product(w):
+        rlx_amd._lib.check(L.rlx_mi355x_gguf_matmul_bt_prepared(wsb.ptr, need, int(x_dtype), (C.c_void_p * 1)(w.ptr), (C.c_void_p * 1)(od.ptr), 1, m, None))
+        ops.sync()
+        return od.to_numpy(np.uint32)
+
+    before = product(ws[0])
+    product(ws[1])
+    assert np.array_equal(product(ws[0]), before)
+    for w in ws:
+        w.free()
 
 
 def check(oracle, scheme, n, k, m, x_dtype, rows=None):
