@@ -1185,8 +1185,15 @@ struct TopkArgs {  // mirrors kernels/topk.hip
     uint32_t *out_idx;
     float *out_val;
 };
-constexpr int64_t TOPK_GROUP = 1024;   // candidates one wave of rlx_topk_select reduces to `cap`
+constexpr int64_t TOPK_GROUP = 1024;   // candidates one wave of rlx_topk_serial / rlx_topk_select reduces to `cap`
 constexpr int64_t TOPK_FINISH = 8192;  // candidates rlx_topk_finish takes
+// Winners one by one or by threshold, in us of the whole call on Q8_0 rows of 1024 columns. Reducing 1024s: 9000 rows at cap 1 20.8
+// one by one, 24.0 by threshold; at cap 10 24.2 against 25.1; at cap 12 25 against 24.
+constexpr int TOPK_SERIAL_CAP = 11;
+// The end, one by one in a single wave or by threshold in a workgroup of sixteen, which up to 128 candidates has nothing to cut: 40 rows
+// at cap 4 9.0 against 9.9, at cap 8 10.0 against 9.9; 300 rows at cap 1 9.3 against 13.4, at cap 17 13.3 against 13.4; 1000 rows at
+// cap 1 11.5 against 14.8, at cap 11 14.0 against 14.8, at cap 12 14.9 against 14.8.
+static bool topk_serial_end(int64_t count, int cap) { return cap <= (count <= 128 ? 7 : count <= 512 ? 17 : count <= TOPK_GROUP ? 11 : 0); }
 constexpr int TOPK_MAX_CAP = 64;
 static int64_t topk_groups(int64_t n) { return (n + TOPK_GROUP - 1) / TOPK_GROUP; }
 }  // namespace rlx
@@ -1225,7 +1232,7 @@ static int tied_lm_topk(const char *who, const void *hidden_dev, int xk, const r
     const rlx_qweight *ws[1] = {embed};
     float *outs[1] = {logits};
     RLX_TRY(launch_gemv(xs, xk, ws, outs, 1, 1, (hipStream_t)stream, nullptr, nullptr, nullptr, norm));
-    // One workgroup orders up to TOPK_FINISH candidates; more than that first lose all but the cap best of every 1024.
+    // One launch orders up to TOPK_FINISH candidates; more than that first lose all but the cap best of every 1024.
     int64_t count = n;
     int side = 0;
     bool first = true;
@@ -1233,13 +1240,13 @@ static int tied_lm_topk(const char *who, const void *hidden_dev, int xk, const r
         const int64_t groups = topk_groups(count);
         TopkArgs p{first ? logits : nullptr, first ? nullptr : keys[side ^ 1], (int)count, cap, keys[side], nullptr, nullptr};
         void *params[] = {&p};
-        RLX_TRY(launch(K_TOPK_SELECT, (unsigned)groups, 1, 64, 0, (hipStream_t)stream, params));
+        RLX_TRY(launch(cap <= TOPK_SERIAL_CAP ? K_TOPK_SERIAL : K_TOPK_SELECT, (unsigned)groups, 1, 64, 0, (hipStream_t)stream, params));
         count = groups * cap;
     }
     TopkArgs p{first ? logits : nullptr, first ? nullptr : keys[side ^ 1], (int)count, cap, nullptr, out_idx_dev, out_val_dev};
     void *params[] = {&p};
-    RLX_TRY(launch(K_TOPK_FINISH, 1, 1, 1024, 0, (hipStream_t)stream, params));
-    return RLX_OK;
+    const bool serial = topk_serial_end(count, cap);
+    return launch(serial ? K_TOPK_SERIAL : K_TOPK_FINISH, 1, 1, serial ? 64 : 1024, 0, (hipStream_t)stream, params);
 }
 
 int rlx_mi355x_gguf_tied_lm_topk(const void *hidden_dev, int x_dtype, const rlx_qweight *embed, int cap, uint32_t *out_idx_dev,

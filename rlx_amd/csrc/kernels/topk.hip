@@ -4,18 +4,21 @@
 // (value, row) keys follows. Keys order as in the argmax: larger value first, among equal values the smaller row; a NaN
 // logit is no candidate; every key is unique, so "the cap-th largest" is one key.
 //
-// Neither kernel takes the winners one by one (cap rounds of a wave-wide maximum, each waiting for the one before, were
-// 12 - 17 us a launch): both find a threshold by bisection over the bits of the key, a count per step, and only the last
-// kernel puts the few survivors in order, every survivor counting the keys above its own.
+// Few winners are taken one by one, many through a threshold found by bisection over the bits of the key, a count per step,
+// after which every survivor counts the keys above its own:
+//   rlx_topk_serial  one wave per 1024 candidates, sixteen per lane, sorted once per lane; cap rounds of a wave-wide maximum of the
+//                    lanes' heads, the lane that held the winner moves its list up. Writes its cap winners as keys or, as
+//                    the only wave, the answer. No LDS, no barrier.
 //   rlx_topk_select  one wave per 1024 candidates, sixteen per lane, leaves their `cap` best in any order. No LDS, no barrier.
 //   rlx_topk_finish  one workgroup, up to 8192 candidates, eight per thread: writes rows and values, largest first.
-// Both are bound by latency (launch, one load, the chain of counts), not by bandwidth: 128256 logits are 0.5 MB. The whole
-// LM-head call at [128256, 4096] Q4_K, cap 40: 93.3 -> 71.6 us, 57 of it the matmul.
+// All are bound by latency (launch, one load, the chain of rounds or counts), not by bandwidth: 128256 logits are 0.5 MB. The whole
+// LM-head call at [128256, 4096] Q4_K, cap 40: 93.3 us with the serial kernel alone, 69 - 72 with the other two, about 54 of it the
+// matmul. Where the lines between them lie: host/ops.cpp.
 #include "common.h"
 
 namespace rlx {
 
-constexpr int TOPK_PER_LANE = 16, TOPK_GROUP = 64 * TOPK_PER_LANE;       // candidates per wave of rlx_topk_select
+constexpr int TOPK_PER_LANE = 16, TOPK_GROUP = 64 * TOPK_PER_LANE;       // candidates per wave of rlx_topk_serial / rlx_topk_select
 constexpr int TOPK_PER_THREAD = 8, TOPK_FINISH = 1024 * TOPK_PER_THREAD;  // candidates rlx_topk_finish takes
 constexpr int TOPK_SURVIVORS = 128;                                       // keys it puts in order (cap <= 64)
 
@@ -47,10 +50,10 @@ __device__ __forceinline__ uint32_t wave_min_u32(uint32_t v) {
 struct TopkArgs {
     const float *vals;                  // first pass: [n] logits; null afterwards
     const unsigned long long *keys_in;  // later passes: [n] keys, zero = no candidate
-    int n;                              // candidates in all; wave g of rlx_topk_select takes [g * TOPK_GROUP, (g + 1) * TOPK_GROUP)
+    int n;                              // candidates in all; wave g of rlx_topk_serial / _select takes [g * TOPK_GROUP, (g + 1) * TOPK_GROUP)
     int cap;
-    unsigned long long *keys_out;       // rlx_topk_select: [waves][cap] keys
-    uint32_t *out_idx;                  // rlx_topk_finish: [cap] rows and values; (0, -inf) where no candidate is left
+    unsigned long long *keys_out;       // rlx_topk_select and all but a last rlx_topk_serial: [waves][cap] keys
+    uint32_t *out_idx;                  // last launch: [cap] rows and values; (0, -inf) where no candidate is left
     float *out_val;
 };
 
@@ -62,6 +65,52 @@ __device__ __forceinline__ unsigned long long topk_load(const TopkArgs &a, long 
 }
 
 }  // namespace rlx
+
+extern "C" __global__ __launch_bounds__(64) void rlx_topk_serial(rlx::TopkArgs a) {
+    using namespace rlx;
+    const int lane = threadIdx.x;
+    const long long base = (long long)blockIdx.x * TOPK_GROUP;
+    unsigned long long mine[TOPK_PER_LANE];
+#pragma unroll
+    for (int e = 0; e < TOPK_PER_LANE; e++) mine[e] = topk_load(a, base + lane + e * 64);
+    // this lane's candidates in descending order (bitonic network over registers: every index is a constant)
+#pragma unroll
+    for (int k = 2; k <= TOPK_PER_LANE; k <<= 1)
+#pragma unroll
+        for (int j = k >> 1; j > 0; j >>= 1)
+#pragma unroll
+            for (int i = 0; i < TOPK_PER_LANE; i++) {
+                const int l = i ^ j;
+                if (l > i) {
+                    const unsigned long long x = mine[i], y = mine[l];
+                    const bool desc = (i & k) == 0;  // descending runs first, so the last merge leaves the whole list descending
+                    const bool swap = desc ? (x < y) : (x > y);
+                    mine[i] = swap ? y : x;
+                    mine[l] = swap ? x : y;
+                }
+            }
+    for (int r = 0; r < a.cap; r++) {
+        const uint32_t hi = (uint32_t)(mine[0] >> 32), lo = (uint32_t)mine[0];
+        const uint32_t whi = wave_max_u32(hi);
+        const uint32_t wlo = wave_max_u32(hi == whi ? lo : 0u);  // keys are unique (they carry the row): one lane matches both
+        const unsigned long long win = ((unsigned long long)whi << 32) | wlo;
+        if (win != 0 && mine[0] == win) {  // the lane that held the winner moves its list up
+#pragma unroll
+            for (int e = 0; e + 1 < TOPK_PER_LANE; e++) mine[e] = mine[e + 1];
+            mine[TOPK_PER_LANE - 1] = 0;
+        }
+        if (lane == 0) {
+            if (a.keys_out) {
+                a.keys_out[(long long)blockIdx.x * a.cap + r] = win;
+            } else {
+                const uint32_t ordered = (uint32_t)(win >> 32);
+                const uint32_t b = (ordered & 0x80000000u) ? (ordered & 0x7FFFFFFFu) : ~ordered;
+                a.out_idx[r] = win ? ~(uint32_t)win : 0u;
+                a.out_val[r] = win ? __builtin_bit_cast(float, b) : -__builtin_inff();
+            }
+        }
+    }
+}
 
 extern "C" __global__ __launch_bounds__(64) void rlx_topk_select(rlx::TopkArgs a) {
     using namespace rlx;

@@ -257,7 +257,10 @@ def test_topk_and_argmax_at_llama3_vocabulary_size():
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("n,cap", [(1, 1), (63, 63), (1025, 64), (8192, 40), (8193, 1), (8193, 64), (140000, 64)])
+@pytest.mark.parametrize("n,cap", [(1, 1), (63, 63), (1025, 64), (8192, 40), (8193, 1), (8193, 64), (140000, 64),
+                                   # both sides of the lines between winners one by one and a threshold
+                                   (128, 7), (128, 8), (129, 8), (512, 17), (512, 18), (513, 11), (513, 12), (1024, 11), (1025, 1), (8193, 11),
+                                   (8193, 12), (140000, 7), (140000, 11)])
 @pytest.mark.parametrize("distinct", [False, True])
 def test_topk_selection_edges_on_device(n, cap, distinct):
     # Both sides of what the finishing workgroup takes in one go (8192 candidates), a second selection pass (140000 rows leave
