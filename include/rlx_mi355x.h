@@ -166,6 +166,13 @@ int rlx_mi355x_dequant(const rlx_qweight *w, float *out_dev, void *stream);
 int rlx_mi355x_gguf_matmul_bt(const void *x_dev, int x_dtype, const rlx_qweight *w, float *out_dev, int64_t m,
                               void *workspace, size_t workspace_bytes, void *stream);
 size_t rlx_mi355x_gguf_matmul_workspace(int scheme, int x_dtype, int64_t m, int64_t k, int64_t n);
+/* What ..._bt_batch (or, with RLX_I8, ..._bt_prepared) does with `count` matrices [ns[i], k] on one x[m, k] when it is given
+ * `workspace_bytes`: the number of prefill launches (0: the decode kernels, no workspace), or a negative error. A line per launch goes
+ * into `buf` (may be NULL): kernel, matrices, and whether K or the tiles are divided. *want_bytes (may be NULL): the workspace with
+ * which every launch has all the room for partial results it can use - less than the sum of the matrices' own sizes, and at times
+ * more than the largest of them. Needs no GPU; without one the 256 CUs of the part are assumed. No counterpart in the reference. */
+int rlx_mi355x_gguf_matmul_plan(int scheme, int x_dtype, int64_t m, int64_t k, const int64_t *ns, int count, size_t workspace_bytes,
+                                size_t *want_bytes, char *buf, size_t cap);
 /* `count` independent matmuls of one scheme, batch size m and activation dtype in one launch per eight of them:
  * outs_dev[i][m, n_i] = xs_dev[i][m, k_i] . W_i^T. No counterpart in the reference, which runs one thunk per node;
  * the graph level uses it to issue together every DequantMatMul whose inputs are ready at the same point of the

@@ -68,6 +68,7 @@ enum KernelId : int {
 int runtime_init();
 // Launches kernel `id`; `args` points at the kernel's single by-value argument struct (or packed scalars).
 int launch(KernelId id, unsigned gx, unsigned gy, unsigned bx, unsigned shmem, hipStream_t stream, void **params);
+const char *kernel_name(KernelId id);
 int launch3(KernelId id, unsigned gx, unsigned gy, unsigned gz, unsigned bx, unsigned shmem, hipStream_t stream, void **params);
 
 struct DeviceProps {

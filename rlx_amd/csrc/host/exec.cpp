@@ -19,6 +19,7 @@
 struct rlx_qweight;
 extern "C" int rlx_mi355x_gguf_matmul_bt(const void *, int, const rlx_qweight *, float *, int64_t, void *, size_t, void *);
 extern "C" size_t rlx_mi355x_gguf_matmul_workspace(int, int, int64_t, int64_t, int64_t);
+extern "C" int rlx_mi355x_gguf_matmul_plan(int, int, int64_t, int64_t, const int64_t *, int, size_t, size_t *, char *, size_t);
 extern "C" int rlx_mi355x_fake_quantize(const float *, float *, int8_t *, int64_t, int64_t, int64_t, int, int, float, float *, int,
                                         void *, void *);
 extern "C" void rlx_mi355x_qweight_destroy(rlx_qweight *);
@@ -202,6 +203,16 @@ size_t rlx_mi355x_supported_ops(const uint32_t **kinds) {
 }  // extern "C"
 
 // Everything of Backend::compile that needs no device: validation, lowering, schedule, memory plan.
+// The matmuls of a step that convert their activations, those on the same input side by side (else in the graph's order): what
+// the batched entry point puts into one launch.
+static std::vector<uint32_t> matmuls_by_input(const rlx_exec &e, const std::vector<uint32_t> &step) {
+    std::vector<uint32_t> order;
+    for (uint32_t id : step)
+        if (e.nodes[id].d.op_kind == RLX_OP_DEQUANT_MATMUL && !e.nodes[id].x_image) order.push_back(id);
+    std::stable_sort(order.begin(), order.end(), [&](uint32_t a, uint32_t b) { return e.nodes[a].d.inputs[0] < e.nodes[b].d.inputs[0]; });
+    return order;
+}
+
 static std::unique_ptr<rlx_exec> plan_graph(const rlx_graph_desc *g, const rlx_compile_opts *opts) {
     clear_error();
     if (!g || !g->nodes || g->n_nodes == 0 || !g->outputs || g->n_outputs == 0) {
@@ -642,12 +653,7 @@ static std::unique_ptr<rlx_exec> plan_graph(const rlx_graph_desc *g, const rlx_c
     }
     for (size_t si = 0; si < e->steps.size(); si++) {
         const std::vector<uint32_t> &step = e->steps[si];
-        size_t step_ws = 0, step_parts = 0;  // operands of the widest matmul; partial results of every matmul whose K is split
-        auto need = [&](const Node &mm, uint32_t dt) {
-            const size_t ops_only = rlx_mi355x_gguf_matmul_workspace((int)mm.d.scheme, (int)dt, mm.m, mm.k, 0);
-            step_ws = std::max(step_ws, ops_only);
-            return rlx_mi355x_gguf_matmul_workspace((int)mm.d.scheme, (int)dt, mm.m, mm.k, mm.n) - ops_only;
-        };
+        size_t step_ws = 0;  // what the widest launch of the step takes: they follow one another on one stream
         for (uint32_t id : step) {
             Node &nd = e->nodes[id];
             if (!(nd.img_step >= 0 && !nd.keep_f32) && !placed_early[id])  // a FakeQuantize result that only travels as a prefill image has no slot
@@ -665,14 +671,24 @@ static std::unique_ptr<rlx_exec> plan_graph(const rlx_graph_desc *g, const rlx_c
                                              rlx_mi355x_gguf_grouped_matmul_workspace((int)nd.d.scheme, RLX_BF16, nd.m, nd.k, ne));
                 if (need) nd.aux = take(need, (int)si, (int)si);
             }
-            if (nd.d.op_kind == RLX_OP_DEQUANT_MATMUL && nd.m > 16)  // may run the prefill kernels (which one is decided by the input dtype at run time): sized for f32
-                step_parts += std::max(need(nd, RLX_F32), need(nd, RLX_BF16));
             if (nd.x_image) {  // the code image a FakeQuantize writes, and this matrix scaled by its column scales
                 const size_t with_w = rlx_mi355x_gguf_matmul_workspace((int)nd.d.scheme, RLX_I8, nd.m, nd.k, nd.n);
                 step_ws = std::max(step_ws, with_w);  // holds that matmul's own partial results too
             }
         }
-        step_ws += step_parts;
+        // The other prefill matmuls as the run issues them: those on one input side by side, so many to a launch
+        const std::vector<uint32_t> order = matmuls_by_input(*e, step);
+        for (size_t at = 0; at < order.size();) {
+            const Node &mm = e->nodes[order[at]], &x = e->nodes[mm.d.inputs[0]];
+            std::vector<int64_t> ns;
+            for (; at < order.size() && e->nodes[order[at]].d.inputs[0] == mm.d.inputs[0]; at++) ns.push_back(e->nodes[order[at]].n);
+            for (uint32_t dt : {(uint32_t)RLX_F32, (uint32_t)RLX_BF16}) {  // an input's dtype is known when it is written
+                if (x.d.op_kind != RLX_OP_INPUT && (dt == RLX_F32) != (x.d.dtype == RLX_F32)) continue;
+                size_t want = 0;
+                if (rlx_mi355x_gguf_matmul_plan((int)mm.d.scheme, (int)dt, mm.m, mm.k, ns.data(), (int)ns.size(), 0, &want, nullptr, 0) > 0)
+                    step_ws = std::max(step_ws, want);
+            }
+        }
         if (step_ws) {  // one workspace for the whole step; it is born earlier when a FakeQuantize writes the step's image into it
             int birth = (int)si;
             for (const Node &fq : e->nodes)
@@ -896,16 +912,11 @@ static int enqueue_schedule(rlx_exec *e) {
         } else if (nd.d.op_kind == RLX_OP_DEQUANT_MATMUL) {
             // The whole step through the batched entry point: up to 16 / 32 rows it issues one decode launch per eight
             // matrices; above that, matrices that share their input (q, k, v; gate, up) share one conversion of it and
-            // one prefill launch per four, all on the step's single workspace. Matrices on the same input are made
-            // neighbours first (stable, so the order among them is the graph's).
-            std::vector<uint32_t> order(step);
-            std::stable_sort(order.begin(), order.end(), [&](uint32_t a, uint32_t b) {
-                return e->nodes[a].d.inputs[0] < e->nodes[b].d.inputs[0];
-            });
+            // one prefill launch per four, all on the step's single workspace.
             {  // matmuls whose activations a FakeQuantize left in the workspace as a code image: first, while it is intact
                 std::vector<const rlx_qweight *> iw;
                 std::vector<float *> io;
-                for (uint32_t id : order) {
+                for (uint32_t id : step) {
                     Node &mm = e->nodes[id];
                     if (!mm.x_image) continue;
                     Node &w = e->nodes[mm.d.inputs[1]];
@@ -933,9 +944,8 @@ static int enqueue_schedule(rlx_exec *e) {
                 xs.clear();
                 return rc;
             };
-            for (uint32_t id : order) {
+            for (uint32_t id : matmuls_by_input(*e, step)) {
                 Node &mm = e->nodes[id];
-                if (mm.x_image) continue;
                 Node &x = e->nodes[mm.d.inputs[0]];
                 Node &w = e->nodes[mm.d.inputs[1]];
                 if (!w.qw) {

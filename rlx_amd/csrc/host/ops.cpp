@@ -400,7 +400,7 @@ struct GemmPlan {
     size_t xh_bytes, sxh_bytes, fac_bytes;  // the image, the block sums (Q4_K / Q5_K per 32 columns, Q2_K per 16), the per-row prescale factors
     size_t cs_bytes, wimg_bytes;
     size_t part_off;                        // where partial results begin
-    size_t part_bytes;                      // split K of one [m, n] matmul on its own: split x m x n floats (0: no split)
+    size_t part_bytes;                      // the partial results of one launch with room for all it wants (0: it leaves none)
     int sums_kind;                          // act_sums_kind of the scheme the plan was made for
     size_t image_end() const { return fac_bytes + cs_bytes + xh_bytes + sxh_bytes; }
     size_t total() const { return part_bytes ? part_off + part_bytes : image_end() + wimg_bytes; }
@@ -470,7 +470,80 @@ static BigPlan big_plan(int scheme, int xk, int64_t m, int64_t m_rows, int64_t t
     if (t_shared < t_whole) return BigPlan{(int)cus, part};
     return BigPlan{(int)tiles, 0};
 }
-static GemmPlan gemm_plan(int scheme, int xk, int64_t m, int64_t k, int64_t n = 0) {
+// How the launch over `count` matrices [ns[i], k] of one scheme that multiply the same x is carried out, decided here for the launch
+// itself, the workspace queries, the graph planner and the plan query. `part_room`: bytes there are for partial results.
+struct GemmLaunch {
+    KernelId kernel;
+    int groups;                      // rlx_gemm_big_* / rlx_gemm_img_*: workgroups
+    bool shared;                     // rlx_gemm_big_*: tiles shared between workgroups, pieces added by rlx_gemm_big_reduce
+    GemmSplit split[GEMVW_MAX_SEG];  // the other kernels: K slices, of every matrix (rlx_gemvw_*) or, in [0], of all of them
+    size_t part_bytes;               // partial results it leaves
+};
+static GemmLaunch launch_plan(int scheme, int xk, int64_t m, int64_t k, const int64_t *ns, int count, size_t part_room) {
+    scheme = kernel_scheme(scheme);
+    const bool codes = xk == XK_CODES, skinny = gemm_skinny(xk, m);
+    const Layout L = codes ? Layout{64, 0, 0, 0, 0} : layout_of(scheme);
+    const int64_t rv = xk == 0 ? 2 * m : m, m_rows = (rv + 255) / 256 * 256, k_pad = (k + 255) / 256 * 256;
+    int64_t n_sum = 0, tiles_n = 0, half_tiles_n = 0;
+    for (int i = 0; i < count; i++) {
+        n_sum += ns[i];
+        tiles_n += (ns[i] + 255) / 256;
+        half_tiles_n += (ns[i] + 127) / 128;
+    }
+    GemmLaunch g{};
+    if (gemm_wide(scheme, xk, m)) {
+        g.kernel = scheme == SCHEME_Q4_0 ? K_GEMVW_Q4_0 : K_GEMVW_Q8_0;
+        // every 64 image rows are a pass of their own over the weights (a second one finds part of them in L2)
+        size_t launch_bytes = 0;
+        for (int i = 0; i < count; i++) launch_bytes += (size_t)weight_dims(L, ns[i], k).bytes * (size_t)((rv + 63) / 64);
+        for (int i = 0; i < count; i++) {
+            g.split[i] = wide_split(L, weight_dims(L, ns[i], k), m, launch_bytes);
+            if (g.split[i].split > 1) g.part_bytes += (size_t)g.split[i].split * (size_t)m * (size_t)ns[i] * 4;
+        }
+        if (g.part_bytes > part_room) {  // a workspace without room for the slices: every matrix in one piece
+            for (int i = 0; i < count; i++) g.split[i] = GemmSplit{1, (int)((weight_dims(L, ns[i], k).units + 1) / 2 * 2)};
+            g.part_bytes = 0;
+        }
+        return g;
+    }
+    if (!skinny) {
+        const int64_t quads = codes ? k_pad / 128 : (k + L.unit_k - 1) / L.unit_k;
+        const BigPlan bp = big_plan(scheme, xk, m, m_rows, tiles_n, half_tiles_n, n_sum, quads, part_room);
+        if (bp.groups) {
+            g.shared = bp.part_bytes > 0;
+            g.groups = bp.groups;
+            g.part_bytes = bp.part_bytes;
+            g.kernel = !codes                          ? (scheme == SCHEME_Q4_0 ? K_GEMM_BIG_Q4_0 : K_GEMM_BIG_Q8_0)
+                       : !g.shared && k_pad < 2048     ? K_GEMM_IMG_F16W  // short K: the kernel with the shorter way in and out of a tile
+                                                       : K_GEMM_BIG_F16W;
+            return g;
+        }
+    }
+    // Up to 128 image rows run the 64-row tile (the weights are decoded once per 64 rows, but nothing is spent on padding rows); beyond
+    // that the 256-row tile.
+    g.kernel = codes                     ? (skinny ? K_GEMM64_F16W : K_GEMM_F16W)
+               : scheme == SCHEME_Q4K    ? (skinny ? K_GEMM64_Q4_K : K_GEMM_Q4_K)
+               : scheme == SCHEME_Q4_0   ? (skinny ? K_GEMM64_Q4_0 : K_GEMM_Q4_0)
+               : scheme == SCHEME_Q6K    ? (skinny ? K_GEMM64_Q6_K : K_GEMM_Q6_K)
+               : scheme == SCHEME_Q5K    ? (skinny ? K_GEMM64_Q5_K : K_GEMM_Q5_K)
+               : scheme == SCHEME_Q8K    ? (skinny ? K_GEMM64_Q8_K : K_GEMM_Q8_K)
+               : scheme == SCHEME_Q2K    ? (skinny ? K_GEMM64_Q2_K : K_GEMM_Q2_K)
+                                         : (skinny ? K_GEMM64_Q8_0 : K_GEMM_Q8_0);
+    // A workspace sized for fewer slices gets fewer.
+    const int64_t k_units = codes ? k_pad / 64 : (k + L.unit_k - 1) / L.unit_k;  // K units of the operand the kernel reads
+    const int steps_per_unit = L.unit_k / 64;
+    const int64_t gy = skinny ? (rv + 63) / 64 : m_rows / 256;
+    const size_t slice_bytes = (size_t)m * (size_t)n_sum * 4;
+    GemmSplit sp = gemm_split(half_tiles_n, gy, k_units, steps_per_unit, skinny);
+    if (sp.split > 1 && (size_t)sp.split * slice_bytes > part_room)
+        sp = gemm_split(half_tiles_n, gy, k_units, steps_per_unit, skinny, (int)std::max<size_t>(1, part_room / slice_bytes));
+    if (sp.split > 1 && (size_t)sp.split * slice_bytes > part_room) sp = gemm_split(half_tiles_n, gy, k_units, steps_per_unit, skinny, 1);
+    g.split[0] = sp;
+    if (sp.split > 1) g.part_bytes = (size_t)sp.split * slice_bytes;
+    return g;
+}
+// Operands of a prefill matmul and, with `count` matrices in one launch, its partial results.
+static GemmPlan gemm_plan(int scheme, int xk, int64_t m, int64_t k, const int64_t *ns = nullptr, int count = 0) {
     GemmPlan p;
     const int64_t rv = xk == 0 ? 2 * m : m;
     p.m_rows = (rv + 255) / 256 * 256;
@@ -480,24 +553,17 @@ static GemmPlan gemm_plan(int scheme, int xk, int64_t m, int64_t k, int64_t n = 
     p.sxh_bytes = (size_t)p.m_rows * (p.k_pad / 256) * 32 * p.sums_kind;  // 16 or 32 halfs per row and super-block
     p.fac_bytes = ((size_t)m * 8 + 255) & ~(size_t)255;
     p.cs_bytes = xk == XK_CODES ? (size_t)p.k_pad * 4 : 0;
-    p.wimg_bytes = xk == XK_CODES ? (size_t)((n + 255) / 256 * 256) * p.k_pad * 2 : 0;  // whole 256-row tiles of the large-m kernel
+    int64_t widest = 0;
+    for (int i = 0; i < count; i++) widest = std::max(widest, ns[i]);
+    p.wimg_bytes = xk == XK_CODES ? (size_t)((widest + 255) / 256 * 256) * p.k_pad * 2 : 0;  // whole 256-row tiles of the large-m kernels
     p.part_off = xk == XK_CODES ? p.image_end() + p.wimg_bytes
                                 : p.fac_bytes + p.xh_bytes + (size_t)p.m_rows * (p.k_pad / 256) * 32 * ACT_SUMS_KIND_MAX;
-    p.part_bytes = 0;
-    if (n > 0 && gemm_wide(scheme, xk, m)) {
-        const WeightDims D = weight_dims(scheme, n, k);
-        const GemmSplit sp = wide_split(layout_of(scheme), D, m, (size_t)D.bytes * (size_t)((rv + 63) / 64));  // alone in its launch: the most slices it can get
-        if (sp.split > 1) p.part_bytes = (size_t)sp.split * (size_t)m * (size_t)n * 4;
-    } else if (n > 0) {
-        const Layout L = layout_of(scheme);
-        const bool skinny = gemm_skinny(xk, m);
-        const int spu = xk == XK_CODES ? 1 : L.unit_k / 64;
-        const int64_t k_units = xk == XK_CODES ? p.k_pad / 64 : (k + L.unit_k - 1) / L.unit_k;
-        const GemmSplit sp = gemm_split((n + 127) / 128, skinny ? (rv + 63) / 64 : p.m_rows / 256, k_units, spu, skinny);
-        if (sp.split > 1) p.part_bytes = (size_t)sp.split * (size_t)m * (size_t)n * 4;
-        if (!skinny) p.part_bytes = std::max(p.part_bytes, big_plan(scheme, xk, m, p.m_rows, (n + 255) / 256, (n + 127) / 128, n, xk == XK_CODES ? p.k_pad / 128 : k_units, SIZE_MAX).part_bytes);
-    }
+    p.part_bytes = count > 0 ? launch_plan(scheme, xk, m, k, ns, count, SIZE_MAX).part_bytes : 0;
     return p;
+}
+// Matrices on one x that one prefill launch takes
+static int prefill_launch_max(int scheme, int xk, int64_t m) {
+    return xk == XK_CODES ? 1 : gemm_wide(kernel_scheme(scheme), xk, m) ? GEMVW_MAX_SEG : GEMM_MAX_SEG;
 }
 
 // The conversion of x [m, k] into the workspace: one look at every row for its prescale factor (none for binary16: a launch of
@@ -531,14 +597,16 @@ static int launch_xprep(const void *x, int xk, int64_t m, int64_t k, const GemmP
 // them) from the previous launch of a batch on the same stream, so the conversion pass is skipped.
 static int launch_gemm(const void *x, int xk, const rlx_qweight *const *ws, float *const *outs, int count, int64_t m,
                        void *workspace, size_t workspace_bytes, hipStream_t stream, bool prepared = false) {
-    if (count < 1 || count > (gemm_wide(ws[0]->scheme, xk, m) ? GEMVW_MAX_SEG : GEMM_MAX_SEG) || (xk == XK_CODES && count != 1)) {
+    if (count < 1 || count > prefill_launch_max(ws[0]->scheme, xk, m)) {
         set_error("gguf_matmul_bt: %d matrices in one prefill launch", count);
         return RLX_ERR_INVALID;
     }
     const rlx_qweight *w = ws[0];
     const bool codes = xk == XK_CODES;  // the workspace holds a FakeQuantize code image; the weights are scaled into it first
     const Layout L = codes ? Layout{64, 0, 0, 0, 0} : w->layout;
-    const GemmPlan p = gemm_plan(w->scheme, xk, m, w->dims.k, codes ? w->dims.n : 0);  // the operands; partial results are fitted below
+    int64_t ns[GEMVW_MAX_SEG];
+    for (int i = 0; i < count; i++) ns[i] = ws[i]->dims.n;
+    const GemmPlan p = gemm_plan(w->scheme, xk, m, w->dims.k, ns, codes ? 1 : 0);  // the operands; partial results are fitted below
     for (int i = 1; i < count; i++)
         if (ws[i]->scheme != w->scheme || ws[i]->dims.k != w->dims.k || ws[i]->dims.units != w->dims.units ||
             ws[i]->layout.unit_bytes != L.unit_bytes || ws[i]->sc_off() != w->sc_off()) {
@@ -561,7 +629,8 @@ static int launch_gemm(const void *x, int xk, const rlx_qweight *const *ws, floa
     void *sxh = p.sxh_bytes ? (uint8_t *)workspace + p.fac_bytes + p.cs_bytes + p.xh_bytes : nullptr;
     uint8_t *wimg = (uint8_t *)workspace + p.image_end();
     uint8_t *part_base = (uint8_t *)workspace + p.part_off;  // partial results; every part of the workspace is a multiple of 256 bytes
-    const size_t part_room = workspace_bytes > p.part_off ? workspace_bytes - p.part_off : 0;
+    RLX_TRY(runtime_init());  // the plan counts the device's CUs
+    const GemmLaunch g = launch_plan(w->scheme, xk, m, w->dims.k, ns, count, workspace_bytes > p.part_off ? workspace_bytes - p.part_off : 0);
     if (codes) {  // B = fl16(W * diag(s) / S) as stage images; fac holds (1 / S, S) for every row
         WScaleArgs wa{w->dev, wimg, (const float *)((uint8_t *)workspace + p.fac_bytes), fac, w->dims.row_tiles, w->dims.units, (int)p.k_pad, w->sc_off()};
         void *wparams[] = {&wa};
@@ -570,31 +639,18 @@ static int launch_gemm(const void *x, int xk, const rlx_qweight *const *ws, floa
     } else if (!prepared) {
         RLX_TRY(launch_xprep(x, xk, m, w->dims.k, p, workspace, stream));
     }
-    const int64_t k_units = codes ? p.k_pad / 64 : w->dims.units;  // K units of the operand the kernel reads
-
-    if (gemm_wide(w->scheme, xk, m)) {
-        // every 64 image rows are a pass of their own over the weights (a second one finds part of them in L2)
-        const int64_t gy = ((xk == 0 ? 2 * m : m) + 63) / 64;
-        size_t launch_bytes = 0, part_need = 0;
-        for (int i = 0; i < count; i++) launch_bytes += (size_t)ws[i]->dims.bytes * (size_t)gy;
-        GemmSplit sps[GEMVW_MAX_SEG];
-        for (int i = 0; i < count; i++) {
-            sps[i] = wide_split(ws[i]->layout, ws[i]->dims, m, launch_bytes);
-            if (sps[i].split > 1) part_need += (size_t)sps[i].split * (size_t)m * (size_t)ws[i]->dims.n * 4;
-        }
-        if (part_need > part_room)  // a workspace without room for the slices: every matrix in one piece
-            for (int i = 0; i < count; i++) sps[i] = GemmSplit{1, (int)((ws[i]->dims.units + 1) / 2 * 2)};
+    if (g.kernel == K_GEMVW_Q4_0 || g.kernel == K_GEMVW_Q8_0) {
         GemvWArgs wa{};
         long long wgs = 0;
         size_t off = 0;
         for (int i = 0; i < count; i++) {
             float *dst = outs[i];
-            if (sps[i].split > 1) {
+            if (g.split[i].split > 1) {
                 dst = (float *)(part_base + off);
-                off += (size_t)sps[i].split * (size_t)m * (size_t)ws[i]->dims.n * 4;
+                off += (size_t)g.split[i].split * (size_t)m * (size_t)ws[i]->dims.n * 4;
             }
-            wa.seg[i] = GemvWSeg{ws[i]->dev, dst, (int)ws[i]->dims.n, (int)ws[i]->dims.row_tiles, (int)wgs, sps[i].split, sps[i].units_per_split};
-            wgs += (ws[i]->dims.row_tiles + 15) / 16 * sps[i].split;
+            wa.seg[i] = GemvWSeg{ws[i]->dev, dst, (int)ws[i]->dims.n, (int)ws[i]->dims.row_tiles, (int)wgs, g.split[i].split, g.split[i].units_per_split};
+            wgs += (ws[i]->dims.row_tiles + 15) / 16 * g.split[i].split;
         }
         wa.nseg = count;
         wa.m = (int)m;
@@ -604,57 +660,47 @@ static int launch_gemm(const void *x, int xk, const rlx_qweight *const *ws, floa
         wa.xh = xh;
         wa.rowfac = fac;
         void *wparams[] = {&wa};
-        RLX_TRY(launch3(w->scheme == SCHEME_Q4_0 ? K_GEMVW_Q4_0 : K_GEMVW_Q8_0, (unsigned)wgs, (unsigned)gy, 1, 512, 2 * 32768, stream, wparams));
+        RLX_TRY(launch3(g.kernel, (unsigned)wgs, (unsigned)(((xk == 0 ? 2 * m : m) + 63) / 64), 1, 512, 2 * 32768, stream, wparams));
         SplitReduceArgs ra{};
         int nred = 0;
         for (int i = 0; i < count; i++)
-            if (sps[i].split > 1) {
+            if (g.split[i].split > 1) {
                 ra.part[nred] = wa.seg[i].out;
                 ra.out[nred] = outs[i];
                 ra.elems[nred] = (long long)m * ws[i]->dims.n;
-                ra.split[nred++] = sps[i].split;
+                ra.split[nred++] = g.split[i].split;
             }
         return launch_split_reduce(ra, nred, stream);
     }
 
-    if (!gemm_skinny(xk, m)) {
-        RLX_TRY(runtime_init());
+    if (g.kernel == K_GEMM_IMG_F16W) {
+        GemmImgArgs ia{xh, wimg, outs[0], fac, (int)m, (int)w->dims.n, (int)(p.k_pad / 64)};
+        void *iparams[] = {&ia};
+        return launch3(g.kernel, (unsigned)((w->dims.n + 255) / 256), (unsigned)(p.m_rows / 256), 1, 512, 2 * 65536, stream, iparams);
+    }
+    if (g.groups) {
         GemmBigArgs ba{};
-        int64_t small_n = 0, n_sum = 0;
         for (int i = 0; i < count; i++) {
             ba.seg[i] = GemmBigSeg{codes ? (const void *)wimg : ws[i]->dev, outs[i], (int)ws[i]->dims.n, (int)ws[i]->dims.row_tiles, ba.tiles_n};
             ba.tiles_n += (int)((ws[i]->dims.n + 255) / 256);
-            small_n += (ws[i]->dims.n + 127) / 128;
-            n_sum += ws[i]->dims.n;
         }
+        ba.nseg = count;
+        ba.a_img = xh;
+        ba.rowfac = fac;
+        ba.part = (float *)part_base;
+        ba.m_out = (int)m;
+        ba.tiles_m = (int)(p.m_rows / 256);
+        ba.a_steps = (int)(p.k_pad / 64);
         ba.quads = codes ? (int)(p.k_pad / 128) : (int)w->dims.units;
-        const BigPlan bp = big_plan(w->scheme, xk, m, p.m_rows, ba.tiles_n, small_n, n_sum, ba.quads, part_room);
-        if (bp.groups) {
-            ba.nseg = count;
-            ba.a_img = xh;
-            ba.rowfac = fac;
-            ba.part = (float *)part_base;
-            ba.m_out = (int)m;
-            ba.tiles_m = (int)(p.m_rows / 256);
-            ba.a_steps = (int)(p.k_pad / 64);
-            ba.pair_rows = xk == 0 ? 1 : 0;
-            if (codes && !bp.part_bytes && p.k_pad < 2048) {  // short K: the kernel with the shorter way in and out of a tile
-                GemmImgArgs ia{xh, wimg, outs[0], fac, (int)m, (int)w->dims.n, (int)(p.k_pad / 64)};
-                void *iparams[] = {&ia};
-                return launch3(K_GEMM_IMG_F16W, (unsigned)ba.tiles_n, (unsigned)ba.tiles_m, 1, 512, 2 * 65536, stream, iparams);
-            }
-            int groups = bp.groups;
-            void *bparams[] = {&ba, &groups};
-            const KernelId bid = codes ? K_GEMM_BIG_F16W : w->scheme == SCHEME_Q4_0 ? K_GEMM_BIG_Q4_0 : K_GEMM_BIG_Q8_0;
-            RLX_TRY(launch(bid, (unsigned)groups, 1, 256, 5 * 32768, stream, bparams));
-            if (!bp.part_bytes) return RLX_OK;
-            return launch(K_GEMM_BIG_REDUCE, (unsigned)(ba.tiles_m * ba.tiles_n), ba.pair_rows ? 8 : 16, 256, 0, stream, bparams);
-        }
+        ba.pair_rows = xk == 0 ? 1 : 0;
+        int groups = g.groups;
+        void *bparams[] = {&ba, &groups};
+        RLX_TRY(launch(g.kernel, (unsigned)groups, 1, 256, 5 * 32768, stream, bparams));
+        if (!g.shared) return RLX_OK;
+        return launch(K_GEMM_BIG_REDUCE, (unsigned)(ba.tiles_m * ba.tiles_n), ba.pair_rows ? 8 : 16, 256, 0, stream, bparams);
     }
 
     const int steps_per_unit = L.unit_k / 64;
-    // Up to 128 activation rows run the 64-row tile (the weights are decoded once per 64 rows, but nothing is spent on
-    // padding rows); beyond that the 256-row tile.
     const int64_t rv = xk == 0 ? 2 * m : m;
     const bool skinny = gemm_skinny(xk, m);
     GemmArgs a{};
@@ -665,15 +711,9 @@ static int launch_gemm(const void *x, int xk, const rlx_qweight *const *ws, floa
     }
     a.nseg = count;
     const int gy = skinny ? (int)((rv + 63) / 64) : (int)(p.m_rows / 256);
-    // Split K: every slice writes its partial result behind the images in the workspace, then one reduce launch per
-    // matrix adds the slices in ascending K into the output. A workspace sized for fewer slices gets fewer.
-    size_t n_sum = 0;
-    for (int i = 0; i < count; i++) n_sum += (size_t)ws[i]->dims.n;
-    GemmSplit sp = gemm_split(gx, gy, k_units, steps_per_unit, skinny);
-    if (sp.split > 1 && (size_t)sp.split * (size_t)m * n_sum * 4 > part_room)
-        sp = gemm_split(gx, gy, k_units, steps_per_unit, skinny, (int)std::max<size_t>(1, part_room / ((size_t)m * n_sum * 4)));
-    if (sp.split > 1 && (size_t)sp.split * (size_t)m * n_sum * 4 > part_room) sp = gemm_split(gx, gy, k_units, steps_per_unit, skinny, 1);
-    const int split = sp.split, units_per_split = sp.units_per_split;
+    // Split K: every slice writes its partial result behind the images in the workspace, then one reduce launch adds the slices in
+    // ascending K into the outputs.
+    const int split = g.split[0].split, units_per_split = g.split[0].units_per_split;
     if (split > 1) {
         size_t off = 0;
         for (int i = 0; i < count; i++) {
@@ -686,23 +726,14 @@ static int launch_gemm(const void *x, int xk, const rlx_qweight *const *ws, floa
     a.m_rows = (int)p.m_rows;
     a.m_out = (int)m;
     a.k_pad = (int)p.k_pad;
-    a.units = (int)k_units;
+    a.units = codes ? (int)(p.k_pad / 64) : (int)w->dims.units;
     a.pair_rows = xk == 0 ? 1 : 0;
     a.steps_per_split = units_per_split * steps_per_unit;
     a.split_out = split > 1 ? 1 : 0;
     a.sc_off = w->sc_off();
     a.rowfac = fac;
     void *params[] = {&a};
-    KernelId id = codes                         ? (skinny ? K_GEMM64_F16W : K_GEMM_F16W)
-                  : w->scheme == SCHEME_Q4K     ? (skinny ? K_GEMM64_Q4_K : K_GEMM_Q4_K)
-                  : w->scheme == SCHEME_Q4_0    ? (skinny ? K_GEMM64_Q4_0 : K_GEMM_Q4_0)
-                  : w->scheme == SCHEME_Q6K     ? (skinny ? K_GEMM64_Q6_K : K_GEMM_Q6_K)
-                  : w->scheme == SCHEME_Q5K     ? (skinny ? K_GEMM64_Q5_K : K_GEMM_Q5_K)
-                  : w->scheme == SCHEME_Q8K     ? (skinny ? K_GEMM64_Q8_K : K_GEMM_Q8_K)
-                  : w->scheme == SCHEME_Q2K     ? (skinny ? K_GEMM64_Q2_K : K_GEMM_Q2_K)
-                                                : (skinny ? K_GEMM64_Q8_0 : K_GEMM_Q8_0);
-    RLX_TRY(runtime_init());
-    RLX_TRY(launch3(id, (unsigned)gx, (unsigned)gy, (unsigned)split, 512, skinny ? 3 * 24 * 1024 : 3 * 48 * 1024, stream, params));
+    RLX_TRY(launch3(g.kernel, (unsigned)gx, (unsigned)gy, (unsigned)split, 512, skinny ? 3 * 24 * 1024 : 3 * 48 * 1024, stream, params));
     SplitReduceArgs ra{};
     if (split > 1)
         for (int i = 0; i < count; i++) {
@@ -835,10 +866,39 @@ int rlx_mi355x_dequant(const rlx_qweight *w, float *out_dev, void *stream) {
 size_t rlx_mi355x_gguf_matmul_workspace(int scheme, int x_dtype, int64_t m, int64_t k, int64_t n) {
     using namespace rlx;
     if (x_dtype == RLX_I8)  // a FakeQuantize code image and the scaled weights of the widest matrix it is multiplied by
-        return !code_image_scheme(scheme) || m <= 0 || k <= 0 || n < 0 ? 0 : gemm_plan(scheme, XK_CODES, m, k, n).total();
+        return !code_image_scheme(scheme) || m <= 0 || k <= 0 || n < 0 ? 0 : gemm_plan(scheme, XK_CODES, m, k, &n, n > 0).total();
     int xk = x_kind(x_dtype);
     if (xk < 0 || layout_of(scheme).unit_k == 0 || m <= decode_rows(xk)) return 0;  // decode path: no workspace
-    return gemm_plan(scheme, xk, m, k, n < 0 ? 0 : n).total();  // n = 0: the operand image alone (what ..._prepare writes)
+    return gemm_plan(scheme, xk, m, k, &n, n > 0).total();  // n = 0: the operand image alone (what ..._prepare writes)
+}
+
+int rlx_mi355x_gguf_matmul_plan(int scheme, int x_dtype, int64_t m, int64_t k, const int64_t *ns, int count, size_t workspace_bytes,
+                                size_t *want_bytes, char *buf, size_t cap) {
+    using namespace rlx;
+    const int xk = x_dtype == RLX_I8 ? XK_CODES : x_kind(x_dtype);
+    bool ok = ns && count > 0 && xk >= 0 && m > 0 && k > 0 && layout_of(scheme).unit_k != 0 && (xk != XK_CODES || code_image_scheme(scheme));
+    for (int i = 0; ok && i < count; i++) ok = ns[i] > 0;
+    if (!ok) {
+        set_error("gguf_matmul_plan: needs a claimed scheme (Q4_0 / Q8_0 on a code image), F32 / BF16 / F16 / I8 activations and sizes above zero");
+        return RLX_ERR_INVALID;
+    }
+    if (want_bytes) *want_bytes = 0;
+    if (buf && cap) buf[0] = 0;
+    if (xk != XK_CODES && m <= decode_rows(xk)) return 0;
+    size_t pos = 0;
+    int launches = 0;
+    for (int i = 0; i < count; launches++) {
+        const int c = std::min(count - i, prefill_launch_max(scheme, xk, m));
+        const GemmPlan p = gemm_plan(scheme, xk, m, k, ns + i, c);
+        if (want_bytes) *want_bytes = std::max(*want_bytes, p.total());
+        const GemmLaunch g = launch_plan(scheme, xk, m, k, ns + i, c, workspace_bytes > p.part_off ? workspace_bytes - p.part_off : 0);
+        if (buf && pos < cap) {
+            pos += (size_t)snprintf(buf + pos, cap - pos, "%s: %d %s, %s, %zu bytes of partial results\n", kernel_name(g.kernel), c,
+                                    c == 1 ? "matrix" : "matrices", g.shared ? "shared tiles" : g.part_bytes ? "split K" : "whole", g.part_bytes);
+        }
+        i += c;
+    }
+    return launches;
 }
 
 int rlx_mi355x_gguf_matmul_bt_batch(const void *const *xs_dev, int x_dtype, const rlx_qweight *const *ws,
@@ -876,7 +936,7 @@ int rlx_mi355x_gguf_matmul_bt_batch(const void *const *xs_dev, int x_dtype, cons
         int have_sums = 0;
         for (int i = 0; i < count;) {
             int c = 1;
-            const int most = gemm_wide(ws[i]->scheme, xk, m) ? GEMVW_MAX_SEG : GEMM_MAX_SEG;
+            const int most = prefill_launch_max(ws[i]->scheme, xk, m);
             while (i + c < count && c < most && xs_dev[i + c] == xs_dev[i] && ws[i + c]->dims.k == ws[i]->dims.k &&
                    ws[i + c]->layout.unit_bytes == ws[i]->layout.unit_bytes && ws[i + c]->sc_off() == ws[i]->sc_off())
                 c++;

@@ -50,6 +50,7 @@ static const char *const kKernelNames[K_COUNT] = {
     "rlx_gemm_q8_k", "rlx_gemm64_q8_k", "rlx_gemm64g_q8_k", "rlx_gemm_q2_k", "rlx_gemm64_q2_k", "rlx_gemm64g_q2_k",
     "rlx_gemm_f16w", "rlx_gemm64_f16w", "rlx_wscale_q4_0", "rlx_wscale_q8_0", "rlx_splitk_reduce", "rlx_gemm_big_f16w", "rlx_gemm_big_q4_0", "rlx_gemm_big_q8_0", "rlx_gemm_big_reduce", "rlx_gemm_img_f16w", "rlx_gemvw_q4_0", "rlx_gemvw_q8_0", "rlx_gemvwg_q4_0", "rlx_gemvwg_q8_0",
 };
+const char *kernel_name(KernelId id) { return kKernelNames[id]; }
 
 static std::once_flag g_once;
 static int g_init_rc = RLX_ERR_NO_DEVICE;

@@ -1,6 +1,7 @@
 """Operator-level wrappers over the C ABI: device buffers, packed weights, dequant, matmul, FakeQuantize,
 plus the host utilities (encoders, repack, Philox). Thin: every call goes to librlx_mi355x.so."""
 import ctypes as C
+import itertools
 
 import numpy as np
 
@@ -165,6 +166,16 @@ def matmul_workspace_bytes(w: QWeight, x_dtype, m):
     return _lib.lib().rlx_mi355x_gguf_matmul_workspace(int(w.scheme), int(x_dtype), m, w.k, w.n)
 
 
+def matmul_plan(scheme, x_dtype, m, k, ns, workspace_bytes=None):
+    """What a batched prefill matmul of [n, k] matrices on one x[m, k] does: (workspace it can use, a line per launch). Planned with
+    that workspace, or with `workspace_bytes`. No lines: the decode kernels."""
+    want, text = C.c_size_t(), C.create_string_buffer(4096)
+    arr = (C.c_int64 * len(ns))(*ns)
+    room = 2 ** 63 if workspace_bytes is None else workspace_bytes
+    _lib.check(_lib.lib().rlx_mi355x_gguf_matmul_plan(int(scheme), int(x_dtype), m, k, arr, len(ns), room, C.byref(want), text, len(text)))
+    return want.value, text.value.decode().splitlines()
+
+
 def gguf_matmul_bt_device(x_dev, x_dtype, w: QWeight, out_dev, m, stream=None, workspace=None):
     """out_dev[m, n] = x_dev[m, k] . W^T on `stream`. `workspace`: DeviceBuffer of matmul_workspace_bytes() (prefill only)."""
     need = matmul_workspace_bytes(w, x_dtype, m)
@@ -195,7 +206,8 @@ def gguf_matmul_bt_batch(xs, ws, m, x_dtype=DType.F32):
         if id(x) not in bufs:
             bufs[id(x)] = DeviceBuffer.from_numpy(x)
     outs = [DeviceBuffer(m * w.n * 4) for w in ws]
-    need = max(matmul_workspace_bytes(w, x_dtype, m) for w in ws)
+    runs = [[w for _, w in run] for _, run in itertools.groupby(zip(xs, ws), key=lambda xw: id(xw[0]))]  # neighbours on one input share a launch
+    need = max(matmul_plan(run[0].scheme, x_dtype, m, run[0].k, [w.n for w in run])[0] for run in runs)
     workspace = DeviceBuffer(need) if need else None
     n = len(ws)
     xp = (C.c_void_p * n)(*[bufs[id(x)].ptr for x in xs])

@@ -243,6 +243,40 @@ def test_plan_grouped_matmul_workspace_covers_both_input_widths():
     assert int(line.split("workspace@")[1].split("+")[1].split()[0]) >= b16
 
 
+@pytest.mark.parametrize("scheme,m,k,ns", [
+    (QuantScheme.GgufQ8_0, 1111, 4096, [4096, 4096, 4096]),         # each alone shares its tiles, side by side they do not: no room for pieces
+    (QuantScheme.GgufQ4_0, 700, 8192, [3072, 3072]),                # neither alone shares its tiles, side by side they do: room for pieces
+    (QuantScheme.GgufQ4_0, 1300, 8192, [2048, 512, 512]),
+    (QuantScheme.GgufQ4_0, 40, 8192, [4096] * 9),                   # nine matrices of the 64-rows-a-pass kernel: eight and one
+    (QuantScheme.GgufQ6K, 300, 2048, [200, 300, 400, 500, 600]),    # split K, four matrices and one
+])
+def test_plan_step_workspace_follows_the_launches(scheme, m, k, ns):
+    # The matmuls of a step run one launch after another on its one workspace, so it holds what the widest launch can use: not the
+    # partial results of every matrix on its own, which is more where the launch leaves none and less where only the group does.
+    g = Graph.new("group")
+    x = g.input("x", Shape.new([m, k], DType.F32))
+    ys = []
+    for i, n in enumerate(ns):
+        w = g.param(f"w{i}", Shape.new([ops.bytes_for(scheme, n * k)], DType.U8))
+        ys.append(g.add_node(Op.DequantMatMul(scheme), [x, w], Shape.new([m, n], DType.F32)))
+    g.set_outputs(ys)
+    line = Session().plan(g)[1].splitlines()[1 + ys[0]]
+    room = int(line.split("workspace@")[1].split("+")[1].split()[0])
+    want = {dt: ops.matmul_plan(scheme, dt, m, k, ns) for dt in (DType.F32, DType.BF16)}  # an input may be written in either width
+    assert room == max(w[0] for w in want.values())
+    for dt, (_, launches) in want.items():
+        assert ops.matmul_plan(scheme, dt, m, k, ns, room)[1] == launches
+        assert len(launches) == -(-len(ns) // (8 if "gemvw" in launches[0] else 4))
+
+
+def test_matmul_plan_refuses_what_has_no_launch():
+    for args in [(QuantScheme.GgufQ4_0, DType.F32, 0, 256, [16]), (QuantScheme.GgufQ4_0, DType.F32, 64, 256, [0]), (QuantScheme.GgufQ4_0, DType.F32, 64, 256, []),
+                 (QuantScheme.GgufQ4K, DType.I8, 64, 256, [16]), (QuantScheme.GgufQ4_0, DType.U8, 64, 256, [16])]:
+        with pytest.raises(rlx_amd.RlxError):
+            ops.matmul_plan(*args)
+    assert ops.matmul_plan(QuantScheme.GgufQ4_0, DType.F32, 16, 256, [16]) == (0, [])  # decode: no workspace, no prefill launch
+
+
 def _llama_mlp_graph(m, k=256, n=512, norm_is_output=False):
     # RmsNorm -> q, k; RmsNorm -> [up | gate] -> FusedSwiGLU -> down: the ops around the hot path as the reference's
     # graphs hold them (rlx-ir/src/op.rs:574-578, 1157-1172)
