@@ -1,5 +1,6 @@
 """The 256 x 256 tile prefill kernel (csrc/kernels/gemm_big.hip): tiles handed out whole and shared between workgroups, ragged rows, columns
-and K, f32 and 16-bit activations, several matrices in one launch. Sizes are the smallest at which the dispatch takes it."""
+and K, f32 and 16-bit activations, code images, several matrices in one launch. Which of these a size is comes from an estimate of
+times, so every case asks the plan of its launch first: a changed estimate fails here instead of testing another kernel."""
 import ctypes as C
 
 import numpy as np
@@ -14,7 +15,14 @@ pytestmark = pytest.mark.gpu
 TOL = 2e-3  # the matmul's bound: one rounding of d * code to binary16 per weight
 
 
-def run(scheme, m, ns, k, x_dtype, seed, lean=False, offset=0):
+def planned(scheme, m, ns, k, x_dtype, room=None):
+    launches = ops.matmul_plan(scheme, x_dtype, m, k, ns, room)[1]
+    assert len(launches) == 1
+    kernel, rest = launches[0].split(": ")
+    return kernel, rest.split(", ")[1]
+
+
+def run(scheme, m, ns, k, x_dtype, seed, plan, lean=False, offset=0):
     rng = np.random.default_rng(seed)
     x = rng.standard_normal((m, k)).astype(np.float32)
     x[3] *= 3e4  # a row whose values are carried with a power of two
@@ -24,7 +32,8 @@ def run(scheme, m, ns, k, x_dtype, seed, lean=False, offset=0):
     packs = [tiled_packed(scheme, n, k, seed + i, 0.02).reshape(-1) for i, n in enumerate(ns)]
     ws = [ops.QWeight(QuantScheme(scheme), p, n, k) for p, n in zip(packs, ns)]
     L = rlx_amd._lib.lib()
-    need = sum(L.rlx_mi355x_gguf_matmul_workspace(scheme, int(x_dtype), m, k, 0 if lean else n) for n in ns)
+    need = L.rlx_mi355x_gguf_matmul_workspace(scheme, int(x_dtype), m, k, 0) if lean else ops.matmul_plan(scheme, x_dtype, m, k, ns)[0]
+    assert planned(scheme, m, ns, k, x_dtype, need) == plan
     wsb, xd = ops.DeviceBuffer(need), ops.DeviceBuffer.from_numpy(bits if x_dtype == DType.BF16 else x)
     outs = [ops.DeviceBuffer(m * n * 4 + 16) for n in ns]
     xp = (C.c_void_p * len(ns))(*[xd.ptr] * len(ns))
@@ -42,16 +51,17 @@ def run(scheme, m, ns, k, x_dtype, seed, lean=False, offset=0):
     return x, packs, got[0]
 
 
-@pytest.mark.parametrize("scheme,m,ns,k,x_dtype,offset", [
-    (Q4_0, 1111, [4100], 4096, DType.F32, 0),          # shared tiles, ragged rows and columns
-    (Q8_0, 1100, [4093], 4128, DType.F32, 0),          # odd columns: no 16-byte stores; K ends inside a 128-column unit of the image
-    (Q4_0, 1111, [4096], 4096, DType.F32, 4),          # an output that is only 4-byte aligned
-    (Q8_0, 2050, [6143], 8992, DType.BF16, 0),         # a tile per workgroup, 16-bit rows
-    (Q4_0, 1090, [4096, 1030, 1024], 8992, DType.F32, 0),  # three matrices side by side
-    (Q8_0, 2050, [3900], 8192, DType.BF16, 0),         # shared tiles, 16-bit rows
+@pytest.mark.parametrize("scheme,m,ns,k,x_dtype,offset,tiles", [
+    (Q4_0, 1111, [4100], 4096, DType.F32, 0, "shared tiles"),          # ragged rows and columns
+    (Q8_0, 1100, [4093], 4128, DType.F32, 0, "shared tiles"),          # odd columns: no 16-byte stores; K ends inside a 128-column unit of the image
+    (Q4_0, 1111, [4096], 4096, DType.F32, 4, "shared tiles"),          # an output that is only 4-byte aligned
+    (Q8_0, 2050, [6143], 8992, DType.BF16, 0, "whole"),                # a tile per workgroup, 16-bit rows
+    (Q4_0, 1090, [4096, 1030, 1024], 8992, DType.F32, 0, "whole"),     # three matrices side by side
+    (Q4_0, 700, [4096, 1030, 1024], 8192, DType.F32, 0, "shared tiles"),  # the same with pieces of the second and third
+    (Q8_0, 2050, [3900], 8192, DType.BF16, 0, "shared tiles"),         # 16-bit rows
 ])
-def test_large_tiles_match_the_oracle(oracle, scheme, m, ns, k, x_dtype, offset):
-    x, packs, got = run(scheme, m, ns, k, x_dtype, m + k, offset=offset)
+def test_large_tiles_match_the_oracle(oracle, scheme, m, ns, k, x_dtype, offset, tiles):
+    x, packs, got = run(scheme, m, ns, k, x_dtype, m + k, ("rlx_gemm_big_q4_0" if scheme == Q4_0 else "rlx_gemm_big_q8_0", tiles), offset=offset)
     rows = [0, 1, 2, 127, 128, 255, 256, m // 2, m - 2, m - 1]
     for p, n, y in zip(packs, ns, got):
         assert rel_err(y[rows], oracle.gguf_matmul_f64(x[rows], p, len(rows), k, n, scheme)) <= TOL
@@ -65,15 +75,21 @@ def test_large_tiles_match_the_oracle(oracle, scheme, m, ns, k, x_dtype, offset)
 def test_shared_tiles_need_room_for_their_pieces(oracle):
     # without room for partial results the tiles are not shared: the same numbers up to the order of the sums
     m, n, k = 1111, 4100, 4096
-    _, _, full = run(Q4_0, m, [n], k, DType.F32, 5)
-    _, _, lean = run(Q4_0, m, [n], k, DType.F32, 5, lean=True)
+    _, _, full = run(Q4_0, m, [n], k, DType.F32, 5, ("rlx_gemm_big_q4_0", "shared tiles"))
+    _, _, lean = run(Q4_0, m, [n], k, DType.F32, 5, ("rlx_gemm_big_q4_0", "whole"), lean=True)
     keep = np.arange(m) != 3
     assert rel_err(lean[0][keep], full[0][keep].astype(np.float64)) <= 1e-5
 
 
-@pytest.mark.parametrize("m,k,n", [(8192, 512, 3900), (8000, 2048, 4001)])  # code images: short K, and the first K of the four-wave kernel
-def test_code_images_of_many_rows(oracle, m, k, n):
+@pytest.mark.parametrize("m,k,n,plan", [
+    (8192, 512, 3900, ("rlx_gemm_img_f16w", "whole")),         # short K
+    (8000, 2048, 4001, ("rlx_gemm_big_f16w", "whole")),        # the first K of the four-wave kernel
+    (4000, 4096, 2500, ("rlx_gemm_big_f16w", "whole")),        # a single round of whole tiles
+    (2050, 8192, 3900, ("rlx_gemm_big_f16w", "shared tiles")),  # pieces of tiles, a K offset into the ready images
+])
+def test_code_images_of_many_rows(oracle, m, k, n, plan):
     from rlx_amd import Graph, Op, Session, Shape
+    assert planned(Q8_0, m, [n], k, DType.I8) == plan
     rng = np.random.default_rng(k)
     x = rng.standard_normal((m, k)).astype(np.float32)
     packed = tiled_packed(Q8_0, n, k, 7, 0.02).reshape(-1)

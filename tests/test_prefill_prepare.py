@@ -21,18 +21,20 @@ def test_no_image_row_is_read_that_was_not_written(oracle, scheme, m, x_dtype):
     check(oracle, scheme, n, k, m, x_dtype)
 
 
-@pytest.mark.parametrize("m,k", [(2047, 64), (2049, 32), (70, 4064), (70, 4096), (70, 16416)])
-def test_row_scan_by_waves_and_by_workgroups(oracle, m, k):
-    check(oracle, Q4_0, 48, k, m, DType.F32, rows=[0, 3, 5, m // 2, m - 1])
+# a workgroup per row below 2048 rows of 16384 bytes or more, else a wave per row: both sides of both lines
+@pytest.mark.parametrize("m,k,x_dtype", [(2047, 64, DType.F32), (2049, 32, DType.F32), (70, 4064, DType.F32), (70, 4096, DType.F32), (70, 16416, DType.F32),
+                                         (2047, 4096, DType.F32), (2048, 4096, DType.F32), (70, 8160, DType.BF16), (70, 8192, DType.BF16)])
+def test_row_scan_by_waves_and_by_workgroups(oracle, m, k, x_dtype):
+    check(oracle, Q4_0, 48, k, m, x_dtype, rows=[0, 3, 5, m // 2, m - 1])
 
 
-@pytest.mark.parametrize("first,second,m,n,k,x_dtype", [
-    (Q4K, Q4_0, 1111, 4100, 4096, DType.F32),   # shared 256 x 256 tiles leave pieces
-    (Q4K, Q8_0, 40, 1100, 4096, DType.F32),     # K slices of the 64-rows-a-pass kernel
-    (Q2K, Q6K, 40, 200, 2048, DType.BF16),      # split K of the 64-row tiles
-    (Q5K, Q6K, 300, 200, 2048, DType.F32),      # split K of the 256-row tiles
+@pytest.mark.parametrize("first,second,m,n,k,x_dtype,leaves", [
+    (Q4K, Q4_0, 1111, 4100, 4096, DType.F32, "rlx_gemm_big_q4_0: 1 matrix, shared tiles"),  # pieces of tiles
+    (Q4K, Q8_0, 40, 1100, 4096, DType.F32, "rlx_gemvw_q8_0: 1 matrix, split K"),            # 64 rows a pass
+    (Q2K, Q6K, 40, 200, 2048, DType.BF16, "rlx_gemm64_q6_k: 1 matrix, split K"),            # 64-row tiles
+    (Q5K, Q6K, 300, 200, 2048, DType.F32, "rlx_gemm_q6_k: 1 matrix, split K"),              # 256-row tiles
 ])
-def test_an_image_stays_whole_through_matmuls_of_other_schemes(first, second, m, n, k, x_dtype):
+def test_an_image_stays_whole_through_matmuls_of_other_schemes(first, second, m, n, k, x_dtype, leaves):
     # prepared once for a scheme with block sums; between two matmuls of that scheme another scheme's partial results go into the
     # same workspace, which holds what either scheme asks for
     rng = np.random.default_rng(m + n)
@@ -42,6 +44,7 @@ def test_an_image_stays_whole_through_matmuls_of_other_schemes(first, second, m,
     ws = [ops.QWeight(QuantScheme(s), random_blocks(s, n, k, seed=i, d_std=2e-3, dmin_std=2e-3) if s in (Q2K, Q5K, Q6K) else make_weights(s, n, k, seed=i)[0], n, k)
           for i, s in enumerate((first, second))]
     need = max(L.rlx_mi355x_gguf_matmul_workspace(s, int(x_dtype), m, k, n) for s in (first, second))
+    assert leaves in ops.matmul_plan(second, x_dtype, m, k, [n], need)[1][0]
     wsb, od = ops.DeviceBuffer(need), ops.DeviceBuffer(m * n * 4)
     rlx_amd._lib.check(L.rlx_mi355x_gguf_matmul_prepare(xd.ptr, int(x_dtype), first, m, k, wsb.ptr, need, None))
 
