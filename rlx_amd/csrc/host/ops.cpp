@@ -430,46 +430,63 @@ static GemmSplit wide_split(const Layout &L, const WeightDims &D, int64_t m, siz
 }
 // The 256 x 256 tiles of kernels/gemm_big.hip (Q4_0, Q8_0, code images) against the 256 x 128 tiles of kernels/gemm.hip, and how the
 // former are handed out: a tile per workgroup, or the whole line of (tile, 128 columns of K) items in equal runs, one per CU, with
-// the pieces of shared tiles added by a launch of their own. `groups` = 0: the 256 x 128 tiles. Estimated times decide, in us, with what
-// was measured on 2222 image rows of f32 activations in Q4_0: a round of whole tiles costs BIG_ROUND and BIG_QUAD per 128 columns
-// (28672 x 4096: 1008 tiles in four rounds, 480 - 520 us in all), half tiles SMALL_QUAD (the same matrix 526); shared tiles cost
-// SHARE_START more than a round (two epilogues and a second prologue per workgroup), their pieces travel at 5 MB / us each way and the
-// launch that adds them costs 4 us. 144 tiles of 4096 x 14336 (386 us as 288 half tiles in two rounds) take 256 us shared + 16 us for the
-// sum, of 4096 x 4096 96 + 16 against 117; of 3072 x 2048 (1500 rows) 75 against 62, which the estimate leaves to the half tiles.
-// Code images run whole tiles from two rounds on in any case ([8192, 4096] x [4096, 4096] 310 -> 282 us; half tiles 14 % slower at K = 1024).
+// the pieces of shared tiles added by a launch of their own. `groups` = 0: the 256 x 128 tiles. Estimated times decide. Their constants,
+// in us, are fitted to 1740 random shapes and checked on 500 more (130 - 8192 image rows, K 512 - 28672, one to four matrices), each
+// timed all three ways, for f32 rows, 16-bit rows and code images apart: these differ in the bytes of a piece and in what a tile's
+// columns cost (no decode on code images). The whole call is 1.03, 1.02 and 1.12 times as fast there as with the smaller tiles on
+// average (1.4 at best, 0.955 at worst) and within 1 % of the fastest of the three on average. Some of them, smaller / whole / shared:
+// f32 [1111, 14336] x 4096 386 / 385 / 272, [528, 6944] x 3426 102 / 190 / 112; bf16 [1424, 8416] x 2794 125 / 236 / 145; codes
+// [3763, 6432] x 2598 282 / 207 / 288, [3138, 6720] x 5014 359 / 364 / 303.
+// Shared tiles of one row of A are at the same K at the same time, and read A together, where their workgroups, 256 / tiles_n apart, are
+// a whole number apart: gcd(tiles_n, 256) at a time. Alone, each reads A by itself: the kernel on code images of 22 x 12 tiles of 6912
+// columns 212 us, of 24 x 11 tiles 305. Packed weights, whose bytes are a quarter or half, feel it less.
 struct BigPlan {
     int groups;
     size_t part_bytes;
 };
-constexpr double BIG_QUAD = 3.65, BIG_ROUND = 6, SHARE_START = 20, SMALL_QUAD = 2.0, PART_BYTES_US = 5e6, REDUCE_US = 4;
-static BigPlan big_plan(int scheme, int xk, int64_t m, int64_t m_rows, int64_t tiles_n, int64_t small_tiles_n, int64_t n_sum, int64_t quads, size_t part_room) {
+struct BigCosts {
+    double half_start, half_quad;      // a round of 256 x 128 tiles: start, every 128 columns
+    double half_idle;                  // share of it that a last round takes however few its tiles are
+    double split_start, split_byte;    // a split of K on top: its reduce launch, its partial results per byte
+    double whole_start, whole_quad;    // a round of whole 256 x 256 tiles
+    double shared_start, shared_quad;  // shared tiles: two ways in and out of a tile and the reduce launch; every 128 columns of a run
+    double alone, pairs;               // added share of the latter where A is read by one workgroup or two at a time
+    double sparse_margin;              // shared tiles against a grid that is not full: the estimate's error there
+};
+constexpr BigCosts BIG_COSTS_F32{0, 1.64, 0.96, 6.5, 7e-8, 8.2, 2.95, 41.6, 3.04, 0.05, 0.05, 0.956};
+constexpr BigCosts BIG_COSTS_16{0.8, 1.83, 0.85, 6.3, 3.4e-7, 13.1, 3.13, 54.3, 3.5, 0.093, 0.035, 0.948};
+constexpr BigCosts BIG_COSTS_CODES{3.8, 1.485, 0.737, 4.5, 1.2e-7, 14.2, 1.752, 52.7, 2.027, 0.56, 0.137, 0.99};
+constexpr double IMG_START = 5.5, IMG_QUAD = 2.3;  // a round of rlx_gemm_img_f16w, every 128 columns of it
+constexpr int64_t IMG_MAX_K = 2304;              // up to here rlx_gemm_img_f16w instead of rlx_gemm_big_f16w: its way in and out of a tile is shorter (kernels/gemm.hip)
+static BigPlan big_plan(int scheme, int xk, int64_t m, int64_t m_rows, int64_t tiles_n, int64_t half_tiles_n, int64_t n_sum, int64_t quads, size_t part_room) {
     BigPlan none{0, 0};
     if (scheme != SCHEME_Q4_0 && scheme != SCHEME_Q8_0) return none;
+    const bool codes = xk == XK_CODES;
+    const BigCosts &c = codes ? BIG_COSTS_CODES : xk == 0 ? BIG_COSTS_F32 : BIG_COSTS_16;
     const long long cus = device_props().cu_count > 0 ? device_props().cu_count : 256;
-    const long long tiles_m = m_rows / 256, tiles = tiles_m * tiles_n;
-    auto rounds = [&](long long t) { return (double)((t + cus - 1) / cus); };
-    // the 256 x 128 tiles, with the split of K gemm_split gives them
-    const long long small = tiles_m * small_tiles_n;
-    // A single round that leaves CUs idle runs at a higher clock: 1.5 us on 160 half tiles, 1.65 on 192, 2.0 on a full chip
-    double t_small = rounds(small) * (double)quads * SMALL_QUAD * (small < cus ? 0.35 + 0.65 * (double)small / (double)cus : 1.0);
-    if (small * 5 < cus * 4) {
-        const long long split = std::min<long long>(quads, cus / small);
-        t_small = t_small / (double)split + 2.0 * 4.0 * (double)split * (double)m * (double)n_sum / PART_BYTES_US + REDUCE_US;
+    const long long tiles_m = m_rows / 256, tiles = tiles_m * tiles_n, half = tiles_m * half_tiles_n;
+    auto rounds = [&](long long t) { return (t + cus - 1) / cus; };
+    // code images run whole tiles from two rounds on in any case ([8192, 4096] x [4096, 4096] 310 -> 282 us; half tiles 14 % slower at K = 1024)
+    if (codes && tiles >= 2 * cus) return BigPlan{(int)tiles, 0};
+    const bool sparse = half * 5 < cus * 4;  // where gemm_split cuts K if two slices or more find a CU each
+    const long long split = sparse ? std::min<long long>(quads, cus / half) : 1;
+    double t_half;
+    if (split > 1) {
+        t_half = c.half_start + (double)((quads + split - 1) / split) * c.half_quad + c.split_start + c.split_byte * 4.0 * (double)split * (double)m * (double)n_sum;
+    } else {
+        const double last = (double)(half - cus * (rounds(half) - 1)) / (double)cus;
+        t_half = ((double)(rounds(half) - 1) + c.half_idle + (1 - c.half_idle) * last) * (c.half_start + (double)quads * c.half_quad);
     }
-    const double t_whole = rounds(tiles) * (BIG_ROUND + (double)quads * BIG_QUAD);
-    const size_t tile_bytes = (size_t)(xk == 0 ? 128 : 256) * 1024;
-    const size_t part = (size_t)cus * 2 * tile_bytes;
-    double t_shared = 1e30;
+    const double t_whole = (double)rounds(tiles) * (codes && quads * 128 <= IMG_MAX_K ? IMG_START + (double)quads * IMG_QUAD : c.whole_start + (double)quads * c.whole_quad);
+    const bool whole = t_whole < t_half;
+    const size_t part = (size_t)cus * 2 * (size_t)(xk == 0 ? 128 : 256) * 1024;  // a workgroup leaves at most two pieces
     if (part <= part_room && tiles * quads >= cus) {
-        // a workgroup leaves at most two pieces; a tile that is not shared leaves none
-        const double pieces = (double)std::min<long long>(2 * cus, cus + tiles);
-        t_shared = SHARE_START + (double)((tiles * quads + cus - 1) / cus) * BIG_QUAD + 2.0 * pieces * (double)tile_bytes / PART_BYTES_US + REDUCE_US;
+        const double quad = c.shared_quad * (1 + (tiles_n % 2 ? c.alone : tiles_n % 4 ? c.pairs : 0));
+        if (c.shared_start + (double)rounds(tiles * quads) * quad < (sparse ? c.sparse_margin : 1) * (whole ? t_whole : t_half)) return BigPlan{(int)cus, part};
     }
-    if (xk == XK_CODES && tiles >= 2 * cus) return BigPlan{(int)tiles, 0};
-    if (std::min(t_whole, t_shared) > 0.97 * t_small) return none;  // within the error of the estimate: the smaller tile
-    if (t_shared < t_whole) return BigPlan{(int)cus, part};
-    return BigPlan{(int)tiles, 0};
+    return whole ? BigPlan{(int)tiles, 0} : none;
 }
+
 // How the launch over `count` matrices [ns[i], k] of one scheme that multiply the same x is carried out, decided here for the launch
 // itself, the workspace queries, the graph planner and the plan query. `part_room`: bytes there are for partial results.
 struct GemmLaunch {
@@ -513,9 +530,9 @@ static GemmLaunch launch_plan(int scheme, int xk, int64_t m, int64_t k, const in
             g.shared = bp.part_bytes > 0;
             g.groups = bp.groups;
             g.part_bytes = bp.part_bytes;
-            g.kernel = !codes                          ? (scheme == SCHEME_Q4_0 ? K_GEMM_BIG_Q4_0 : K_GEMM_BIG_Q8_0)
-                       : !g.shared && k_pad < 2048     ? K_GEMM_IMG_F16W  // short K: the kernel with the shorter way in and out of a tile
-                                                       : K_GEMM_BIG_F16W;
+            g.kernel = !codes                            ? (scheme == SCHEME_Q4_0 ? K_GEMM_BIG_Q4_0 : K_GEMM_BIG_Q8_0)
+                       : !g.shared && k_pad <= IMG_MAX_K ? K_GEMM_IMG_F16W
+                                                         : K_GEMM_BIG_F16W;
             return g;
         }
     }

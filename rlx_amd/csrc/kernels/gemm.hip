@@ -710,9 +710,9 @@ __device__ __forceinline__ void gemm_body(const GemmArgs &a) {
 }
 
 // Two ready operand images (SCHEME_F16W), many rows, short K: eight waves of 128 x 64 on a 256 x 256 tile, two 64 KB LDS stages filled by
-// buffer loads while the other is multiplied, one barrier per 64 columns. From 2048 columns on rlx_gemm_big_f16w is faster (4096: 228 us
+// buffer loads while the other is multiplied, one barrier per 64 columns. Above 2304 columns rlx_gemm_big_f16w is faster (4096: 228 us
 // against 211); below, its longer way in and out of a tile costs more than its loop saves: whole chain [8192, 1024] x [4096, 1024] 105 us
-// against 112, at 512 columns 73 against 84.
+// against 112, at 512 columns 73 against 84; a round of tiles is 5 us shorter at 1536 columns, as long at 2304, 7 us longer at 3072.
 constexpr int IMG_STAGE = 2 * GEMM_STAGE_A;
 struct GemmImgArgs {
     const uint8_t *a_img;  // [m_rows / 256][steps][32 KB]

@@ -52,7 +52,7 @@ def run(scheme, m, ns, k, x_dtype, seed, plan, lean=False, offset=0):
 
 
 @pytest.mark.parametrize("scheme,m,ns,k,x_dtype,offset,tiles", [
-    (Q4_0, 1111, [4100], 4096, DType.F32, 0, "shared tiles"),          # ragged rows and columns
+    (Q4_0, 1111, [4100], 4608, DType.F32, 0, "shared tiles"),          # ragged rows and columns
     (Q8_0, 1100, [4093], 4128, DType.F32, 0, "shared tiles"),          # odd columns: no 16-byte stores; K ends inside a 128-column unit of the image
     (Q4_0, 1111, [4096], 4096, DType.F32, 4, "shared tiles"),          # an output that is only 4-byte aligned
     (Q8_0, 2050, [6143], 8992, DType.BF16, 0, "whole"),                # a tile per workgroup, 16-bit rows
@@ -74,18 +74,21 @@ def test_large_tiles_match_the_oracle(oracle, scheme, m, ns, k, x_dtype, offset,
 
 def test_shared_tiles_need_room_for_their_pieces(oracle):
     # without room for partial results the tiles are not shared: the same numbers up to the order of the sums
-    m, n, k = 1111, 4100, 4096
+    m, n, k = 1111, 4100, 4608
     _, _, full = run(Q4_0, m, [n], k, DType.F32, 5, ("rlx_gemm_big_q4_0", "shared tiles"))
-    _, _, lean = run(Q4_0, m, [n], k, DType.F32, 5, ("rlx_gemm_big_q4_0", "whole"), lean=True)
+    plan = planned(Q4_0, m, [n], k, DType.F32, 0)
+    assert plan[1] == "whole"
+    _, _, lean = run(Q4_0, m, [n], k, DType.F32, 5, plan, lean=True)
     keep = np.arange(m) != 3
     assert rel_err(lean[0][keep], full[0][keep].astype(np.float64)) <= 1e-5
 
 
 @pytest.mark.parametrize("m,k,n,plan", [
     (8192, 512, 3900, ("rlx_gemm_img_f16w", "whole")),         # short K
-    (8000, 2048, 4001, ("rlx_gemm_big_f16w", "whole")),        # the first K of the four-wave kernel
+    (8000, 2304, 4001, ("rlx_gemm_img_f16w", "whole")),        # the last K of the eight-wave kernel
+    (8000, 2336, 4001, ("rlx_gemm_big_f16w", "whole")),        # the first K of the four-wave kernel, ragged
     (4000, 4096, 2500, ("rlx_gemm_big_f16w", "whole")),        # a single round of whole tiles
-    (2050, 8192, 3900, ("rlx_gemm_big_f16w", "shared tiles")),  # pieces of tiles, a K offset into the ready images
+    (2050, 6016, 7500, ("rlx_gemm_big_f16w", "shared tiles")),  # pieces of tiles, a K offset into the ready images
 ])
 def test_code_images_of_many_rows(oracle, m, k, n, plan):
     from rlx_amd import Graph, Op, Session, Shape

@@ -269,6 +269,21 @@ def test_plan_step_workspace_follows_the_launches(scheme, m, k, ns):
         assert len(launches) == -(-len(ns) // (8 if "gemvw" in launches[0] else 4))
 
 
+@pytest.mark.parametrize("scheme,x_dtype,m,k,ns,faster", [
+    # whole calls in us: 256 x 128 tiles / whole 256 x 256 tiles / shared ones
+    (QuantScheme.GgufQ8_0, DType.F32, 2565, 3488, [3155, 3174], "rlx_gemm_q8_0"),               # 305 / 340 / 323
+    (QuantScheme.GgufQ4_0, DType.F32, 1357, 2848, [8523, 5712, 9088, 488], "rlx_gemm_q4_0"),    # 436 / 464 / 455
+    (QuantScheme.GgufQ4_0, DType.F32, 528, 6944, [3426], "rlx_gemm_q4_0"),                      # 102 / 190 / 112, K split
+    (QuantScheme.GgufQ4_0, DType.F32, 1111, 14336, [4096], "rlx_gemm_big_q4_0"),                # 386 / 385 / 272
+    (QuantScheme.GgufQ4_0, DType.BF16, 361, 3904, [2604, 3163, 290, 11691], "rlx_gemm_q4_0"),   # 120 / 126 / 132
+    (QuantScheme.GgufQ8_0, DType.BF16, 1792, 7584, [11351], "rlx_gemm_q8_0"),                   # 376 / 452 / 394
+    (QuantScheme.GgufQ8_0, DType.I8, 1588, 7360, [6223], "rlx_gemm_big_f16w: 1 matrix, whole"),  # 301 / 222 / 309
+    (QuantScheme.GgufQ4_0, DType.I8, 7766, 1856, [6338], "rlx_gemm_img_f16w"),                  # 332 on rlx_gemm_big_f16w, 308 on this
+])
+def test_plan_takes_the_way_that_was_measured_faster(scheme, x_dtype, m, k, ns, faster):
+    assert ops.matmul_plan(scheme, x_dtype, m, k, ns)[1][0].startswith(faster)
+
+
 def test_matmul_plan_refuses_what_has_no_launch():
     for args in [(QuantScheme.GgufQ4_0, DType.F32, 0, 256, [16]), (QuantScheme.GgufQ4_0, DType.F32, 64, 256, [0]), (QuantScheme.GgufQ4_0, DType.F32, 64, 256, []),
                  (QuantScheme.GgufQ4K, DType.I8, 64, 256, [16]), (QuantScheme.GgufQ4_0, DType.U8, 64, 256, [16])]:

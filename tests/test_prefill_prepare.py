@@ -29,7 +29,7 @@ def test_row_scan_by_waves_and_by_workgroups(oracle, m, k, x_dtype):
 
 
 @pytest.mark.parametrize("first,second,m,n,k,x_dtype,leaves", [
-    (Q4K, Q4_0, 1111, 4100, 4096, DType.F32, "rlx_gemm_big_q4_0: 1 matrix, shared tiles"),  # pieces of tiles
+    (Q4K, Q4_0, 1111, 4100, 4608, DType.F32, "rlx_gemm_big_q4_0: 1 matrix, shared tiles"),  # pieces of tiles
     (Q4K, Q8_0, 40, 1100, 4096, DType.F32, "rlx_gemvw_q8_0: 1 matrix, split K"),            # 64 rows a pass
     (Q2K, Q6K, 40, 200, 2048, DType.BF16, "rlx_gemm64_q6_k: 1 matrix, split K"),            # 64-row tiles
     (Q5K, Q6K, 300, 200, 2048, DType.F32, "rlx_gemm_q6_k: 1 matrix, split K"),              # 256-row tiles
