@@ -342,22 +342,16 @@ __device__ __forceinline__ void compute_unit(const UnitRegs<SCHEME> &w, const ha
         uint32_t sc[2], mn[2];
         q4k_scales(w.meta[1], w.meta[2], w.meta[3], sc, mn);
         float psum[4] = {0.f, 0.f, 0.f, 0.f}, msum[4] = {0.f, 0.f, 0.f, 0.f};  // RG == 1: the super-block's two sums per output row
-        // The min term, sum over the blocks of mn * (sum of x over the block). With one activation row (NREG == 2) a table of block sums in
-        // LDS and one multiply-add per block and row. With more rows it is a matrix product of its own on the same activation
-        // fragments: B = mn in every place, exact, eight instructions chained in smin; no table to make between two barriers, no
-        // reads of it, four multiply-adds per block less. 4096 x 14336 at six f32 rows 26.3 -> 22.4 us; on the 128256-row LM head at one
-        // row the other way round, 61.5 against 54.4.
-        constexpr bool MIN_MFMA = NREG == 4;
-        float4_t smin[RG];
-        auto splat_min = [&](int h, int t) {
-            const half2_t m2 = splat_code_half(mn[h], t);
-            Frag f;
+        // The min term, sum over the blocks of mn * (sum of x over the block). The block sums come from a table in LDS where a launch has
+        // one f32 row or two 16-bit rows (NREG == 2), else from a matrix product of the activation fragments with ones: no table to make
+        // between two barriers, no reads of it. Six f32 rows of a Llama-3-8B layer 78.1 -> 73.2 us, 17 bf16 rows of [8192, 8192] 28.3 ->
+        // 25.2; the LM head at one row the other way round, 54.4 from the table against 61.5. The products stay block by block: chained
+        // over the super-block with B = mn they are 1 - 4 % faster, but the two terms no longer cancel as they go, and the error against
+        // 64 bits grows from 1.5e-7 to 6e-7 (Q5_K) or 9e-7 (Q4_K, two groups) on activations with a mean of 0.3.
+        constexpr bool SUMS_MFMA = NREG == 4;
+        Frag ones;
 #pragma unroll
-            for (int e = 0; e < 4; e++) f.h2[e] = m2;
-            return f;
-        };
-#pragma unroll
-        for (int rg = 0; rg < RG; rg++) smin[rg] = zero;
+        for (int e = 0; e < 4; e++) ones.h2[e] = half2_t{(half_t)1.0f, (half_t)1.0f};
 #pragma unroll
         for (int h = 0; h < 2; h++) {
             Frag b[4];
@@ -369,12 +363,12 @@ __device__ __forceinline__ void compute_unit(const UnitRegs<SCHEME> &w, const ha
                 else unpack_q4<0>(q[t], b[t]);
             }
             if constexpr (RG == 1) {
-                float4_t blk[4];
+                float4_t blk[4], sx[4];
 #pragma unroll
                 for (int t = 0; t < 4; t++) blk[t] = mfma16(a[t], b[t], zero);
-                if constexpr (MIN_MFMA) {
+                if constexpr (SUMS_MFMA) {
 #pragma unroll
-                    for (int t = 0; t < 4; t++) smin[0] = mfma16(a[t], splat_min(h, t), smin[0]);
+                    for (int t = 0; t < 4; t++) sx[t] = mfma16(a[t], ones, zero);
                 }
                 // Q4_K: the super-block's d and dmin are applied once, to the sums of sc * (block product) and of m * (block's
                 // activation sum) over its eight blocks: one conversion and one multiply-add per block, row and term
@@ -384,16 +378,15 @@ __device__ __forceinline__ void compute_unit(const UnitRegs<SCHEME> &w, const ha
                 for (int t = 0; t < 4; t++) {
                     const float scf = ubyte_to_float(sc[h], t), mnf = ubyte_to_float(mn[h], t);
                     // sum of the activations of this 32-column block for the four output rows this lane holds
-                    float4_t sx = zero;
-                    if constexpr (!MIN_MFMA) sx = *(const float4_t *)(sxs + (ublk + 4 * h + t) * 16 + 4 * g);
+                    if constexpr (!SUMS_MFMA) sx[t] = *(const float4_t *)(sxs + (ublk + 4 * h + t) * 16 + 4 * g);
 #pragma unroll
                     for (int r = 0; r < NREG; r++) {
                         if constexpr (SCHEME == SCHEME_Q4K) {
                             psum[r] = __builtin_fmaf(scf, blk[t][r], psum[r]);
-                            if constexpr (!MIN_MFMA) msum[r] = __builtin_fmaf(mnf, sx[r], msum[r]);
+                            msum[r] = __builtin_fmaf(mnf, sx[t][r], msum[r]);
                         } else {
                             acc[0][r] = __builtin_fmaf(d * scf, blk[t][r], acc[0][r]);
-                            if constexpr (!MIN_MFMA) acc[0][r] = __builtin_fmaf(-(dmin * mnf), sx[r], acc[0][r]);
+                            acc[0][r] = __builtin_fmaf(-(dmin * mnf), sx[t][r], acc[0][r]);
                         }
                     }
                 }
@@ -401,7 +394,7 @@ __device__ __forceinline__ void compute_unit(const UnitRegs<SCHEME> &w, const ha
 #pragma unroll
                     for (int r = 0; r < NREG; r++) {
                         acc[0][r] = __builtin_fmaf(d, psum[r], acc[0][r]);
-                        if constexpr (!MIN_MFMA) acc[0][r] = __builtin_fmaf(-dmin, msum[r], acc[0][r]);
+                        acc[0][r] = __builtin_fmaf(-dmin, msum[r], acc[0][r]);
                     }
                 }
             } else {
@@ -410,28 +403,25 @@ __device__ __forceinline__ void compute_unit(const UnitRegs<SCHEME> &w, const ha
 #pragma unroll
                 for (int t = 0; t < 4; t++) {
                     const float dj = d * ubyte_to_float(sc[h], t);
-                    const Frag fm = splat_min(h, t);
-                    float4_t blk[RG];
+                    const float mj = dmin * ubyte_to_float(mn[h], t);
+                    float4_t blk[RG], sx[RG];
 #pragma unroll
                     for (int rg = 0; rg < RG; rg++) {
                         Frag af;
                         af.u4 = *(const uint4_t *)(xrow[rg] + ucol + h * 128 + t * 32);
                         blk[rg] = mfma16(af, b[t], zero);
-                        smin[rg] = mfma16(af, fm, smin[rg]);
+                        sx[rg] = mfma16(af, ones, zero);
                     }
 #pragma unroll
                     for (int rg = 0; rg < RG; rg++)
 #pragma unroll
-                        for (int r = 0; r < NREG; r++) acc[rg][r] = __builtin_fmaf(dj, blk[rg][r], acc[rg][r]);
+                        for (int r = 0; r < NREG; r++) {
+                            acc[rg][r] = __builtin_fmaf(dj, blk[rg][r], acc[rg][r]);
+                            acc[rg][r] = __builtin_fmaf(-mj, sx[rg][r], acc[rg][r]);
+                        }
                     __builtin_amdgcn_sched_barrier(0);
                 }
             }
-        }
-        if constexpr (MIN_MFMA) {
-#pragma unroll
-            for (int rg = 0; rg < RG; rg++)
-#pragma unroll
-                for (int r = 0; r < NREG; r++) acc[rg][r] = __builtin_fmaf(-dmin, smin[rg][r], acc[rg][r]);
         }
     }
 }

@@ -305,6 +305,35 @@ def test_k_quant_matmul_error_is_below_a_binary16_rounding_of_the_weights(scheme
 
 
 @pytest.mark.gpu
+@pytest.mark.gpu
+@pytest.mark.parametrize("scheme,m,dtype", [(Q5K, 3, DType.F32), (Q5K, 6, DType.F32), (Q5K, 12, DType.F32), (Q5K, 24, DType.BF16),
+                                            (Q4K, 12, DType.F32), (Q4K, 24, DType.BF16)])
+def test_min_term_cancels_block_by_block(scheme, m, dtype):
+    # Weights around zero with the minimum in the middle of the codes, activations with a mean: sc * d * q and mn * dmin are both
+    # several times their difference. Every block adds both to the f32 accumulator, one after the other, so the accumulator stays near the
+    # size of the result: 64 roundings of at most 2^-25 of it at k = 1024, a random walk of 2.4e-7 at most. Summed apart over a
+    # super-block and then subtracted, they leave 6e-7 and more.
+    n, k = 256, 1024
+    rng = np.random.default_rng(m)
+    p = rng.integers(0, 256, (n * k // 256, BLOCK[scheme][1]), dtype=np.uint8)
+    d = (rng.uniform(0.6, 1.4, len(p)) * 1e-4).astype(np.float16)
+    mid = 15.5 if scheme == Q5K else 7.5
+    p[:, 0:2] = d.view(np.uint8).reshape(-1, 2)
+    p[:, 2:4] = (mid * d.astype(np.float32)).astype(np.float16).view(np.uint8).reshape(-1, 2)
+    p[:, 8:12] = p[:, 4:8]                      # mn = sc in all eight blocks
+    p[:, 12:16] = (p[:, 12:16] & 0xF) * 17
+    x = rng.standard_normal((m, k)).astype(np.float32) + np.float32(0.3)
+    xin = x
+    if dtype == DType.BF16:
+        xin = (x.view(np.uint32) >> 16).astype(np.uint16)
+        x = (xin.astype(np.uint32) << 16).view(np.float32)
+    w = ops.QWeight(QuantScheme(scheme), p.reshape(-1), n, k)
+    got = ops.gguf_matmul_bt(xin, w, m, dtype)
+    want = oracle.gguf_matmul_f64(x, p.reshape(-1), m, k, n, scheme)
+    assert np.linalg.norm(got - want) <= 2.4e-7 * np.linalg.norm(want)
+    w.free()
+
+
 def test_q8k_layout_for_n_gt_1():
     """rlx-runtime/tests/dequant_matmul_gguf.rs:176-240: weight [n, k] row-major in blocks, out[mi, j] = sum_p x[mi, p] w[j, p]."""
     m, k, n = 2, 256, 3
