@@ -732,13 +732,14 @@ def other_configs(rlx_amd, stream, with_cpu):
     ms_mm = time_launches(ops, stream, mm_image, 30, 5)
     ms_fqi = time_launches(ops, stream, fq_image, 60, 5)
     flop = 2.0 * rows * cols * n
+    mm_kernel = ops.matmul_plan(QuantScheme.GgufQ8_0, DType.I8, rows, cols, [n])[1][0].split(":")[0]
     cpu_rows = 8  # the scalar loop is linear in the rows of x
     out["config4_fake_quantize_then_q8_0_gemm_8192x4096x4096"] = {
         "us_chain": round(ms_chain * 1e3, 1), "us_fake_quantize_writing_the_code_image": round(ms_fqi * 1e3, 1),
         "us_matmul_from_the_image": round(ms_mm * 1e3, 1), "TFLOP/s_matmul": round(flop / ms_mm / 1e9, 1),
         "roofline": {"bound": "mfma", "frac": round(flop / ms_mm / 1e9 / MFMA_F16_PEAK_TFLOPS, 4),
                      "frac_chain": round(flop / ms_chain / 1e9 / MFMA_F16_PEAK_TFLOPS, 4)},
-        "flop": flop, "launches": "rlx_fq_col_absmax + rlx_fq_scale_parts + rlx_fq_col_apply_img | rlx_wscale_q8_0 + rlx_gemm_f16w",
+        "flop": flop, "launches": "rlx_fq_col_absmax + rlx_fq_scale_parts + rlx_fq_col_apply_img | rlx_wscale_q8_0 + " + mm_kernel,
         "note": "the matmul runs on the integer codes (exact in binary16, one MFMA row per token) against W * diag(s) rounded once to binary16",
         "cpu_baseline": cpu(lambda: oracle.gguf_matmul_bt(xq0[:cpu_rows * cols], _packed_of(ops, QuantScheme.GgufQ8_0, n, cols, 45, 0.02), cpu_rows, cols, n,
                                                           oracle.Q8_0), 2.0 * cpu_rows * cols * n / 1e12, "TFLOP/s")}
@@ -777,13 +778,15 @@ def other_configs(rlx_amd, stream, with_cpu):
         total_ms = time_launches(ops, stream, layer, 30 if m > 16 else 100, 10)
         ops.sync(stream)
         flops = sum(2.0 * m * nn * kk for _, nn, kk in shapes70)
+        plans = [ops.matmul_plan(QuantScheme.GgufQ4_0, DType.BF16, m, kk, [nn for _, nn, k2 in shapes70[a:b]], need)[1] for a, b, kk in ((0, 6, 8192), (6, 7, 28672))]
+        prefill = sorted({line.split(":")[0] for lines in plans for line in lines})
         algo = wbytes + sum(2 * m * kk + 4 * m * nn for _, nn, kk in shapes70)
         t_hbm, t_mfma = algo / (HBM_PEAK_GBS * 1e9), flops / (MFMA_F16_PEAK_TFLOPS * 1e12)
         sweep[f"M={m}"] = {"us_layer": round(total_ms * 1e3, 1), "GB/s": round(algo / total_ms / 1e6, 1),
                            "TFLOP/s": round(flops / total_ms / 1e9, 2),
                            "roofline": {"bound": "hbm" if t_hbm >= t_mfma else "mfma", "frac": round(max(t_hbm, t_mfma) / (total_ms * 1e-3), 4)},
-                           "kernels": "rlx_gemv_q4_0_* (one batched launch)" if m <= 32 else
-                                      ("rlx_xprep + rlx_gemvw_q4_0" if m <= 192 else "rlx_xprep + rlx_gemm_q4_0") + " (+ rlx_splitk_reduce where K is cut)"}
+                           "kernels": "rlx_gemv_q4_0_* (one batched launch)" if not prefill else
+                                      "rlx_xprep + " + " / ".join(prefill) + " (+ rlx_splitk_reduce where K is cut)"}
         for bfr in list(bufs.values()) + list(outs.values()) + ([ws] if ws else []):
             bfr.free()
     if with_cpu:  # the q projection at M = 1, in full
