@@ -305,7 +305,6 @@ def test_k_quant_matmul_error_is_below_a_binary16_rounding_of_the_weights(scheme
 
 
 @pytest.mark.gpu
-@pytest.mark.gpu
 @pytest.mark.parametrize("scheme,m,dtype", [(Q5K, 3, DType.F32), (Q5K, 6, DType.F32), (Q5K, 12, DType.F32), (Q5K, 24, DType.BF16),
                                             (Q4K, 12, DType.F32), (Q4K, 24, DType.BF16)])
 def test_min_term_cancels_block_by_block(scheme, m, dtype):
@@ -334,6 +333,7 @@ def test_min_term_cancels_block_by_block(scheme, m, dtype):
     w.free()
 
 
+@pytest.mark.gpu
 def test_q8k_layout_for_n_gt_1():
     """rlx-runtime/tests/dequant_matmul_gguf.rs:176-240: weight [n, k] row-major in blocks, out[mi, j] = sum_p x[mi, p] w[j, p]."""
     m, k, n = 2, 256, 3
