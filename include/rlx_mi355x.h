@@ -155,10 +155,10 @@ int rlx_mi355x_dequant(const rlx_qweight *w, float *out_dev, void *stream);
  * x_dev is [m,k] row-major of x_dtype in {RLX_F32, RLX_BF16, RLX_F16}; 16-bit activations stand for the values
  * the reference's typed boundary would widen to f32 (rlx-runtime/src/backend.rs:49-53). out_dev is f32.
  * `workspace` must hold rlx_mi355x_gguf_matmul_workspace() bytes (may be NULL when that is 0): the converted
- * activations and, where the output tiles alone would leave most of the chip idle and K is cut across workgroups, the
- * partial results of the K slices, which a reduce launch adds in ascending K (the order the reference walks a row in), so
+ * activations and, where the output tiles alone would leave CUs idle and K or a tile is cut across workgroups, the
+ * partial results, which a reduce launch adds in ascending K (the order the reference walks a row in), so
  * results are the same bits on every run. A workspace that holds only the activations (n = 0 in the size call) is
- * accepted: K is then cut in fewer slices or not at all.
+ * accepted: K is then cut in fewer slices or not at all, and no tile is shared.
  * m <= 16 (f32 activations) or m <= 32 (bf16 / f16) runs the decode kernels (weights streamed once, MFMA 16x16x32, one
  * or two groups of 16 rows per decoded weight fragment, an f32 row taking two); larger m converts the activations once
  * (binary16 image in the workspace) and runs, for Q4_0 / Q8_0 up to 192 image rows, a kernel that still decodes the

@@ -193,14 +193,6 @@ __device__ __forceinline__ half2_t ubyte_bias(int off) {
     return half2_t{v, v};
 }
 
-// half2 (v, v) with v = byte `byte` of word as an exact binary16 integer: bytes [b, 0x64, b, 0x64] = 1024 + b
-__device__ __forceinline__ half2_t splat_code_half(uint32_t word, int byte) {
-    uint32_t sel = 0x04000400u | (uint32_t)byte | ((uint32_t)byte << 16);
-    half2_t t = as_half2(__builtin_amdgcn_perm(0x64646464u, word, sel));
-    const half2_t k1024 = {(half_t)1024.0f, (half_t)1024.0f};
-    return t - k1024;
-}
-
 __device__ __forceinline__ float ubyte_to_float(uint32_t w, int byte) { return (float)((w >> (8 * byte)) & 0xFFu); }
 
 // D(16x16) += A(16x32) * B(32x16), halfs in, f32 accumulate. Lane l: A row / B column l & 15, k-slice 8*(l>>4)..+7;

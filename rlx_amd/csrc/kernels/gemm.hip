@@ -50,6 +50,14 @@ struct GemmArgs {
     long long slab_bytes;
 };
 
+// half2 (v, v) with v = byte `byte` of word as an exact binary16 integer: bytes [b, 0x64, b, 0x64] = 1024 + b
+__device__ __forceinline__ half2_t splat_code_half(uint32_t word, int byte) {
+    uint32_t sel = 0x04000400u | (uint32_t)byte | ((uint32_t)byte << 16);
+    half2_t t = as_half2(__builtin_amdgcn_perm(0x64646464u, word, sel));
+    const half2_t k1024 = {(half_t)1024.0f, (half_t)1024.0f};
+    return t - k1024;
+}
+
 // LDS slot of (k-slice ks, sub-tile s of NS, row r in 0..31, half h): lanes r + 32 h; the low bits of the lane are
 // XORed with c = 2 ks + h so that the eight 16-byte stores of one activation row, and the stores of the decode
 // threads, land in eight different bank groups. Reads of one fragment are a permutation of 64 consecutive slots.

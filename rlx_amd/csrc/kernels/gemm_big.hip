@@ -8,14 +8,15 @@
 //
 // Four waves, one per SIMD, own 128 x 128 of the 256 x 256 tile each (256 accumulator registers): sixteen fragment reads feed 64
 // matrix instructions. K advances in 32-column quanta through a ring of LDS slots that buffer loads fill directly; one barrier per
-// quantum. What bounds it is power: on all-zero operands the ready-image kernel reaches 1.55 PFLOP/s, on real ones 1.3 in a burst and 1.1
-// - 1.2 sustained. 16 x 16 x 32 instructions read and write half the accumulator bits per product of 32 x 32 x 16 ones: [8192, 4096]
-// x [4096, 4096] on ready images 210 us against 229 (and 232 for eight waves of 128 x 64 on 32 x 32 x 16, the kernel before).
+// quantum. What bounds it is the loop: [8192, 4096] x [4096, 4096] on ready images takes 450 K clocks, on drawn data as on zeros, and
+// the matrix unit is busy for 57 % of them; the data moves the clock by a tenth (2.09 against 2.32 GHz: 219 against 193 us in a burst,
+// 1.2 PFLOP/s sustained). 16 x 16 x 32 instructions read and write half the accumulator bits per product of 32 x 32 x 16 ones: 210 us
+// against 229 (and 232 for eight waves of 128 x 64 on 32 x 32 x 16, the kernel before).
 // An XCD-wise tile order and a ring without address arithmetic (four slots, depth two) measured the same or 2 % slower.
 //
 // Decoding packed weights here costs what writing them out as images first would (about 10 % of the kernel), without 2 bytes per weight
 // of workspace. A wave issues its own vector instructions under its matrix instructions: 16 x 16 x 32 alone takes 18.1 clocks, with one
-// vector instruction behind each 20.1, two 20.6, three 25.1, four 29.1. Layer of 1111 f32 tokens (Llama-3-8B, Q4_0): 1280 -> 1116 us.
+// vector instruction behind each 20.1, two 20.6, three 25.1, four 29.1. Layer of 1111 f32 tokens (Llama-3-8B, Q4_0): 1280 -> 1074 - 1118 us.
 #include "common.h"
 
 namespace rlx {

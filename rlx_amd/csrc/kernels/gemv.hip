@@ -206,7 +206,7 @@ __device__ __forceinline__ void load_afrags(const half_t *xrow, bool live, int c
 // One K unit of one 16-row weight tile against RG groups of 16 activation rows: the fragments are decoded once and
 // every group runs its own matrix instructions on them. xrow[rg] / live[rg]: the lane's row of group rg in LDS and
 // whether that row exists; acc[rg]: the four output rows 4 g + r of group rg this lane holds. sxs: the Q4_K / Q5_K
-// block-sum table of the one-row kernels, [block][16].
+// block-sum table of the two-row kernels (NREG == 2: one f32 row or two 16-bit rows), [block][16].
 template <int SCHEME, int NREG, int RG>
 __device__ __forceinline__ void compute_unit(const UnitRegs<SCHEME> &w, const half_t *const (&xrow)[RG], const bool (&live)[RG],
                                              Frag (&a)[4], const float *sxs, int g, int ucol, int ublk, float (&acc)[RG][4],
@@ -700,7 +700,7 @@ __device__ __forceinline__ bool gemv_pass(const GemvArgs &a) {
 
     const int kc = kc_units * L.unit_k;
     const int row_stride = kc + XS_PAD_HALFS;
-    // LDS: [partial sums: tiles_per_wg x nwaves x (4 ng) x 16 f32][staged activations: rv rows][Q4_K / Q5_K block sums of the one-row kernels]
+    // LDS: [partial sums: tiles_per_wg x nwaves x (4 ng) x 16 f32][staged activations: rv rows][Q4_K / Q5_K block sums, NREG == 2]
     const int slot_floats = ng * 64;
     float *part = (float *)smem;
     // kw waves split the K units of one tile, tw = nwaves / kw tiles are walked side by side (kw = nwaves: every wave
