@@ -53,6 +53,8 @@ struct GemvArgs {
     int lds_bytes;
     int kw;
     int sc_off;
+    int tw, slices;
+    uint32_t kw_div, tw_div, slices_div, m_div;
 };
 struct RmsNorm {  // RMSNorm prologue of a decode launch (f32 activations only)
     const float *gamma, *beta;
@@ -192,6 +194,9 @@ static int64_t decode_rows(int xk) { return xk == 0 ? 16 : 32; }
 
 constexpr int ARGMAX_MAX_WGS = 4096;  // keys in the tied-LM-head scratch: one per workgroup of the decode launch
 
+// div_by() of kernels/gemv.hip
+static uint32_t div_magic(uint32_t d) { return d <= 1 ? 0u : (uint32_t)(((1ull << 32) + d - 1) / d); }
+
 static int launch_gemv(const void *const *xs, int xk, const rlx_qweight *const *ws, float *const *outs, int count, int m,
                        hipStream_t stream, const float *expert_idx = nullptr, unsigned long long *argmax_key = nullptr,
                        const rlx_qweight *const *pairs = nullptr, const RmsNorm *norm = nullptr, int *wgs_out = nullptr) {
@@ -297,9 +302,9 @@ static int launch_gemv(const void *const *xs, int xk, const rlx_qweight *const *
         }
         const size_t part_bytes = (size_t)max_tpw * kw * slot_bytes;
         sh.kcu = max_units;
-        // the last LDS_TAIL bytes: 1 / rms per activation row (RMSNorm prologue), the per-row factors of the binary16 range
-        // prescale and its bookkeeping (GEMV_LDS_TAIL in kernels/gemv.hip)
-        constexpr size_t LDS_TAIL = 448;
+        // the last LDS_TAIL bytes: the per-row factors of the binary16 range prescale and its bookkeeping, the sums of squares of
+        // the RMSNorm prologue (GEMV_LDS_TAIL in kernels/gemv.hip)
+        constexpr size_t LDS_TAIL = 384;
         while (sh.kcu > 1 && part_bytes + stage_bytes(sh.kcu) + LDS_TAIL > budget) sh.kcu--;
         sh.fits = part_bytes + stage_bytes(sh.kcu) + LDS_TAIL <= budget;
         sh.lds = part_bytes + stage_bytes(sh.kcu) + LDS_TAIL;
@@ -315,6 +320,12 @@ static int launch_gemv(const void *const *xs, int xk, const rlx_qweight *const *
         sh.a.eps = norm ? norm->eps : 0.f;
         sh.a.lds_bytes = (int)sh.lds;
         sh.a.kw = kw;
+        sh.a.tw = tw;
+        sh.a.slices = m >= sh.nwaves ? 1 : (sh.nwaves + m - 1) / m;
+        sh.a.kw_div = div_magic((uint32_t)kw);
+        sh.a.tw_div = div_magic((uint32_t)tw);
+        sh.a.slices_div = div_magic((uint32_t)sh.a.slices);
+        sh.a.m_div = div_magic((uint32_t)m);
         sh.a.slab_bytes = ws[0]->dims.bytes;
         sh.a.num_experts = ws[0]->experts;
         sh.a.sc_off = ws[0]->sc_off();

@@ -59,15 +59,23 @@ struct GemvArgs {
     int lds_bytes;     // dynamic LDS of the launch
     int kw;            // waves that split the K units of one tile; divides the waves of a workgroup
     int sc_off;        // Q6_K: a stored scale byte stands for byte - sc_off (0 unsigned reading, 128 signed)
+    int tw;            // tiles walked side by side: waves of a workgroup / kw
+    int slices;        // waves that share a row of activations while it is staged
+    uint32_t kw_div, tw_div, slices_div, m_div;  // div_by() of these
 };
+
+// x / d for x d < 2^32, `magic` = ceil(2^32 / d), or 0 for d = 1 (set by the host). The divisors of a launch are not known at compile
+// time, and the compiler's division is some forty dependent instructions: eight of them stood between a wave's start and its
+// first loads, 0.5 us of every launch.
+__device__ __forceinline__ uint32_t div_by(uint32_t x, uint32_t magic) { return magic ? __umulhi(x, magic) : x; }
 
 constexpr int XS_PAD_HALFS = 8;      // 16 bytes of padding per LDS row: rows land in different bank groups
 constexpr float LO_SCALE = 2048.0f;  // f32 activation x = hi + lo / LO_SCALE with hi, lo binary16
 
-// The last GEMV_LDS_TAIL bytes of a workgroup's LDS: [0,64) 1 / rms per activation row (RMSNorm prologue); then
-// GEMV_RANGE_AREA bytes: [0,128) un-scale factor per virtual activation row and [128,256) per logical row the bits of
-// max |x| of the staged chunk, then the forward scale (both only in the slow pass, below); [256,384) two row masks per
-// wave (up to 16 waves), written once by every wave at the end of the common pass.
+// The last GEMV_LDS_TAIL bytes of a workgroup's LDS: [0,128) un-scale factor per virtual activation row and [128,256) per logical
+// row the bits of max |x| of the staged chunk, then the forward scale (both only in the slow pass, below); [256,264) two row
+// masks, OR-ed together by the waves in the common pass; [272,384) sums of squares per (row, slice) (RMSNorm prologue: at most
+// eight rows, so 23 slices with sixteen waves).
 //
 // Activations travel as binary16. A row whose values leave the range binary16 carries well - some |x| >= 2^15, or no
 // |x| >= 2^-8 at all - is multiplied by a power of two that puts its largest value in [2^14, 2^15) while it is staged,
@@ -78,7 +86,7 @@ constexpr float LO_SCALE = 2048.0f;  // f32 activation x = hi + lo / LO_SCALE wi
 // nothing left in registers) and writes its outputs if there is no such row. Otherwise it writes nothing and the slow
 // pass does the same work again with the rescaling in its staging. The rescaling code sits in a part of the kernel the
 // common pass never enters; inside the common pass's staging it cost every launch registers, scalar spills and 0.5 us.
-constexpr int GEMV_RANGE_AREA = 384, GEMV_LDS_TAIL = 448;
+constexpr int GEMV_NORM_SUMS = 272, GEMV_LDS_TAIL = 384;
 constexpr float X_BIG = 32768.0f, X_SMALL = 0.00390625f;
 typedef _Float16 half4_t __attribute__((ext_vector_type(4)));
 
@@ -426,6 +434,48 @@ __device__ __forceinline__ void compute_unit(const UnitRegs<SCHEME> &w, const ha
     }
 }
 
+// RMSNorm prologue: out = (sum of x gamma w) / rms(x). The activations are staged as x gamma, their squares are summed on the way
+// (one sum per (row, slice) task, in `sums`), and the epilogue multiplies by the row's 1 / sqrt(mean + eps): x is read once and
+// nothing waits for the sum. (The slow pass, below, knows the sums and stages the normalized values.) With the normalization in the staging a second read of x and a barrier stood in front of the first
+// product: 2 us of a launch of one row of 4096 columns, and 4.5 us when one wave made the sum ahead of the first weights (the gate /
+// up launch of a Llama-3-8B layer 21.9 us then).
+// A beta (null in most models) has to be added to the normalized value: then the squares are summed first.
+__device__ __forceinline__ float wave_sum(float v) {  // the total, in lane 63
+    auto add = [&](auto ctrl, auto rows) {
+        v += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), decltype(ctrl)::value, decltype(rows)::value, 0xF, true));
+    };
+    add(std::integral_constant<int, 0x111>{}, std::integral_constant<int, 0xF>{});  // row_shr 1, 2, 4, 8
+    add(std::integral_constant<int, 0x112>{}, std::integral_constant<int, 0xF>{});
+    add(std::integral_constant<int, 0x114>{}, std::integral_constant<int, 0xF>{});
+    add(std::integral_constant<int, 0x118>{}, std::integral_constant<int, 0xF>{});
+    add(std::integral_constant<int, 0x142>{}, std::integral_constant<int, 0xA>{});  // row_bcast 15, 31
+    add(std::integral_constant<int, 0x143>{}, std::integral_constant<int, 0xC>{});
+    return v;
+}
+__device__ __forceinline__ void norm_square_sums(const GemvArgs &a, const GemvSeg &sg, float *sums) {
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), nwaves = (int)(blockDim.x >> 6);
+    const int groups = sg.k / 4, gps = ((int)div_by(groups + a.slices - 1, a.slices_div) + 63) & ~63;
+    for (int t = wave; t < a.m * a.slices; t += nwaves) {
+        const int row = (int)div_by(t, a.slices_div), g0 = (t - row * a.slices) * gps, g1 = min(groups, g0 + gps);
+        const float4_t *src = (const float4_t *)((const float *)sg.x + (long long)row * sg.k);
+        float sq = 0.f;
+        for (int cg = g0 + lane; cg < g1; cg += 64) {
+            const float4_t v = src[cg];
+            sq += v[0] * v[0] + v[1] * v[1] + v[2] * v[2] + v[3] * v[3];
+        }
+        sq = wave_sum(sq);
+        if (lane == 63) sums[t] = sq;
+    }
+    __syncthreads();
+}
+__device__ __forceinline__ float norm_scale(const GemvArgs &a, int k, const float *sums, int row) {
+    float sq = 0.f;
+#pragma unroll 8
+    for (int i = 0; i < a.slices; i++) sq += sums[row * a.slices + i];
+    return 1.0f / sqrtf(sq * (1.0f / (float)k) + a.eps);
+}
+
 // Convert one K chunk of the activations into LDS as halfs: f32 -> hi rows [0,m) + lo rows [m,2m); 16-bit -> rows [0,m).
 // The work is cut into (row, slice of the row's 16-byte groups) tasks, one wave per task: with fewer rows than waves a row
 // is shared by several waves, otherwise a wave takes whole rows in turn. A wave therefore works on one row at a time -
@@ -444,9 +494,9 @@ __device__ __forceinline__ float max3_abs(float acc, float x, float y) {  // max
 }
 template <int XD, bool NORM = false, int PASS = 0>
 __device__ __forceinline__ void stage_x_typed(const GemvArgs &a, const GemvSeg &sg, half_t *xs, int row_stride, int k0, int kc,
-                                              const float *inv_rms = nullptr, uint32_t *masks = nullptr, uint32_t *rowmax = nullptr,
+                                              float *norm_sums = nullptr, uint32_t *masks = nullptr, uint32_t *rowmax = nullptr,
                                               const float *fwd = nullptr) {
-    constexpr int U = 8;
+    constexpr int U = NORM ? 4 : 8;  // (with a norm, gamma is loaded beside them)
     constexpr int G = XD == X_F32 ? 4 : 8;  // columns per 16-byte load
     constexpr int ESZ = XD == X_F32 ? 4 : 2;
     typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
@@ -454,21 +504,24 @@ __device__ __forceinline__ void stage_x_typed(const GemvArgs &a, const GemvSeg &
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), nwaves = (int)(blockDim.x >> 6);
     const int groups = kc / G;  // kc is a multiple of 64
-    const int slices = a.m >= nwaves ? 1 : (nwaves + a.m - 1) / a.m;  // waves that share a row
-    const int gps = ((groups + slices - 1) / slices + 63) & ~63;      // groups per slice: whole wave-loads
+    const int slices = a.slices;
+    const int gps = ((int)div_by(groups + slices - 1, a.slices_div) + 63) & ~63;  // groups per slice: whole wave-loads
     const int tasks = a.m * slices;
     const int lo_rows = a.m * row_stride;  // halfs from a hi row to its lo row
     for (int t = wave; t < tasks; t += nwaves) {
-        const int row = t / slices, slice = t - row * slices;
+        const int row = (int)div_by(t, a.slices_div), slice = t - row * slices;
         const int g0 = slice * gps, g1 = min(groups, g0 + gps);
         const uint8_t *src = (const uint8_t *)sg.x + ((long long)row * sg.k + k0) * ESZ;
         half_t *dst = xs + row * row_stride;
         float vmax = 0.f;  // the largest |x| this lane has seen in the row
         float rowscale = 1.f, scale = 1.f;
+        float sq = 0.f;
         if constexpr (PASS == 2) rowscale = fwd[row];
-        if constexpr (NORM) scale = inv_rms[row];
+        if constexpr (NORM)
+            if (PASS != 0 || a.beta) scale = norm_scale(a, sg.k, norm_sums, row);
         for (int cg0 = g0 + lane; cg0 < g1; cg0 += 64 * U) {
             raw_t raw[U];
+            float4_t gm[NORM ? U : 1];  // fetched with the activations, not behind them
 #pragma unroll
             for (int u = 0; u < U; u++) {
                 const int c = (cg0 + 64 * u) * G;
@@ -476,6 +529,10 @@ __device__ __forceinline__ void stage_x_typed(const GemvArgs &a, const GemvSeg &
                 // k is a multiple of 32: a group is inside or outside as a whole
                 if (cg0 + 64 * u < g1 && k0 + c < sg.k) v = *(const raw_t *)(src + (long long)c * ESZ);
                 raw[u] = v;
+                if constexpr (NORM) {
+                    gm[u] = float4_t{1.f, 1.f, 1.f, 1.f};
+                    if (cg0 + 64 * u < g1 && k0 + c < sg.k) gm[u] = *(const float4_t *)(a.gamma + k0 + c);
+                }
             }
 #pragma unroll
             for (int u = 0; u < U; u++) {
@@ -483,12 +540,9 @@ __device__ __forceinline__ void stage_x_typed(const GemvArgs &a, const GemvSeg &
                 if (cg0 + 64 * u >= g1) continue;
                 if constexpr (XD == X_F32) {
                     half4_t hi, lo;
-                    float4_t gm = {1.f, 1.f, 1.f, 1.f}, bt = {0.f, 0.f, 0.f, 0.f};
+                    float4_t bt = {0.f, 0.f, 0.f, 0.f};
                     if constexpr (NORM) {
-                        if (k0 + c < sg.k) {
-                            gm = *(const float4_t *)(a.gamma + k0 + c);
-                            if (a.beta) bt = *(const float4_t *)(a.beta + k0 + c);
-                        }
+                        if (a.beta && k0 + c < sg.k) bt = *(const float4_t *)(a.beta + k0 + c);
                     }
 #pragma unroll
                     for (int e = 0; e < 4; e += 2) {
@@ -496,7 +550,10 @@ __device__ __forceinline__ void stage_x_typed(const GemvArgs &a, const GemvSeg &
 #pragma unroll
                         for (int i = 0; i < 2; i++) {
                             v[i] = raw[u][e + i];
-                            if constexpr (NORM) v[i] = v[i] * scale * gm[e + i] + bt[e + i];  // in_row[i] * inv_rms * gamma[i] + beta[i], unfused
+                            if constexpr (NORM) {
+                                if constexpr (PASS == 0) sq += v[i] * v[i];
+                                v[i] = v[i] * scale * gm[u][e + i] + bt[e + i];  // scale 1: x gamma
+                            }
                         }
                         if constexpr (PASS != 2) vmax = max3_abs(vmax, v[0], v[1]);
                         half2_t h, l;
@@ -543,6 +600,10 @@ __device__ __forceinline__ void stage_x_typed(const GemvArgs &a, const GemvSeg &
                 }
             }
         }
+        if constexpr (NORM && PASS == 0) {
+            sq = wave_sum(sq);
+            if (lane == 63 && !a.beta) norm_sums[t] = k0 == 0 ? sq : norm_sums[t] + sq;  // the same wave takes task t of every chunk
+        }
         if constexpr (XD != X_F16) {
             if constexpr (PASS == 0) {  // into the wave's two masks: one vote each per task
                 masks[0] |= (__ballot(vmax >= X_BIG) != 0 ? 1u : 0u) << row;
@@ -561,13 +622,12 @@ __device__ __forceinline__ void stage_x_typed(const GemvArgs &a, const GemvSeg &
 template <bool NORM>
 __device__ __forceinline__ void stage_chunk(const GemvArgs &a, const GemvSeg &sg, half_t *xs, int row_stride, int k0, int kc, uint8_t *tail,
                                             uint32_t *wm) {
-    const float *inv_rms = (const float *)tail;
     if constexpr (NORM) {
-        stage_x_typed<X_F32, true, 0>(a, sg, xs, row_stride, k0, kc, inv_rms, wm);
+        stage_x_typed<X_F32, true, 0>(a, sg, xs, row_stride, k0, kc, (float *)(tail + GEMV_NORM_SUMS), wm);
     } else {
-        if (a.x_dtype == X_F32) stage_x_typed<X_F32, false, 0>(a, sg, xs, row_stride, k0, kc, inv_rms, wm);
-        else if (a.x_dtype == X_BF16) stage_x_typed<X_BF16, false, 0>(a, sg, xs, row_stride, k0, kc, inv_rms, wm);
-        else stage_x_typed<X_F16, false, 0>(a, sg, xs, row_stride, k0, kc, inv_rms, wm);
+        if (a.x_dtype == X_F32) stage_x_typed<X_F32, false, 0>(a, sg, xs, row_stride, k0, kc, nullptr, wm);
+        else if (a.x_dtype == X_BF16) stage_x_typed<X_BF16, false, 0>(a, sg, xs, row_stride, k0, kc, nullptr, wm);
+        else stage_x_typed<X_F16, false, 0>(a, sg, xs, row_stride, k0, kc, nullptr, wm);
     }
     __syncthreads();
 }
@@ -577,16 +637,16 @@ __device__ __forceinline__ void stage_chunk(const GemvArgs &a, const GemvSeg &sg
 template <int XD, bool NORM>
 __device__ __forceinline__ void stage_chunk_rescaled(const GemvArgs &a, const GemvSeg &sg, half_t *xs, int row_stride, int k0, int kc,
                                                      uint8_t *tail) {
-    const float *inv_rms = (const float *)tail;
-    float *rsv = (float *)(tail + 64);
-    uint32_t *rowmax = (uint32_t *)(tail + 64 + 128);
+    float *norm_sums = (float *)(tail + GEMV_NORM_SUMS);
+    float *rsv = (float *)tail;
+    uint32_t *rowmax = (uint32_t *)(tail + 128);
     const int tid = threadIdx.x;
     if (tid < 32) {
         rowmax[tid] = 0;
         rsv[tid] = 1.f;
     }
     __syncthreads();
-    stage_x_typed<XD, NORM, 1>(a, sg, xs, row_stride, k0, kc, inv_rms, nullptr, rowmax);
+    stage_x_typed<XD, NORM, 1>(a, sg, xs, row_stride, k0, kc, norm_sums, nullptr, rowmax);
     __syncthreads();
     if (tid < a.m) {
         const uint32_t mb = rowmax[tid];
@@ -603,7 +663,7 @@ __device__ __forceinline__ void stage_chunk_rescaled(const GemvArgs &a, const Ge
         ((float *)rowmax)[tid] = fwd;
     }
     __syncthreads();
-    stage_x_typed<XD, NORM, 2>(a, sg, xs, row_stride, k0, kc, inv_rms, nullptr, nullptr, (const float *)rowmax);
+    stage_x_typed<XD, NORM, 2>(a, sg, xs, row_stride, k0, kc, norm_sums, nullptr, nullptr, (const float *)rowmax);
     __syncthreads();
 }
 
@@ -681,6 +741,9 @@ __device__ __forceinline__ bool gemv_pass(const GemvArgs &a) {
     const int ng = (rv + 3) >> 2;                         // groups of four output rows that exist (16 RG at most)
     const half2_t sc_bias = ubyte_bias(a.sc_off);
 
+    // All scalar arguments in one round of loads: fetched where each is first used they were eight rounds, one behind the other.
+    asm volatile("" ::"s"(a.nseg), "s"(a.m), "s"(a.kc_units), "s"(a.x_dtype), "s"(a.max_tiles_per_wg), "s"(a.expert_idx), "s"(a.lds_bytes), "s"(a.kw), "s"(a.tw),
+                 "s"(a.slices), "s"(a.kw_div), "s"(a.tw_div), "s"(a.slices_div), "s"(a.m_div));
     int s = 0;
 #pragma unroll
     for (int i = 1; i < GEMV_MAX_SEG; i++)
@@ -705,8 +768,8 @@ __device__ __forceinline__ bool gemv_pass(const GemvArgs &a) {
     float *part = (float *)smem;
     // kw waves split the K units of one tile, tw = nwaves / kw tiles are walked side by side (kw = nwaves: every wave
     // on the same tile, the decode shape; a small kw keeps the partial-sum area small when the slots are large).
-    const int kw = a.kw, tw = nwaves / kw;
-    const int kl = __builtin_amdgcn_readfirstlane(wave % kw), tl = __builtin_amdgcn_readfirstlane(wave / kw);
+    const int kw = a.kw, tw = a.tw;
+    const int tl = __builtin_amdgcn_readfirstlane((int)div_by(wave, a.kw_div)), kl = wave - tl * kw;
     const size_t part_bytes = (size_t)a.max_tiles_per_wg * kw * slot_floats * 4;
     half_t *xs = (half_t *)(smem + part_bytes);
     float *sxs = (float *)(smem + part_bytes + (((size_t)rv * row_stride * 2 + 15) & ~(size_t)15));  // [blk][16]
@@ -721,25 +784,7 @@ __device__ __forceinline__ bool gemv_pass(const GemvArgs &a) {
         live[rg] = RG > 1 || nrow < rv;
     }
 
-    for (int i = tid; i < ((MODE & GEMV_PAIRED) ? 2 : 1) * ntiles * kw * slot_floats; i += blockDim.x) part[i] = 0.f;
-    // RMSNorm prologue: one wave per activation row sums the squares of the whole row (the sum is needed before any
-    // element can be scaled), 1 / sqrt(mean + eps) lands in the last 64 bytes of the workgroup's LDS.
     uint8_t *tail = smem + a.lds_bytes - GEMV_LDS_TAIL;
-    float *inv_rms = (float *)tail;
-    if constexpr ((MODE & GEMV_NORM) != 0) {
-        for (int row = wave; row < a.m; row += nwaves) {
-            const float *xr = (const float *)seg.x + (long long)row * seg.k;
-            float sq = 0.f;
-            for (int c = l * 4; c < seg.k; c += 256) {
-                const float4_t v = *(const float4_t *)(xr + c);
-                sq += v[0] * v[0] + v[1] * v[1] + v[2] * v[2] + v[3] * v[3];
-            }
-#pragma unroll
-            for (int off = 32; off > 0; off >>= 1) sq += __shfl_xor(sq, off);
-            if (l == 0) inv_rms[row] = 1.0f / sqrtf(sq * (1.0f / (float)seg.k) + a.eps);
-        }
-        __syncthreads();
-    }
 
     // With a paired matrix every tile is walked twice, first in `w`, then in `w_pair`: virtual tile vt = 2 t + which.
     constexpr bool paired = (MODE & GEMV_PAIRED) != 0;
@@ -749,22 +794,18 @@ __device__ __forceinline__ bool gemv_pass(const GemvArgs &a) {
     const uint8_t *wbase2 = paired ? seg.w_pair + (long long)tile0 * seg.units * L.unit_bytes : wbase;
     auto vtile_ptr = [&](int vt) { return paired ? ((vt & 1) ? wbase2 : wbase) + (vt >> 1) * tile_bytes : wbase + vt * tile_bytes; };
 
-    const float *rsv = (const float *)(tail + 64);
+    const float *rsv = (const float *)tail;
     uint32_t wm[2] = {0, a.x_dtype == X_F16 ? 0xFFFFFFFFu : 0u};  // this wave's notes: rows with a big value, rows with a value that is not tiny
-    uint32_t *notes = (uint32_t *)(tail + 64 + 256);               // the workgroup's: the waves' notes OR-ed together
-    if constexpr (!SLOW) {
-        if (tid == 0) notes[0] = notes[1] = 0;
-    }
+    uint32_t *notes = (uint32_t *)(tail + 256);               // the workgroup's: the waves' notes OR-ed together
     for (int u0 = 0; u0 < seg.units; u0 += kc_units) {
         const int nu = min(kc_units, seg.units - u0);  // units in this chunk
         if (u0 > 0) __syncthreads();  // every wave is done with the previous chunk: its activations, its factors
-        if constexpr (SLOW) stage_chunk_slow<(MODE & GEMV_NORM) != 0>(a, seg, xs, row_stride, u0 * L.unit_k, nu * L.unit_k, tail);
         // This wave's items: for each tile, units wave, wave + nwaves, ... < nu. Two cursors walk them: `pf_*` issues
         // loads DEPTH items ahead into a register ring, `cu_*` consumes.
         // An item is UPI consecutive units (the host picks UPI > 1 only when every chunk holds a multiple of UPI).
         const int nug = nu / UPI;
-        const int my_units = kl < nug ? (nug - kl + kw - 1) / kw : 0;
-        const int my_tiles = tl < nvt ? (nvt - tl + tw - 1) / tw : 0;
+        const int my_units = kl < nug ? (int)div_by(nug - kl + kw - 1, a.kw_div) : 0;
+        const int my_tiles = tl < nvt ? (int)div_by(nvt - tl + tw - 1, a.tw_div) : 0;
         const int nitems = my_tiles * my_units;
         int pf_t = tl, pf_u = kl, pf_n = 0;
         const uint8_t *pf_ptr = vtile_ptr(tl) + (long long)(u0 + kl * UPI) * L.unit_bytes;
@@ -793,6 +834,17 @@ __device__ __forceinline__ bool gemv_pass(const GemvArgs &a) {
             for (int p = 0; p < UPI; p++) ring[d].u[p].clear();
             prefetch(ring[d]);
         }
+        // The first weights are on their way: now clear the partial sums (every slot: a wave may have no unit of a tile) and the notes.
+        // (The barrier behind the staging orders this before the first use.)
+        if (u0 == 0) {
+            for (int i = tid * 4; i < nvt * kw * slot_floats; i += blockDim.x * 4) *(float4_t *)(part + i) = float4_t{0.f, 0.f, 0.f, 0.f};
+            if constexpr (!SLOW) {
+                if (tid == 0) notes[0] = notes[1] = 0;
+                if constexpr ((MODE & GEMV_NORM) != 0)
+                    if (a.beta) norm_square_sums(a, seg, (float *)(tail + GEMV_NORM_SUMS));
+            }
+        }
+        if constexpr (SLOW) stage_chunk_slow<(MODE & GEMV_NORM) != 0>(a, seg, xs, row_stride, u0 * L.unit_k, nu * L.unit_k, tail);
         if constexpr (!SLOW) {
             stage_chunk<(MODE & GEMV_NORM) != 0>(a, seg, xs, row_stride, u0 * L.unit_k, nu * L.unit_k, tail, wm);
             if (l == 0) {  // behind the barrier that also ordered the clearing of the notes; nothing waits for these
@@ -867,16 +919,28 @@ __device__ __forceinline__ bool gemv_pass(const GemvArgs &a) {
     }
     // out[mr][tile*16 + col] = sum over waves of row mr (+ 2^-11 * row m+mr for f32 activations)
     unsigned long long best = 0;  // below every key a real value produces
+    // (The slots are read eight at a time: one by one behind each other's additions they were 1.3 us of a launch, 3.7 with a pair.)
     for (int idx = tid; idx < ntiles * a.m * 16; idx += blockDim.x) {
-        const int col = idx & 15, mr = (idx >> 4) % a.m, t = idx / (16 * a.m);
+        const int col = idx & 15, t = (int)div_by(idx >> 4, a.m_div), mr = (idx >> 4) - t * a.m;
+        float scale = 1.f;
+        if constexpr ((MODE & GEMV_NORM) != 0 && !SLOW)
+            if (!a.beta) scale = norm_scale(a, seg.k, (const float *)(tail + GEMV_NORM_SUMS), mr);
         auto tile_sum = [&](int vt) {
-            float sum = 0.f;
-            for (int wv = 0; wv < kw; wv++) {
-                const float *slot = part + ((size_t)vt * kw + wv) * slot_floats + col;
-                sum += slot[mr * 16];
-                if (a.x_dtype == X_F32) sum += slot[(a.m + mr) * 16] * (1.0f / LO_SCALE);
+            const float *slot = part + (size_t)vt * kw * slot_floats + mr * 16 + col;
+            // (f64 with a norm: the factor at the end is then the only rounding, where a product's own used to be the last)
+            typename std::conditional<(MODE & GEMV_NORM) != 0, double, float>::type sum = 0;
+            if (a.x_dtype == X_F32) {
+#pragma unroll 8
+                for (int wv = 0; wv < kw; wv++) {
+                    sum += slot[wv * slot_floats];
+                    sum += slot[wv * slot_floats + a.m * 16] * (1.0f / LO_SCALE);
+                }
+            } else {
+#pragma unroll 8
+                for (int wv = 0; wv < kw; wv++) sum += slot[wv * slot_floats];
             }
-            return sum;
+            if constexpr ((MODE & GEMV_NORM) != 0 && !SLOW) sum = sum * scale;
+            return (float)sum;
         };
         float sum;
         if (paired) {
@@ -915,6 +979,14 @@ __device__ __forceinline__ bool gemv_pass(const GemvArgs &a) {
     return false;
 }
 
+// The kernel's arguments (its only ones) through a pointer the compiler knows nothing about: the slow pass loads them again instead
+// of keeping those of the common pass in registers (some forty scalars spilled into lanes of vector registers).
+__device__ __forceinline__ const GemvArgs &args_again() {
+    auto p = __builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(p));
+    return *(const GemvArgs *)p;
+}
+
 }  // namespace rlx
 
 #define RLX_GEMV_INST(name, SCHEME, NREG, DEPTH, MODE, UPI) RLX_GEMV_INST_RG(name, SCHEME, NREG, DEPTH, MODE, UPI, 1, 1024)
@@ -922,7 +994,7 @@ __device__ __forceinline__ bool gemv_pass(const GemvArgs &a) {
     extern "C" __global__ __launch_bounds__(THREADS) void name(rlx::GemvArgs a) {                            \
         if (rlx::gemv_pass<SCHEME, NREG, DEPTH, MODE, UPI, RG, false>(a)) {                                  \
             __syncthreads();                                                                                  \
-            rlx::gemv_pass<SCHEME, NREG, DEPTH, MODE, UPI, RG, true>(a);                                      \
+            rlx::gemv_pass<SCHEME, NREG, DEPTH, MODE, UPI, RG, true>(rlx::args_again());                      \
         }                                                                                                     \
     }
 // NREG = 2: at most two virtual rows (m = 1 f32, or m <= 2 16-bit); NREG = 4 otherwise.

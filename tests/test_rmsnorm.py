@@ -62,6 +62,29 @@ def test_rmsnorm_prologue_matches_norm_then_matmul(scheme, m, k, ns, with_beta):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("scheme,m,k,n", [(Q4_0, 1, 128, 33), (Q8_0, 5, 2080, 48), (Q4K, 7, 1024, 272), (Q4_0, 3, 4096, 4112), (Q8_0, 8, 14336, 16)])
+@pytest.mark.parametrize("size", [1e-6, 1.0, 1e6, 1e21])
+def test_rmsnorm_scale_is_applied_to_the_sums(scheme, m, k, n, size):
+    """x gamma is staged and the sums are scaled, unless x gamma is outside the range of binary16 (the first and the last two sizes:
+    normalized values are staged then); squares that overflow make a factor of 0, as in the reference's own f32 arithmetic."""
+    rng = np.random.default_rng(5)
+    x = (rng.standard_normal((m, k)) * size).astype(np.float32)
+    gamma = (1.0 + 0.1 * rng.standard_normal(k)).astype(np.float32)
+    p = weights(scheme, n, k, 20)
+    w = ops.QWeight(QuantScheme(scheme), p, n, k)
+    got = ops.rmsnorm_gguf_matmul_bt_batch(x, gamma, None, 1e-12, [w], m)[0]
+    if size > 1e20:
+        assert not oracle.rms_norm(x, gamma, None, 1e-12).any() and not got.any()
+    else:
+        x64 = x.astype(np.float64)
+        xn = x64 / np.sqrt((x64 ** 2).mean(axis=1, keepdims=True) + 1e-12) * gamma
+        ref = xn @ oracle.dequant(scheme, p, n * k).reshape(n, k).astype(np.float64).T
+        # at most 448 f32 additions of block sums, a random walk of half an ulp of the row's largest values: 2^-24 sqrt(448)
+        assert np.max(np.abs(got - ref)) <= 1.3e-6 * np.max(np.abs(ref))
+    w.free()
+
+
+@pytest.mark.gpu
 def test_rmsnorm_swiglu_and_argmax():
     rng = np.random.default_rng(3)
     m, k, n = 1, 2048, 700
