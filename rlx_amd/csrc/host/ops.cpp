@@ -1275,13 +1275,13 @@ struct TopkArgs {  // mirrors kernels/topk.hip
 };
 constexpr int64_t TOPK_GROUP = 1024;   // candidates one wave of rlx_topk_serial / rlx_topk_select reduces to `cap`
 constexpr int64_t TOPK_FINISH = 8192;  // candidates rlx_topk_finish takes
-// Winners one by one or by threshold, in us of the whole call on Q8_0 rows of 1024 columns. Reducing 1024s: 9000 rows at cap 1 20.8
-// one by one, 24.0 by threshold; at cap 10 24.2 against 25.1; at cap 12 25 against 24.
-constexpr int TOPK_SERIAL_CAP = 11;
-// The end, one by one in a single wave or by threshold in a workgroup of sixteen, which up to 128 candidates has nothing to cut: 40 rows
-// at cap 4 9.0 against 9.9, at cap 8 10.0 against 9.9; 300 rows at cap 1 9.3 against 13.4, at cap 17 13.3 against 13.4; 1000 rows at
-// cap 1 11.5 against 14.8, at cap 11 14.0 against 14.8, at cap 12 14.9 against 14.8.
-static bool topk_serial_end(int64_t count, int cap) { return cap <= (count <= 128 ? 7 : count <= 512 ? 17 : count <= TOPK_GROUP ? 11 : 0); }
+// Winners one by one or by threshold, in us of the whole call on Q8_0 rows of 1024 columns. Reducing 1024s: 128256 rows at cap 1 29.7
+// one by one, 30.0 by threshold; 9000 rows at cap 8 18.3 either way, at cap 11 19.0 against 18.7.
+constexpr int TOPK_SERIAL_CAP = 8;
+// The end, one by one in a single wave or by threshold in a workgroup of sixteen, which up to 128 candidates has nothing to cut: 128 rows
+// at cap 1 7.9 against 9.7, at cap 8 9.7 either way; 300 rows at cap 1 7.9 against 9.7, at cap 20 12.8 against 13.1, at cap 24 14.0
+// against 13.1; 1000 rows at cap 1 8.0 against 9.9, at cap 4 8.8 against 14.3, at cap 24 14.1 against 14.4.
+static bool topk_serial_end(int64_t count, int cap) { return cap <= (count <= 128 ? 8 : count <= 512 ? 20 : count <= TOPK_GROUP ? 24 : 0); }
 constexpr int TOPK_MAX_CAP = 64;
 static int64_t topk_groups(int64_t n) { return (n + TOPK_GROUP - 1) / TOPK_GROUP; }
 }  // namespace rlx

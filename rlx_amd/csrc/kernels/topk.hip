@@ -9,11 +9,10 @@
 //   rlx_topk_serial  one wave per 1024 candidates, sixteen per lane, sorted once per lane; cap rounds of a wave-wide maximum of the
 //                    lanes' heads, the lane that held the winner moves its list up. Writes its cap winners as keys or, as
 //                    the only wave, the answer. No LDS, no barrier.
-//   rlx_topk_select  one wave per 1024 candidates, sixteen per lane, leaves their `cap` best in any order. No LDS, no barrier.
+//   rlx_topk_select  one wave per 1024 candidates, sixteen per lane, leaves their `cap` best in any order.
 //   rlx_topk_finish  one workgroup, up to 8192 candidates, eight per thread: writes rows and values, largest first.
 // All are bound by latency (launch, one load, the chain of rounds or counts), not by bandwidth: 128256 logits are 0.5 MB. The whole
-// LM-head call at [128256, 4096] Q4_K, cap 40: 93.3 us with the serial kernel alone, 69 - 72 with the other two, about 54 of it the
-// matmul. Where the lines between them lie: host/ops.cpp.
+// LM-head call at [128256, 4096] Q4_K, cap 40: 63 us, about 53 of it the matmul. Where the lines between them lie: host/ops.cpp.
 #include "common.h"
 
 namespace rlx {
@@ -21,6 +20,7 @@ namespace rlx {
 constexpr int TOPK_PER_LANE = 16, TOPK_GROUP = 64 * TOPK_PER_LANE;       // candidates per wave of rlx_topk_serial / rlx_topk_select
 constexpr int TOPK_PER_THREAD = 8, TOPK_FINISH = 1024 * TOPK_PER_THREAD;  // candidates rlx_topk_finish takes
 constexpr int TOPK_SURVIVORS = 128;                                       // keys it puts in order (cap <= 64)
+constexpr int TOPK_FEW = 256;                                             // keys rlx_topk_select counts four per lane
 
 __device__ __forceinline__ unsigned long long topk_key_of(float v, uint32_t row) {
     const uint32_t b = __builtin_bit_cast(uint32_t, v + 0.0f);  // -0 and +0 compare equal
@@ -57,11 +57,27 @@ struct TopkArgs {
     float *out_val;
 };
 
-__device__ __forceinline__ unsigned long long topk_load(const TopkArgs &a, long long i) {
-    if (i >= a.n) return 0;
-    if (!a.vals) return a.keys_in[i];
-    const float v = a.vals[i];
-    return v == v ? topk_key_of(v, (uint32_t)i) : 0;
+// N candidates per lane, `stride` apart from `first` on. All loads are issued before the first one is used: behind a branch each they
+// were N latencies one after the other, and logits that other XCDs have just written are 0.5 us away (6 of the 12 us of a
+// rlx_topk_select).
+template <int N>
+__device__ __forceinline__ void topk_load(const TopkArgs &a, long long first, int stride, unsigned long long (&key)[N]) {
+    const long long last = a.n - 1;
+    if (a.vals) {
+        float v[N];
+#pragma unroll
+        for (int e = 0; e < N; e++) v[e] = a.vals[min(first + (long long)e * stride, last)];
+#pragma unroll
+        for (int e = 0; e < N; e++) {
+            const long long i = first + (long long)e * stride;
+            key[e] = i <= last && v[e] == v[e] ? topk_key_of(v[e], (uint32_t)i) : 0;
+        }
+    } else {
+#pragma unroll
+        for (int e = 0; e < N; e++) key[e] = a.keys_in[min(first + (long long)e * stride, last)];
+#pragma unroll
+        for (int e = 0; e < N; e++) key[e] = first + (long long)e * stride <= last ? key[e] : 0;
+    }
 }
 
 }  // namespace rlx
@@ -71,8 +87,7 @@ extern "C" __global__ __launch_bounds__(64) void rlx_topk_serial(rlx::TopkArgs a
     const int lane = threadIdx.x;
     const long long base = (long long)blockIdx.x * TOPK_GROUP;
     unsigned long long mine[TOPK_PER_LANE];
-#pragma unroll
-    for (int e = 0; e < TOPK_PER_LANE; e++) mine[e] = topk_load(a, base + lane + e * 64);
+    topk_load(a, base + lane, 64, mine);
     // this lane's candidates in descending order (bitonic network over registers: every index is a constant)
 #pragma unroll
     for (int k = 2; k <= TOPK_PER_LANE; k <<= 1)
@@ -112,41 +127,82 @@ extern "C" __global__ __launch_bounds__(64) void rlx_topk_serial(rlx::TopkArgs a
     }
 }
 
+// The bound comes first: the cap-th largest of the 64 lanes' own maxima, one ballot a step. At least cap keys reach it, and few more do
+// (about 62 of 1024 at cap 40 where the values lie in no particular order), so the search for the cap-th largest key counts four keys
+// per lane instead of sixteen: the whole LM-head call at [128256, 4096] Q4_K, cap 40, 67.1 -> 63.2 us with loads
+// that do not wait for each other. Where more survive (long runs of
+// values in descending order) it counts all sixteen.
 extern "C" __global__ __launch_bounds__(64) void rlx_topk_select(rlx::TopkArgs a) {
     using namespace rlx;
+    __shared__ unsigned long long few[TOPK_FEW];
     const int lane = threadIdx.x;
     const long long base = (long long)blockIdx.x * TOPK_GROUP;
     unsigned long long mine[TOPK_PER_LANE];
-#pragma unroll
-    for (int e = 0; e < TOPK_PER_LANE; e++) mine[e] = topk_load(a, base + lane + e * 64);
+    topk_load(a, base + lane, 64, mine);
     uint32_t best = 0;
 #pragma unroll
     for (int e = 0; e < TOPK_PER_LANE; e++) best = max(best, (uint32_t)(mine[e] >> 32));
-    // The lanes' own maxima bound the threshold: at least 64 >= cap keys reach the smallest of them, none passes the
-    // largest, so the bits the two share are decided.
     const uint32_t top = wave_max_u32(best), low = wave_min_u32(best);
-    unsigned long long t = 0;  // the largest value with at least cap keys >= t (0: fewer than cap candidates, take them all)
-    const int bits = top == low ? 32 : 64 - __builtin_clz(top ^ low);  // undecided low bits of t
-    if (bits < 64) t = (unsigned long long)top << 32 >> bits << bits;
-    for (int bit = bits - 1; bit >= 0; bit--) {
-        const unsigned long long trial = t | (1ull << bit);
-        int count = 0;
-#pragma unroll
-        for (int e = 0; e < TOPK_PER_LANE; e++) count += __builtin_popcountll(__ballot(mine[e] >= trial));
-        if (count >= a.cap) t = trial;
-        if (count == a.cap) break;
+    uint32_t bound = low;  // all 64 >= cap maxima reach it
+    if (top != low) {
+        const int open = 32 - __builtin_clz(top ^ low);  // undecided low bits
+        bound = open < 32 ? top >> open << open : 0u;
+        for (int bit = open - 1; bit >= 0; bit--) {
+            const uint32_t trial = bound | (1u << bit);
+            if (__builtin_popcountll(__ballot(best >= trial)) >= a.cap) bound = trial;
+        }
     }
-    if (t == 0) t = 1;  // an absent candidate is key 0
-    int at = 0;
+    if (bound == 0) bound = 1;  // fewer than cap lanes have a candidate, an absent one is key 0
+    unsigned long long t = (unsigned long long)bound << 32;  // keys >= t are taken in the end
+    int count = 0;
 #pragma unroll
-    for (int e = 0; e < TOPK_PER_LANE; e++) {
-        const bool take = mine[e] >= t;
-        const unsigned long long who = __ballot(take);
-        const int pos = at + __builtin_popcountll(who & ((1ull << lane) - 1ull));
-        if (take) a.keys_out[(long long)blockIdx.x * a.cap + pos] = mine[e];
-        at += __builtin_popcountll(who);
+    for (int e = 0; e < TOPK_PER_LANE; e++) count += __builtin_popcountll(__ballot(mine[e] >= t));
+    auto write = [&](auto &keys) {
+        int at = 0;
+#pragma unroll
+        for (unsigned e = 0; e < sizeof(keys) / 8; e++) {
+            const bool take = keys[e] >= t;
+            const unsigned long long who = __ballot(take);
+            const int pos = at + __builtin_popcountll(who & ((1ull << lane) - 1ull));
+            if (take) a.keys_out[(long long)blockIdx.x * a.cap + pos] = keys[e];
+            at += __builtin_popcountll(who);
+        }
+        if (at + lane < a.cap) a.keys_out[(long long)blockIdx.x * a.cap + at + lane] = 0;
+    };
+    // t: the largest value with at least cap keys >= t, a bit a step
+    auto search = [&](auto &keys) {
+        const int bits = top == bound ? 32 : 64 - __builtin_clz(top ^ bound);  // undecided low bits of t
+        t = bits < 64 ? (unsigned long long)top << 32 >> bits << bits : 0;
+        for (int bit = bits - 1; bit >= 0; bit--) {
+            const unsigned long long trial = t | (1ull << bit);
+            int c = 0;
+#pragma unroll
+            for (unsigned e = 0; e < sizeof(keys) / 8; e++) c += __builtin_popcountll(__ballot(keys[e] >= trial));
+            if (c >= a.cap) t = trial;
+            if (c == a.cap) break;
+        }
+    };
+    if (count <= a.cap) {
+        write(mine);
+    } else if (count <= TOPK_FEW) {
+        int at = 0;
+#pragma unroll
+        for (int e = 0; e < TOPK_PER_LANE; e++) {
+            const bool take = mine[e] >= t;
+            const unsigned long long who = __ballot(take);
+            if (take) few[at + __builtin_popcountll(who & ((1ull << lane) - 1ull))] = mine[e];
+            at += __builtin_popcountll(who);
+        }
+        __syncthreads();
+        unsigned long long kept[TOPK_FEW / 64];
+#pragma unroll
+        for (int e = 0; e < TOPK_FEW / 64; e++) kept[e] = lane + 64 * e < count ? few[lane + 64 * e] : 0;
+        search(kept);
+        write(kept);
+    } else {
+        search(mine);
+        write(mine);
     }
-    if (at + lane < a.cap) a.keys_out[(long long)blockIdx.x * a.cap + at + lane] = 0;
 }
 
 extern "C" __global__ __launch_bounds__(1024) void rlx_topk_finish(rlx::TopkArgs a) {
@@ -157,8 +213,7 @@ extern "C" __global__ __launch_bounds__(1024) void rlx_topk_finish(rlx::TopkArgs
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     unsigned long long mine[TOPK_PER_THREAD];
-#pragma unroll
-    for (int e = 0; e < TOPK_PER_THREAD; e++) mine[e] = topk_load(a, tid + e * 1024);
+    topk_load(a, tid, 1024, mine);
     uint32_t best = 0;
 #pragma unroll
     for (int e = 0; e < TOPK_PER_THREAD; e++) best = max(best, (uint32_t)(mine[e] >> 32));

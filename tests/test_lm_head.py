@@ -275,3 +275,28 @@ def test_topk_selection_edges_on_device(n, cap, distinct):
     want_idx, want_val = full_sort_topk(logits, cap)
     assert np.array_equal(idx, want_idx) and np.array_equal(val.view(np.uint32), want_val.view(np.uint32))
     w.free()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,cap", [(128, 8), (128, 9), (512, 20), (512, 21), (1024, 24), (1024, 25), (8193, 8), (8193, 9), (9000, 64), (20000, 40)])
+@pytest.mark.parametrize("order", ["rising", "falling", "one_lane", "few_values"])
+def test_topk_in_any_order_of_the_logits(n, cap, order):
+    """Both sides of the lines of the dispatch again, and the three ways rlx_topk_select can go: the bound leaves no more than cap keys
+    (rising, falling: each lane's maximum is among the best), a few more (one lane holds the sixteen best of its 1024), or most of
+    them (four values in all)."""
+    value = {"rising": np.arange(n), "falling": -np.arange(n), "one_lane": np.where(np.arange(n) % 64 == 5, 1, -1) * (1 + np.arange(n)),
+             "few_values": np.arange(n) % 4}[order].astype(np.float32)
+    packed = np.zeros((n, 34), np.uint8)  # Q8_0 rows of one block: d = 1, codes (hi, lo, 0, ...) against x = (256, 1, 0, ...)
+    packed[:, 0:2] = np.frombuffer(np.float16(1).tobytes(), np.uint8)
+    hi = np.floor((value + 128) / 256)  # leaves -128 .. 127
+    packed[:, 2] = hi.astype(np.int8).view(np.uint8)
+    packed[:, 3] = (value - 256 * hi).astype(np.int8).view(np.uint8)
+    w = ops.QWeight(QuantScheme.GgufQ8_0, packed.reshape(-1), n, 32)
+    hidden = np.zeros(32, np.float32)
+    hidden[:2] = 256, 1
+    logits = ops.gguf_matmul_bt(hidden.reshape(1, 32), w, 1)[0]
+    assert np.array_equal(logits, value)
+    idx, val = ops.gguf_tied_lm_topk(hidden, w, cap)
+    want_idx, want_val = full_sort_topk(logits, cap)
+    assert np.array_equal(idx, want_idx) and np.array_equal(val, want_val)
+    w.free()
