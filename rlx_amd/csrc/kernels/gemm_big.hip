@@ -16,7 +16,8 @@
 //
 // Decoding packed weights here costs what writing them out as images first would (about 10 % of the kernel), without 2 bytes per weight
 // of workspace. A wave issues its own vector instructions under its matrix instructions: 16 x 16 x 32 alone takes 18.1 clocks, with one
-// vector instruction behind each 20.1, two 20.6, three 25.1, four 29.1. Layer of 1111 f32 tokens (Llama-3-8B, Q4_0): 1280 -> 1074 - 1118 us.
+// vector instruction behind each 20.1, two 20.6, three 25.1, four 29.1. Layer of 1111 f32 tokens (Llama-3-8B, Q4_0): 1280 -> 1074 - 1118 us
+// with an epilogue through LDS, 6 % less without.
 #include "common.h"
 
 namespace rlx {
@@ -235,7 +236,7 @@ __device__ __forceinline__ void gemm_big_body(const GemmBigArgs &a) {
 #pragma unroll
                 for (int jj = 0; jj < 2; jj++) {
                     const int x = (st & 3) * 2 + jj, j = (r & 1) ? 7 - x : x;
-                    acc[r][j] = mfma16(fa[r], fb[ph & 1][j], acc[r][j]);
+                    acc[r][j] = mfma16(fb[ph & 1][j], fa[r], acc[r][j]);  // rows of the product: columns of the result
                 }
                 __builtin_amdgcn_sched_barrier(0);
             }
@@ -255,14 +256,22 @@ __device__ __forceinline__ void gemm_big_body(const GemmBigArgs &a) {
             quantum(i + 2, 2);
             quantum(i + 3, 3);
         }
+        // The sums stay in accumulation registers until their row is stored (here and below): left to itself the allocator moves them
+        // between the register files inside the loop, some four hundred moves a quad, and spills around the epilogue.
+#pragma unroll
+        for (int i = 0; i < 8; i++)
+#pragma unroll
+            for (int j = 0; j < 8; j++) asm volatile("" : "+a"(acc[i][j]));
         __builtin_amdgcn_s_waitcnt(0);
         __syncthreads();  // nothing is on its way into LDS any more
 
-        // Epilogue. Register r of tile (i, j) is row 16 i + 4 lg + r, column 16 j + lr of the wave's quarter. Each wave turns 16 rows
-        // at a time around in LDS of its own, so that a store instruction covers 512 contiguous bytes of two rows; the rows'
-        // factors come through LDS too.
+        // Epilogue. W is the first operand of the products, so register r of tile (i, j) is row 16 i + lr, column 16 j + 4 lg + r of the
+        // wave's quarter: a lane holds four neighbouring columns and stores them as they are, four lanes 64 bytes of a row. With
+        // the rows in the registers the wave had to turn its quarter around in LDS first: 41 K clocks of the 205 K of a tile of
+        // [8192, 4096] x [4096, 4096], 17 K now; f32 rows 30 K and 12.5 K (no stores at all: 4 K). The clock that power allows takes
+        // some of it back: 277 -> 262 us, 519 -> 506 on [2222 image rows, 4096] x [28672, 4096]. The rows' factors come through LDS.
         const int rows = a.pair_rows ? 128 : 256;
-        float *fac_s = (float *)smem, *turn_w = (float *)(smem + 1024 + wave * 2 * 16 * 132 * 4);  // two buffers: rows are written while the 16 before are read
+        float *fac_s = (float *)smem;
         if (tid < rows) {
             const int row = by * rows + tid;
             fac_s[tid] = row < a.m_out ? a.rowfac[2 * row + 1] : 0.f;
@@ -272,45 +281,45 @@ __device__ __forceinline__ void gemm_big_body(const GemmBigArgs &a) {
         float *dst = piece ? a.part + ((long long)blockIdx.x * 2 + (k0 > 0 ? 0 : 1)) * rows * 256 : sg.out + ((long long)by * rows * sg.n + bx * 256);
         const int ld = piece ? 256 : sg.n;
         const int row_lim = piece ? rows : min(rows, a.m_out - by * rows), col_lim = piece ? 256 : min(256, sg.n - bx * 256);
-        const bool wide = (ld & 3) == 0 && ((uintptr_t)dst & 15) == 0;
-        const int scol = wn * 128 + (lane & 31) * 4;
-#pragma unroll
-        for (int ii = 0; ii < 9; ii++) {
-            __builtin_amdgcn_sched_barrier(0);
-            asm volatile("" ::: "memory");
-            const int i = ii;
-            int t0 = wm * 128 + i * 16;  // image row
-            float *turn_s = turn_w + (i & 1) * 16 * 132;
-            if (ii == 8) {
-            } else if (a.pair_rows) {
-#pragma unroll
-                for (int r = 0; r < 4; r += 2)
-#pragma unroll
-                    for (int j = 0; j < 8; j++)
-                        turn_s[(2 * lg + (r >> 1)) * 132 + j * 16 + lr] = (acc[i & 7][j][r] + acc[i & 7][j][r + 1] * (1.0f / BIG_LO_SCALE)) * fac_s[t0 / 2 + 2 * lg + (r >> 1)];
+        const bool wide = (ld & 3) == 0 && ((uintptr_t)dst & 15) == 0;  // then col_lim is a multiple of four
+        auto store4 = [&](float *o, int col, float4_t v) {
+            if (wide) {
+                if (col < col_lim) *(float4_t *)(o + col) = v;
             } else {
 #pragma unroll
-                for (int r = 0; r < 4; r++)
-#pragma unroll
-                    for (int j = 0; j < 8; j++) turn_s[(4 * lg + r) * 132 + j * 16 + lr] = acc[i & 7][j][r] * fac_s[t0 + 4 * lg + r];
+                for (int e = 0; e < 4; e++)
+                    if (col + e < col_lim) o[col + e] = v[e];
             }
-            asm volatile("" ::: "memory");
-            if (ii == 0) continue;
-            t0 -= 16;
-            turn_s = turn_w + ((i & 1) ^ 1) * 16 * 132;
-            const int r0 = a.pair_rows ? t0 / 2 : t0;
-            for (int g = 0; g < (a.pair_rows ? 4 : 8); g++) {
-                const int tr = 2 * g + (lane >> 5), row = r0 + tr;
-                const float4_t v = *(const float4_t *)(turn_s + tr * 132 + (lane & 31) * 4);
-                if (row < row_lim) {
-                    float *o = dst + (long long)row * ld + scol;
-                    if (wide) {  // then col_lim is a multiple of four
-                        if (scol < col_lim) __builtin_nontemporal_store(v, (float4_t *)o);
-                    } else {
+        };
+        const bool odd = lr & 1;
 #pragma unroll
-                        for (int e = 0; e < 4; e++)
-                            if (scol + e < col_lim) o[e] = v[e];
+        for (int i = 0; i < 8; i++) {
+            __builtin_amdgcn_sched_barrier(0);
+            const int t0 = wm * 128 + i * 16 + lr, row = a.pair_rows ? t0 >> 1 : t0;  // image row, output row
+            const float fac = fac_s[row];
+            float *o = dst + (long long)row * ld;
+#pragma unroll
+            for (int j = 0; j < 8; j++) asm volatile("" : "+a"(acc[i][j]));
+            if (a.pair_rows) {
+                // neighbouring lanes hold the leading and the residual sums of one row: the even lane finishes tile j, the odd one j + 1
+#pragma unroll
+                for (int j = 0; j < 8; j += 2) {
+                    float4_t v;
+#pragma unroll
+                    for (int r = 0; r < 4; r++) {
+                        const float keep = odd ? acc[i][j + 1][r] : acc[i][j][r], give = odd ? acc[i][j][r] : acc[i][j + 1][r];
+                        const float got = __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, give), 0xB1, 0xF, 0xF, true));
+                        v[r] = ((odd ? got : keep) + (odd ? keep : got) * (1.0f / BIG_LO_SCALE)) * fac;
                     }
+                    if (row < row_lim) store4(o, wn * 128 + (j + (odd ? 1 : 0)) * 16 + lg * 4, v);
+                }
+            } else if (row < row_lim) {
+#pragma unroll
+                for (int j = 0; j < 8; j++) {
+                    float4_t v;
+#pragma unroll
+                    for (int r = 0; r < 4; r++) v[r] = acc[i][j][r] * fac;
+                    store4(o, wn * 128 + j * 16 + lg * 4, v);
                 }
             }
         }
