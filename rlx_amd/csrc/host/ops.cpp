@@ -1200,8 +1200,12 @@ int rlx_mi355x_rms_norm(const float *x_dev, const float *gamma_dev, const float 
     RowOpArgs a{x_dev, gamma_dev, beta_dev, out_dev, rows, h, eps, 0, 0};
     a.vec4 = h % 4 == 0 && ((uintptr_t)x_dev | (uintptr_t)gamma_dev | (uintptr_t)beta_dev | (uintptr_t)out_dev) % 16 == 0;
     void *params[] = {&a};
-    const unsigned bx = h >= 4096 ? 1024 : 256;
-    return launch(K_RMSNORM_ROWS, (unsigned)std::min<int64_t>(rows, 1 << 20), 1, bx, 0, (hipStream_t)stream, params);
+    // Rows that up to 1024 threads can hold, four 16-byte groups each (ROW_KEEP in kernels/rowops.hip): as few threads as do, so that the
+    // rows of a prompt are on the chip at once. us, read twice against kept: 1111 rows of 4096 9.3 / 6.8, 4096 rows of 4096 26.0 / 21.0,
+    // 2000 of 16384 54 / 48; 8192 rows of 2048 22.0 / 21.9, 1111 of 1024 4.0 / 4.3 (most of the four groups past the end).
+    const bool keep = a.vec4 && h > 2048 && h <= 16384;
+    const unsigned bx = keep ? (h <= 4096 ? 256 : h <= 8192 ? 512 : 1024) : h >= 4096 ? 1024 : 256;
+    return launch(keep ? K_RMSNORM_ROWS_KEEP : K_RMSNORM_ROWS, (unsigned)std::min<int64_t>(rows, 1 << 20), 1, bx, 0, (hipStream_t)stream, params);
 }
 
 int rlx_mi355x_fused_swiglu(const float *in_dev, float *out_dev, int64_t rows, int64_t n_half, int gate_first, void *stream) {

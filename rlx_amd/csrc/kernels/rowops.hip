@@ -16,9 +16,12 @@ struct RowOpArgs {
     int vec4;           // h % 4 == 0 and every pointer 16-byte aligned
 };
 
-// rlx-cpu/src/thunk.rs:8839-8869: out = x * (1 / sqrt(mean(x^2) + eps)) * gamma + beta per row. One workgroup per row;
-// the row is read twice (the second time from cache). The sum of squares is taken per thread, then over the wave and the
-// waves in a fixed order, so results do not change from run to run.
+// rlx-cpu/src/thunk.rs:8839-8869: out = x * (1 / sqrt(mean(x^2) + eps)) * gamma + beta per row. One workgroup per row. The sum of
+// squares is taken per thread, then over the wave and the waves in a fixed order, so results do not change from run to run.
+// KEEP (rows of whole 16-byte groups, at most ROW_KEEP per thread): the row stays in registers between the sum and the product and
+// gamma is fetched beside it, so a row is one memory latency instead of three, one behind the other. Else the row is read twice.
+constexpr int ROW_KEEP = 4;
+template <bool KEEP>
 __device__ __forceinline__ void rmsnorm_rows(const RowOpArgs &a) {
     __shared__ float wave_sum[16];
     const int tid = threadIdx.x, nthr = blockDim.x;
@@ -26,10 +29,22 @@ __device__ __forceinline__ void rmsnorm_rows(const RowOpArgs &a) {
         const float *xr = a.x + row * a.h;
         float *orow = a.out + row * a.h;
         float ss = 0.f;
-        if (a.vec4) {
+        float4_t v[KEEP ? ROW_KEEP : 1], g[KEEP ? ROW_KEEP : 1];
+        if constexpr (KEEP) {
+            const int last = (int)a.h - 4;
+#pragma unroll
+            for (int u = 0; u < ROW_KEEP; u++) v[u] = *(const float4_t *)(xr + min((tid + u * nthr) * 4, last));
+#pragma unroll
+            for (int u = 0; u < ROW_KEEP; u++) g[u] = *(const float4_t *)(a.gamma + min((tid + u * nthr) * 4, last));
+#pragma unroll
+            for (int u = 0; u < ROW_KEEP; u++) {
+                const float q = v[u][0] * v[u][0] + v[u][1] * v[u][1] + v[u][2] * v[u][2] + v[u][3] * v[u][3];
+                ss += (tid + u * nthr) * 4 <= last ? q : 0.f;
+            }
+        } else if (a.vec4) {
             for (long long i = tid * 4LL; i < a.h; i += nthr * 4LL) {
-                const float4_t v = *(const float4_t *)(xr + i);
-                ss += v[0] * v[0] + v[1] * v[1] + v[2] * v[2] + v[3] * v[3];
+                const float4_t v4 = *(const float4_t *)(xr + i);
+                ss += v4[0] * v4[0] + v4[1] * v4[1] + v4[2] * v4[2] + v4[3] * v4[3];
             }
         } else {
             for (long long i = tid; i < a.h; i += nthr) ss += xr[i] * xr[i];
@@ -42,14 +57,26 @@ __device__ __forceinline__ void rmsnorm_rows(const RowOpArgs &a) {
         for (int w = 0; w < (nthr >> 6); w++) total += wave_sum[w];
         __syncthreads();  // wave_sum is written again for the next row
         const float inv = 1.0f / __builtin_sqrtf(total * (1.0f / (float)a.h) + a.eps);
-        if (a.vec4) {
-            for (long long i = tid * 4LL; i < a.h; i += nthr * 4LL) {
-                const float4_t v = *(const float4_t *)(xr + i), g = *(const float4_t *)(a.gamma + i);
+        if constexpr (KEEP) {
+#pragma unroll
+            for (int u = 0; u < ROW_KEEP; u++) {
+                const int i = (tid + u * nthr) * 4;
+                if (i >= a.h) continue;
                 float4_t b = {0.f, 0.f, 0.f, 0.f};
                 if (a.beta) b = *(const float4_t *)(a.beta + i);
                 float4_t o;
 #pragma unroll
-                for (int e = 0; e < 4; e++) o[e] = v[e] * inv * g[e] + b[e];
+                for (int e = 0; e < 4; e++) o[e] = v[u][e] * inv * g[u][e] + b[e];
+                *(float4_t *)(orow + i) = o;
+            }
+        } else if (a.vec4) {
+            for (long long i = tid * 4LL; i < a.h; i += nthr * 4LL) {
+                const float4_t v4 = *(const float4_t *)(xr + i), g4 = *(const float4_t *)(a.gamma + i);
+                float4_t b = {0.f, 0.f, 0.f, 0.f};
+                if (a.beta) b = *(const float4_t *)(a.beta + i);
+                float4_t o;
+#pragma unroll
+                for (int e = 0; e < 4; e++) o[e] = v4[e] * inv * g4[e] + b[e];
                 *(float4_t *)(orow + i) = o;
             }
         } else {
@@ -88,5 +115,6 @@ __device__ __forceinline__ void swiglu_rows(const RowOpArgs &a) {
 
 }  // namespace rlx
 
-extern "C" __global__ __launch_bounds__(1024) void rlx_rmsnorm_rows(rlx::RowOpArgs a) { rlx::rmsnorm_rows(a); }
+extern "C" __global__ __launch_bounds__(1024) void rlx_rmsnorm_rows(rlx::RowOpArgs a) { rlx::rmsnorm_rows<false>(a); }
+extern "C" __global__ __launch_bounds__(1024) void rlx_rmsnorm_rows_keep(rlx::RowOpArgs a) { rlx::rmsnorm_rows<true>(a); }
 extern "C" __global__ __launch_bounds__(256) void rlx_swiglu_rows(rlx::RowOpArgs a) { rlx::swiglu_rows(a); }

@@ -115,3 +115,19 @@ def test_rmsnorm_argument_errors():
     with pytest.raises(rlx_amd.RlxError, match="decode path"):
         ops.rmsnorm_gguf_matmul_bt_batch(np.zeros((9, 256), np.float32), np.ones(256, np.float32), None, 1e-5, [w], 9)
     w.free()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("h", [2048, 2052, 2056, 4096, 4100, 8192, 8196, 14336, 16384, 16388, 4097])
+@pytest.mark.parametrize("rows,with_beta", [(1, True), (700, False)])
+def test_rms_norm_rows_kept_in_registers(h, rows, with_beta):
+    """Both sides of every row length at which rlx_rmsnorm_rows_keep changes its workgroup or hands over to the kernel that reads a row twice."""
+    rng = np.random.default_rng(h + rows)
+    x = (rng.standard_normal((rows, h)) * 3).astype(np.float32)
+    gamma = rng.standard_normal(h).astype(np.float32)
+    beta = rng.standard_normal(h).astype(np.float32) if with_beta else None
+    got = ops.rms_norm(x, gamma, beta, 1e-5)
+    x64 = x.astype(np.float64)
+    want = x64 / np.sqrt((x64 ** 2).mean(axis=1, keepdims=True) + 1e-5) * gamma + (0 if beta is None else beta)
+    # per thread at most 64 additions of squares, then a tree: the factor is good to 32 ulp, the element itself adds four roundings
+    assert np.max(np.abs(got - want) / np.maximum(np.abs(want), 1.0)) <= 36 * 2.0 ** -24
