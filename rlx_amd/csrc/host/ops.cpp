@@ -442,12 +442,12 @@ static GemmSplit wide_split(const Layout &L, const WeightDims &D, int64_t m, siz
 // The 256 x 256 tiles of kernels/gemm_big.hip (Q4_0, Q8_0, code images) against the 256 x 128 tiles of kernels/gemm.hip, and how the
 // former are handed out: a tile per workgroup, or the whole line of (tile, 128 columns of K) items in equal runs, one per CU, with
 // the pieces of shared tiles added by a launch of their own. `groups` = 0: the 256 x 128 tiles. Estimated times decide. Their constants,
-// in us, are fitted to 1740 random shapes and checked on 500 more (130 - 8192 image rows, K 512 - 28672, one to four matrices), each
-// timed all three ways, for f32 rows, 16-bit rows and code images apart: these differ in the bytes of a piece and in what a tile's
-// columns cost (no decode on code images). The whole call is 1.03, 1.02 and 1.12 times as fast there as with the smaller tiles on
-// average (1.4 at best, 0.955 at worst) and within 1 % of the fastest of the three on average. Some of them, smaller / whole / shared:
-// f32 [1111, 14336] x 4096 386 / 385 / 272, [528, 6944] x 3426 102 / 190 / 112; bf16 [1424, 8416] x 2794 125 / 236 / 145; codes
-// [3763, 6432] x 2598 282 / 207 / 288, [3138, 6720] x 5014 359 / 364 / 303.
+// in us, are fitted to 1740 random shapes (130 - 8192 image rows, K 512 - 28672, one to four matrices), each timed all three ways, for
+// f32 rows, 16-bit rows and code images apart: these differ in the bytes of a piece and in what a tile's columns cost (no decode on
+// code images). The whole call is 1.06, 1.03 and 1.13 times as fast there as with the smaller tiles on average (1.4 at best, 0.94 at
+// worst) and within 1 % of the fastest of the three on average; against the constants fitted to an epilogue that was twice as long
+// 1.013, 1.008 and 1.005 (1.2 at best, 0.96 at worst). Some of them, smaller / whole / shared: f32 [528, 6944] x 3426 102 / 186 / 94 (the estimate
+// stays with the smaller ones here); bf16 [1424, 8416] x 2794 126 / 230 / 116; codes [3763, 6432] x 2598 276 / 203 / 274, [3138, 6720] x 5014 364 / 362 / 302.
 // Shared tiles of one row of A are at the same K at the same time, and read A together, where their workgroups, 256 / tiles_n apart, are
 // a whole number apart: gcd(tiles_n, 256) at a time. Alone, each reads A by itself: the kernel on code images of 22 x 12 tiles of 6912
 // columns 212 us, of 24 x 11 tiles 305. Packed weights, whose bytes are a quarter or half, feel it less.
@@ -464,9 +464,9 @@ struct BigCosts {
     double alone, pairs;               // added share of the latter where A is read by one workgroup or two at a time
     double sparse_margin;              // shared tiles against a grid that is not full: the estimate's error there
 };
-constexpr BigCosts BIG_COSTS_F32{0, 1.64, 0.96, 6.5, 7e-8, 8.2, 2.95, 41.6, 3.04, 0.05, 0.05, 0.956};
-constexpr BigCosts BIG_COSTS_16{0.8, 1.83, 0.85, 6.3, 3.4e-7, 13.1, 3.13, 54.3, 3.5, 0.093, 0.035, 0.948};
-constexpr BigCosts BIG_COSTS_CODES{3.8, 1.485, 0.737, 4.5, 1.2e-7, 14.2, 1.752, 52.7, 2.027, 0.56, 0.137, 0.99};
+constexpr BigCosts BIG_COSTS_F32{0, 1.64, 0.96, 6.5, 7e-8, 1.48, 3.024, 37.4, 2.792, 0.148, 0.14, 0.998};
+constexpr BigCosts BIG_COSTS_16{0.8, 1.83, 0.85, 6.3, 3.4e-7, 6.51, 3.285, 45.3, 3.455, 0.085, 0.021, 0.999};
+constexpr BigCosts BIG_COSTS_CODES{3.8, 1.485, 0.737, 4.5, 1.2e-7, 9.822, 1.734, 27.032, 2.271, 0.502, 0.192, 0.985};
 constexpr double IMG_START = 5.5, IMG_QUAD = 2.3;  // a round of rlx_gemm_img_f16w, every 128 columns of it
 constexpr int64_t IMG_MAX_K = 2304;              // up to here rlx_gemm_img_f16w instead of rlx_gemm_big_f16w: its way in and out of a tile is shorter (kernels/gemm.hip)
 static BigPlan big_plan(int scheme, int xk, int64_t m, int64_t m_rows, int64_t tiles_n, int64_t half_tiles_n, int64_t n_sum, int64_t quads, size_t part_room) {
@@ -493,7 +493,10 @@ static BigPlan big_plan(int scheme, int xk, int64_t m, int64_t m_rows, int64_t t
     const size_t part = (size_t)cus * 2 * (size_t)(xk == 0 ? 128 : 256) * 1024;  // a workgroup leaves at most two pieces
     if (part <= part_room && tiles * quads >= cus) {
         const double quad = c.shared_quad * (1 + (tiles_n % 2 ? c.alone : tiles_n % 4 ? c.pairs : 0));
-        if (c.shared_start + (double)rounds(tiles * quads) * quad < (sparse ? c.sparse_margin : 1) * (whole ? t_whole : t_half)) return BigPlan{(int)cus, part};
+        // From three rounds of whole tiles on there is little left to fill, and the estimates are within a few percent of each other:
+        // f32 [1111, 4096] x 28672, 3.94 rounds, layer 1059 us shared, 1052 whole.
+        const double margin = sparse ? c.sparse_margin : whole && rounds(tiles) > 2 ? 0.97 : 1;
+        if (c.shared_start + (double)rounds(tiles * quads) * quad < margin * (whole ? t_whole : t_half)) return BigPlan{(int)cus, part};
     }
     return whole ? BigPlan{(int)tiles, 0} : none;
 }
