@@ -8,9 +8,9 @@
 //
 // Four waves, one per SIMD, own 128 x 128 of the 256 x 256 tile each (256 accumulator registers): sixteen fragment reads feed 64
 // matrix instructions. K advances in 32-column quanta through a ring of LDS slots that buffer loads fill directly; one barrier per
-// quantum. What bounds it is the loop: [8192, 4096] x [4096, 4096] on ready images takes 450 K clocks, on drawn data as on zeros, and
-// the matrix unit is busy for 57 % of them; the data moves the clock by a tenth (2.09 against 2.32 GHz: 219 against 193 us in a burst,
-// 1.2 PFLOP/s sustained). 16 x 16 x 32 instructions read and write half the accumulator bits per product of 32 x 32 x 16 ones: 210 us
+// quantum. What bounds it is power: on [8192, 4096] x [4096, 4096] ready images the loop takes 160 K clocks a tile, 19.5 per matrix instruction
+// (16 and a bubble of 2 at best), at the 1.5 - 1.6 GHz that sustained products of drawn data leave of 2.4; 1.0 - 1.1 PFLOP/s. With packed weights decoded in
+// it 26.6 clocks at 1.8 - 2.0 GHz, as much. 16 x 16 x 32 instructions read and write half the accumulator bits per product of 32 x 32 x 16 ones: 210 us
 // against 229 (and 232 for eight waves of 128 x 64 on 32 x 32 x 16, the kernel before).
 // An XCD-wise tile order and a ring without address arithmetic (four slots, depth two) measured the same or 2 % slower.
 //
