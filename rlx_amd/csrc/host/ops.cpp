@@ -306,6 +306,12 @@ static int launch_gemv(const void *const *xs, int xk, const rlx_qweight *const *
         // the RMSNorm prologue (GEMV_LDS_TAIL in kernels/gemv.hip)
         constexpr size_t LDS_TAIL = 384;
         while (sh.kcu > 1 && part_bytes + stage_bytes(sh.kcu) + LDS_TAIL > budget) sh.kcu--;
+        // Where the staging of a chunk is even over the waves (8 f32 or 16 sixteen-bit rows on sixteen of them, 16 f32 rows on eight), so are
+        // its units: 17 units leave fifteen waves waiting for one, chunk after chunk. us, Q4_0 / Q8_0 / Q4_K / Q5_K: [4096, 14336], 8 f32
+        // rows 22.2 / 24.8 / 24.7 / 27.4 -> 20.3 / 23.8 / 22.4 / 25.0, [8192, 28672] 47.1 / 57.4 / 55.2 / 65.8 -> 43.2 / 55.1 / 51.0 / 59.5; 16 f32 rows
+        // 91 / 97 -> 79 / 84 there (Q4_0, Q8_0). With other row counts the waves' shares of the staging differ, which uneven units happen to make up for:
+        // 5 - 7 and 10 f32 rows 3 - 20 % slower, 12 16-bit rows 8 %.
+        if ((rv == 16 || (xk == 0 && m == 16)) && sh.kcu < max_units && sh.kcu > kw) sh.kcu -= sh.kcu % kw;
         sh.fits = part_bytes + stage_bytes(sh.kcu) + LDS_TAIL <= budget;
         sh.lds = part_bytes + stage_bytes(sh.kcu) + LDS_TAIL;
         sh.a.nseg = count;

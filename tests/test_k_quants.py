@@ -12,7 +12,7 @@ import pytest
 import oracle
 import rlx_amd
 from rlx_amd import DType, QuantScheme, ops
-from helpers import BLOCK, Q2K, Q3K, Q4K, Q5K, Q6K, Q8K, decode_device_layout, random_blocks, rel_err
+from helpers import BLOCK, Q2K, Q3K, Q4K, Q4_0, Q5K, Q6K, Q8K, Q8_0, decode_device_layout, random_blocks, rel_err
 
 PACKED = (Q5K, Q6K, Q8K, Q2K, Q3K)
 FIVE = PACKED
@@ -477,3 +477,23 @@ def test_k_quant_grouped_matmul(scheme, m):
     got = ops.gguf_grouped_matmul_bt(x, w, idx)
     w.free()
     assert rel_err(got, oracle.gguf_grouped_matmul_f64(x, packed, idx, m, k, n, experts, scheme)) <= 2e-3
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("scheme", [Q4_0, Q8_0, Q4K])
+@pytest.mark.parametrize("m,dtype", [(8, DType.F32), (16, DType.F32), (16, DType.BF16)])
+@pytest.mark.parametrize("k,n", [(4352, 48), (14336, 33), (28672, 16)])
+def test_chunks_of_whole_rounds(scheme, m, dtype, k, n):
+    """Row counts at which a staged chunk of K holds a multiple of the waves of a tile: one chunk and a little, several, many."""
+    rng = np.random.default_rng(k + m)
+    p = ops.quantize(QuantScheme(scheme), (rng.standard_normal(n * k) * 0.02).astype(np.float32))
+    x = rng.standard_normal((m, k)).astype(np.float32)
+    if dtype == DType.BF16:
+        x = (x.view(np.uint32) & np.uint32(0xFFFF0000)).view(np.float32)
+    w = ops.QWeight(QuantScheme(scheme), p, n, k)
+    got = ops.gguf_matmul_bt((x.view(np.uint32) >> 16).astype(np.uint16) if dtype == DType.BF16 else x, w, m, dtype)
+    want = x.astype(np.float64) @ oracle.dequant(scheme, p, n * k).reshape(n, k).astype(np.float64).T
+    # at most 896 f32 additions of block sums, a random walk of half an ulp of the largest values: 2^-24 sqrt(896). Q4_K's
+    # code and min terms are each up to four times their difference.
+    assert np.max(np.abs(got - want)) <= (7.2e-6 if scheme == Q4K else 1.8e-6) * np.max(np.abs(want))
+    w.free()
