@@ -72,10 +72,10 @@ __device__ __forceinline__ uint32_t div_by(uint32_t x, uint32_t magic) { return 
 constexpr int XS_PAD_HALFS = 8;      // 16 bytes of padding per LDS row: rows land in different bank groups
 constexpr float LO_SCALE = 2048.0f;  // f32 activation x = hi + lo / LO_SCALE with hi, lo binary16
 
-// The last GEMV_LDS_TAIL bytes of a workgroup's LDS: [0,128) un-scale factor per virtual activation row and [128,256) per logical
-// row the bits of max |x| of the staged chunk, then the forward scale (both only in the slow pass, below); [256,264) two row
-// masks, OR-ed together by the waves in the common pass; [272,384) sums of squares per (row, slice) (RMSNorm prologue: at most
-// eight rows, so 23 slices with sixteen waves).
+// The last GEMV_LDS_TAIL bytes of a workgroup's LDS: [0,128) un-scale factor per virtual activation row (slow pass, below; per
+// logical row in the common pass of an RMSNorm prologue) and [128,256) per logical row the bits of max |x| of the staged chunk,
+// then the forward scale (slow pass only); [256,264) two row masks, OR-ed together by the waves in the common pass; [272,384)
+// sums of squares per (row, slice) (RMSNorm prologue: at most eight rows, so 21 slices with sixteen waves).
 //
 // Activations travel as binary16. A row whose values leave the range binary16 carries well - some |x| >= 2^15, or no
 // |x| >= 2^-8 at all - is multiplied by a power of two that puts its largest value in [2^14, 2^15) while it is staged,
@@ -434,11 +434,17 @@ __device__ __forceinline__ void compute_unit(const UnitRegs<SCHEME> &w, const ha
     }
 }
 
-// RMSNorm prologue: out = (sum of x gamma w) / rms(x). The activations are staged as x gamma, their squares are summed on the way
-// (one sum per (row, slice) task, in `sums`), and the epilogue multiplies by the row's 1 / sqrt(mean + eps): x is read once and
-// nothing waits for the sum. (The slow pass, below, knows the sums and stages the normalized values.) With the normalization in the staging a second read of x and a barrier stood in front of the first
-// product: 2 us of a launch of one row of 4096 columns, and 4.5 us when one wave made the sum ahead of the first weights (the gate /
-// up launch of a Llama-3-8B layer 21.9 us then).
+// RMSNorm prologue: out = (sum of x gamma w) / rms(x). The activations are staged as x gamma 2^s, their squares are summed on the
+// way (one sum per (row, slice) task, in `sums`), and the epilogue multiplies by the row's 1 / sqrt(mean + eps) and 2^-s: x is read
+// once and nothing waits for the sum. With the normalization in the staging a second read of x and a barrier stood in front of the
+// first product: 2 us of a launch of one row of 4096 columns, and 4.5 us when one wave made the sum ahead of the first weights
+// (the gate / up launch of a Llama-3-8B layer 21.9 us then).
+// The power of two, from the row's first four columns (norm_prescale), does for the range what the normalization would: x gamma itself
+// is outside what binary16 carries well in rows of small or large activations, and a launch with one such row ran the common and
+// the slow pass, 1.3 to 2 times as long (us, rows of 2^-12: gate / up [14336, 4096] Q4_K, six rows, 44.8; q / k / v of 4096 columns,
+// Q4_0, one row, 16.3; normalized in the staging 25.2 and 11.5; now 22.5 and 8.8). It costs a launch 0.05 - 0.1 us. What is left to
+// the slow pass: rows whose largest x gamma is 2^15 times those columns or more, or all below 2^-8 of them. It knows the sums and
+// stages the normalized values.
 // A beta (null in most models) has to be added to the normalized value: then the squares are summed first.
 __device__ __forceinline__ float wave_sum(float v) {  // the total, in lane 63
     auto add = [&](auto ctrl, auto rows) {
@@ -476,6 +482,19 @@ __device__ __forceinline__ float norm_scale(const GemvArgs &a, int k, const floa
     return 1.0f / sqrtf(sq * (1.0f / (float)k) + a.eps);
 }
 
+__device__ __forceinline__ float max3_abs(float acc, float x, float y) {  // max(acc, |x|, |y|); a NaN operand is skipped
+    float r;
+    asm("v_max3_f32 %0, %1, |%2|, |%3|" : "=v"(r) : "v"(acc), "v"(x), "v"(y));
+    return r;
+}
+// 2^-s of a row: the largest |x| of its first four columns (`x4`, as bits) times 2^s is in [1, 2). 1 where that value is 0 or beyond
+// 2^+-63: there squares may under- or overflow, and the slow pass does what f32 arithmetic does.
+__device__ __forceinline__ float norm_prescale(uint4_t x4) {
+    const uint32_t b = max(max(x4[0] & 0x7FFFFFFFu, x4[1] & 0x7FFFFFFFu), max(x4[2] & 0x7FFFFFFFu, x4[3] & 0x7FFFFFFFu));
+    return __builtin_bit_cast(float, b >= 64u << 23 && b < 191u << 23 ? b & 0x7F800000u : 127u << 23);
+}
+__device__ __forceinline__ float pow2_inverse(float p) { return __builtin_bit_cast(float, (254u << 23) - __builtin_bit_cast(uint32_t, p)); }
+
 // Convert one K chunk of the activations into LDS as halfs: f32 -> hi rows [0,m) + lo rows [m,2m); 16-bit -> rows [0,m).
 // The work is cut into (row, slice of the row's 16-byte groups) tasks, one wave per task: with fewer rows than waves a row
 // is shared by several waves, otherwise a wave takes whole rows in turn. A wave therefore works on one row at a time -
@@ -487,15 +506,11 @@ __device__ __forceinline__ float norm_scale(const GemvArgs &a, int k, const floa
 // multiplied by fwd[r].
 // Every wave of the launch runs PASS 0 at the same moment, before there is other work to hide it behind, so its VALU
 // count is launch latency: the largest |x| costs one v_max3_f32 per two values.
-__device__ __forceinline__ float max3_abs(float acc, float x, float y) {  // max(acc, |x|, |y|); a NaN operand is skipped
-    float r;
-    asm("v_max3_f32 %0, %1, |%2|, |%3|" : "=v"(r) : "v"(acc), "v"(x), "v"(y));
-    return r;
-}
-template <int XD, bool NORM = false, int PASS = 0>
+enum { NORM_NONE = 0, NORM_SUMS = 1, NORM_KNOWN = 2 };  // RMSNorm prologue: on the sums; in the staging, the squares' sums being known
+template <int XD, int NORM = NORM_NONE, int PASS = 0>
 __device__ __forceinline__ void stage_x_typed(const GemvArgs &a, const GemvSeg &sg, half_t *xs, int row_stride, int k0, int kc,
                                               float *norm_sums = nullptr, uint32_t *masks = nullptr, uint32_t *rowmax = nullptr,
-                                              const float *fwd = nullptr) {
+                                              const float *fwd = nullptr, float *unscale = nullptr) {
     constexpr int U = NORM ? 4 : 8;  // (with a norm, gamma is loaded beside them)
     constexpr int G = XD == X_F32 ? 4 : 8;  // columns per 16-byte load
     constexpr int ESZ = XD == X_F32 ? 4 : 2;
@@ -517,8 +532,10 @@ __device__ __forceinline__ void stage_x_typed(const GemvArgs &a, const GemvSeg &
         float rowscale = 1.f, scale = 1.f;
         float sq = 0.f;
         if constexpr (PASS == 2) rowscale = fwd[row];
-        if constexpr (NORM)
-            if (PASS != 0 || a.beta) scale = norm_scale(a, sg.k, norm_sums, row);
+        if constexpr (NORM == NORM_KNOWN) scale = norm_scale(a, sg.k, norm_sums, row);
+        uint4_t x4;
+        if constexpr (NORM == NORM_SUMS)  // through the scalar cache, under the loads below
+            x4 = *(const uint4_t __attribute__((address_space(4))) *)(uintptr_t)((const float *)sg.x + (long long)row * sg.k);
         for (int cg0 = g0 + lane; cg0 < g1; cg0 += 64 * U) {
             raw_t raw[U];
             float4_t gm[NORM ? U : 1];  // fetched with the activations, not behind them
@@ -534,6 +551,11 @@ __device__ __forceinline__ void stage_x_typed(const GemvArgs &a, const GemvSeg &
                     if (cg0 + 64 * u < g1 && k0 + c < sg.k) gm[u] = *(const float4_t *)(a.gamma + k0 + c);
                 }
             }
+            if constexpr (NORM == NORM_SUMS) {
+                uint4_t y4 = x4;
+                asm volatile("" : "+s"(y4));  // not ahead of the loads
+                scale = pow2_inverse(norm_prescale(y4));
+            }
 #pragma unroll
             for (int u = 0; u < U; u++) {
                 const int c = (cg0 + 64 * u) * G;
@@ -541,7 +563,7 @@ __device__ __forceinline__ void stage_x_typed(const GemvArgs &a, const GemvSeg &
                 if constexpr (XD == X_F32) {
                     half4_t hi, lo;
                     float4_t bt = {0.f, 0.f, 0.f, 0.f};
-                    if constexpr (NORM) {
+                    if constexpr (NORM == NORM_KNOWN) {
                         if (a.beta && k0 + c < sg.k) bt = *(const float4_t *)(a.beta + k0 + c);
                     }
 #pragma unroll
@@ -551,8 +573,9 @@ __device__ __forceinline__ void stage_x_typed(const GemvArgs &a, const GemvSeg &
                         for (int i = 0; i < 2; i++) {
                             v[i] = raw[u][e + i];
                             if constexpr (NORM) {
-                                if constexpr (PASS == 0) sq += v[i] * v[i];
-                                v[i] = v[i] * scale * gm[u][e + i] + bt[e + i];  // scale 1: x gamma
+                                if constexpr (NORM == NORM_SUMS) sq += v[i] * v[i];
+                                v[i] = v[i] * scale * gm[u][e + i];
+                                if constexpr (NORM == NORM_KNOWN) v[i] += bt[e + i];  // in_row[i] * inv_rms * gamma[i] + beta[i], unfused
                             }
                         }
                         if constexpr (PASS != 2) vmax = max3_abs(vmax, v[0], v[1]);
@@ -600,9 +623,12 @@ __device__ __forceinline__ void stage_x_typed(const GemvArgs &a, const GemvSeg &
                 }
             }
         }
-        if constexpr (NORM && PASS == 0) {
+        if constexpr (NORM == NORM_SUMS) {
             sq = wave_sum(sq);
-            if (lane == 63 && !a.beta) norm_sums[t] = k0 == 0 ? sq : norm_sums[t] + sq;  // the same wave takes task t of every chunk
+            if (lane == 63) {
+                norm_sums[t] = k0 == 0 ? sq : norm_sums[t] + sq;  // the same wave takes task t of every chunk
+                if (slice == 0) unscale[row] = norm_prescale(x4);
+            }
         }
         if constexpr (XD != X_F16) {
             if constexpr (PASS == 0) {  // into the wave's two masks: one vote each per task
@@ -623,11 +649,13 @@ template <bool NORM>
 __device__ __forceinline__ void stage_chunk(const GemvArgs &a, const GemvSeg &sg, half_t *xs, int row_stride, int k0, int kc, uint8_t *tail,
                                             uint32_t *wm) {
     if constexpr (NORM) {
-        stage_x_typed<X_F32, true, 0>(a, sg, xs, row_stride, k0, kc, (float *)(tail + GEMV_NORM_SUMS), wm);
+        float *sums = (float *)(tail + GEMV_NORM_SUMS);
+        if (a.beta) stage_x_typed<X_F32, NORM_KNOWN, 0>(a, sg, xs, row_stride, k0, kc, sums, wm);
+        else stage_x_typed<X_F32, NORM_SUMS, 0>(a, sg, xs, row_stride, k0, kc, sums, wm, nullptr, nullptr, (float *)tail);
     } else {
-        if (a.x_dtype == X_F32) stage_x_typed<X_F32, false, 0>(a, sg, xs, row_stride, k0, kc, nullptr, wm);
-        else if (a.x_dtype == X_BF16) stage_x_typed<X_BF16, false, 0>(a, sg, xs, row_stride, k0, kc, nullptr, wm);
-        else stage_x_typed<X_F16, false, 0>(a, sg, xs, row_stride, k0, kc, nullptr, wm);
+        if (a.x_dtype == X_F32) stage_x_typed<X_F32>(a, sg, xs, row_stride, k0, kc, nullptr, wm);
+        else if (a.x_dtype == X_BF16) stage_x_typed<X_BF16>(a, sg, xs, row_stride, k0, kc, nullptr, wm);
+        else stage_x_typed<X_F16>(a, sg, xs, row_stride, k0, kc, nullptr, wm);
     }
     __syncthreads();
 }
@@ -646,7 +674,7 @@ __device__ __forceinline__ void stage_chunk_rescaled(const GemvArgs &a, const Ge
         rsv[tid] = 1.f;
     }
     __syncthreads();
-    stage_x_typed<XD, NORM, 1>(a, sg, xs, row_stride, k0, kc, norm_sums, nullptr, rowmax);
+    stage_x_typed<XD, NORM ? NORM_KNOWN : NORM_NONE, 1>(a, sg, xs, row_stride, k0, kc, norm_sums, nullptr, rowmax);
     __syncthreads();
     if (tid < a.m) {
         const uint32_t mb = rowmax[tid];
@@ -663,7 +691,7 @@ __device__ __forceinline__ void stage_chunk_rescaled(const GemvArgs &a, const Ge
         ((float *)rowmax)[tid] = fwd;
     }
     __syncthreads();
-    stage_x_typed<XD, NORM, 2>(a, sg, xs, row_stride, k0, kc, norm_sums, nullptr, nullptr, (const float *)rowmax);
+    stage_x_typed<XD, NORM ? NORM_KNOWN : NORM_NONE, 2>(a, sg, xs, row_stride, k0, kc, norm_sums, nullptr, nullptr, (const float *)rowmax);
     __syncthreads();
 }
 
@@ -924,7 +952,7 @@ __device__ __forceinline__ bool gemv_pass(const GemvArgs &a) {
         const int col = idx & 15, t = (int)div_by(idx >> 4, a.m_div), mr = (idx >> 4) - t * a.m;
         float scale = 1.f;
         if constexpr ((MODE & GEMV_NORM) != 0 && !SLOW)
-            if (!a.beta) scale = norm_scale(a, seg.k, (const float *)(tail + GEMV_NORM_SUMS), mr);
+            if (!a.beta) scale = norm_scale(a, seg.k, (const float *)(tail + GEMV_NORM_SUMS), mr) * rsv[mr];
         auto tile_sum = [&](int vt) {
             const float *slot = part + (size_t)vt * kw * slot_floats + mr * 16 + col;
             // (f64 with a norm: the factor at the end is then the only rounding, where a product's own used to be the last)

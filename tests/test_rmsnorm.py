@@ -65,8 +65,8 @@ def test_rmsnorm_prologue_matches_norm_then_matmul(scheme, m, k, ns, with_beta):
 @pytest.mark.parametrize("scheme,m,k,n", [(Q4_0, 1, 128, 33), (Q8_0, 5, 2080, 48), (Q4K, 7, 1024, 272), (Q4_0, 3, 4096, 4112), (Q8_0, 8, 14336, 16)])
 @pytest.mark.parametrize("size", [1e-6, 1.0, 1e6, 1e21])
 def test_rmsnorm_scale_is_applied_to_the_sums(scheme, m, k, n, size):
-    """x gamma is staged and the sums are scaled, unless x gamma is outside the range of binary16 (the first and the last two sizes:
-    normalized values are staged then); squares that overflow make a factor of 0, as in the reference's own f32 arithmetic."""
+    """x gamma times a power of two is staged and the sums are scaled; squares that overflow (the last size) make a factor of 0, as in
+    the reference's own f32 arithmetic."""
     rng = np.random.default_rng(5)
     x = (rng.standard_normal((m, k)) * size).astype(np.float32)
     gamma = (1.0 + 0.1 * rng.standard_normal(k)).astype(np.float32)
@@ -82,6 +82,47 @@ def test_rmsnorm_scale_is_applied_to_the_sums(scheme, m, k, n, size):
         # at most 448 f32 additions of block sums, a random walk of half an ulp of the row's largest values: 2^-24 sqrt(448)
         assert np.max(np.abs(got - ref)) <= 1.3e-6 * np.max(np.abs(ref))
     w.free()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("scheme,m,k,n", [(Q4_0, 1, 128, 33), (Q4_0, 1, 4096, 64), (Q8_0, 8, 14336, 16), (Q4K, 6, 2048, 272)])
+def test_rmsnorm_launch_takes_rows_of_any_size(scheme, m, k, n):
+    """Without eps the outputs of x and of x 2^p have the same bits as long as both go the same way: every factor on it is a power of two.
+    (The slow pass stages normalized values, whose roundings differ.)"""
+    rng = np.random.default_rng(6)
+    x = rng.standard_normal((m, k)).astype(np.float32)
+    gamma = (1.0 + 0.1 * rng.standard_normal(k)).astype(np.float32)
+    w = ops.QWeight(QuantScheme(scheme), weights(scheme, n, k, 21), n, k)
+    first = ops.rmsnorm_gguf_matmul_bt_batch(x, gamma, None, 0.0, [w], m)[0]
+    for p in (-40, -13, -9, 12, 14, 30):
+        assert np.array_equal(ops.rmsnorm_gguf_matmul_bt_batch(x * np.float32(2.0 ** p), gamma, None, 0.0, [w], m)[0], first), p
+    w.free()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("scheme,m,k,n", [(Q4_0, 1, 512, 33), (Q8_0, 3, 2080, 48), (Q4K, 8, 14336, 16)])
+@pytest.mark.parametrize("first,largest", [(0.0, 2.0 ** p) for p in (-13, -10, -9, -8, -7, 0, 14, 15, 17)] +
+                         [(1.0, 2.0 ** p) for p in (13, 14, 15, 16, 20)] + [(2.0 ** -20, 1.0), (2.0 ** 40, 2.0 ** 41)])
+@pytest.mark.parametrize("gamma_size,with_beta", [(1.0, False), (1.0, True), (2.0 ** 16, True)])
+def test_rmsnorm_range_around_the_limits(scheme, m, k, n, first, largest, gamma_size, with_beta):
+    """Rows whose first columns (`first`) say little about the largest value: zeros, or smaller by as much as the range of binary16. With
+    a beta, or a large gamma, normalized values are staged."""
+    rng = np.random.default_rng(7)
+    x = np.clip(rng.standard_normal((m, k)) / 4, -1, 1) * largest
+    x[:, 300] = largest
+    x[:, :256] = np.clip(rng.standard_normal((m, 256)) / 2, -1, 1) * first
+    x = x.astype(np.float32)
+    gamma = (gamma_size * (1.0 + 0.1 * rng.standard_normal(k))).astype(np.float32)
+    beta = (0.05 * rng.standard_normal(k)).astype(np.float32) if with_beta else None
+    p = weights(scheme, n, k, 22)
+    w = ops.QWeight(QuantScheme(scheme), p, n, k)
+    got = ops.rmsnorm_gguf_matmul_bt_batch(x, gamma, beta, 1e-12, [w], m)[0]
+    w.free()
+    x64 = x.astype(np.float64)
+    xn = x64 / np.sqrt((x64 ** 2).mean(axis=1, keepdims=True) + 1e-12) * gamma + (0 if beta is None else beta)
+    ref = xn @ oracle.dequant(scheme, p, n * k).reshape(n, k).astype(np.float64).T
+    # at most 448 f32 additions of block sums, a random walk of half an ulp of the row's largest values: 2^-24 sqrt(448)
+    assert np.max(np.abs(got - ref)) <= 1.3e-6 * np.max(np.abs(ref))
 
 
 @pytest.mark.gpu
