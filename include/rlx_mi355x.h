@@ -173,6 +173,10 @@ size_t rlx_mi355x_gguf_matmul_workspace(int scheme, int x_dtype, int64_t m, int6
  * more than the largest of them. Needs no GPU; without one the 256 CUs of the part are assumed. No counterpart in the reference. */
 int rlx_mi355x_gguf_matmul_plan(int scheme, int x_dtype, int64_t m, int64_t k, const int64_t *ns, int count, size_t workspace_bytes,
                                 size_t *want_bytes, char *buf, size_t cap);
+/* What one decode launch of up to eight matrices [ns[i], k] on x[m, k] looks like, as text in `buf` (may be NULL): kernel, workgroups,
+ * waves, waves on one tile of 16 rows, tiles of a workgroup, units of K that are staged at a time. Needs no GPU; without one the
+ * 256 CUs of the part are assumed. No counterpart in the reference. */
+int rlx_mi355x_gguf_decode_plan(int scheme, int x_dtype, int64_t m, int64_t k, const int64_t *ns, int count, char *buf, size_t cap);
 /* `count` independent matmuls of one scheme, batch size m and activation dtype in one launch per eight of them:
  * outs_dev[i][m, n_i] = xs_dev[i][m, k_i] . W_i^T. No counterpart in the reference, which runs one thunk per node;
  * the graph level uses it to issue together every DequantMatMul whose inputs are ready at the same point of the

@@ -81,6 +81,7 @@ SIGNATURES = {
     "rlx_mi355x_gguf_matmul_bt": (_i, [_vp, _i, _vp, _vp, _i64, _vp, _sz, _vp]),
     "rlx_mi355x_gguf_matmul_workspace": (_sz, [_i, _i, _i64, _i64, _i64]),
     "rlx_mi355x_gguf_matmul_plan": (_i, [_i, _i, _i64, _i64, C.POINTER(_i64), _i, _sz, C.POINTER(_sz), C.c_char_p, _sz]),
+    "rlx_mi355x_gguf_decode_plan": (_i, [_i, _i, _i64, _i64, C.POINTER(_i64), _i, C.c_char_p, _sz]),
     "rlx_mi355x_gguf_matmul_bt_batch": (_i, [_pvp, _i, _pvp, _pvp, _i, _i64, _vp, _sz, _vp]),
     "rlx_mi355x_gguf_matmul_prepare": (_i, [_vp, _i, _i, _i64, _i64, _vp, _sz, _vp]),
     "rlx_mi355x_gguf_matmul_bt_prepared": (_i, [_vp, _sz, _i, _pvp, _pvp, _i, _i64, _vp]),

@@ -197,9 +197,14 @@ constexpr int ARGMAX_MAX_WGS = 4096;  // keys in the tied-LM-head scratch: one p
 // div_by() of kernels/gemv.hip
 static uint32_t div_magic(uint32_t d) { return d <= 1 ? 0u : (uint32_t)(((1ull << 32) + d - 1) / d); }
 
-static int launch_gemv(const void *const *xs, int xk, const rlx_qweight *const *ws, float *const *outs, int count, int m,
-                       hipStream_t stream, const float *expert_idx = nullptr, unsigned long long *argmax_key = nullptr,
-                       const rlx_qweight *const *pairs = nullptr, const RmsNorm *norm = nullptr, int *wgs_out = nullptr) {
+struct GemvLaunch {
+    KernelId kernel;
+    GemvArgs a;
+    int wgs, waves;
+    size_t lds;
+};
+static int plan_gemv(const void *const *xs, int xk, const rlx_qweight *const *ws, float *const *outs, int count, int m, const float *expert_idx,
+                     unsigned long long *argmax_key, const rlx_qweight *const *pairs, const RmsNorm *norm, GemvLaunch &out) {
     const int scheme = ws[0]->scheme;
     const Layout L = ws[0]->layout;
     for (int i = 0; i < count; i++) {
@@ -250,12 +255,20 @@ static int launch_gemv(const void *const *xs, int xk, const rlx_qweight *const *
     int order[GEMV_MAX_SEG];
     for (int i = 0; i < count; i++) order[i] = i;
     std::stable_sort(order, order + count, [&](int a, int b) { return ws[a]->dims.units < ws[b]->dims.units; });
-    const int cus = std::max(1, device_props().cu_count);
+    const int cus = device_props().cu_count > 0 ? device_props().cu_count : 256;  // (none opened: a plan query)
     const size_t slot_bytes = (size_t)ng * 256;
     auto stage_bytes = [&](int kcu) {
         size_t b = ((size_t)rv * ((size_t)kcu * L.unit_k + 8) * 2 + 15) & ~(size_t)15;
         if (r2 && (scheme == SCHEME_Q4K || scheme == SCHEME_Q5K)) b += (size_t)kcu * (L.unit_k / 32) * 16 * 4;  // block sums
         return b;
+    };
+    // Two K units per loop item halve the per-item bookkeeping; every chunk of every segment must then hold an even number of units, and
+    // every wave still needs an item.
+    static const bool env_u1 = getenv("RLX_GEMV_UPI") && atoi(getenv("RLX_GEMV_UPI")) == 1;
+    auto two_units = [&](int nwaves) {
+        bool ok = family == K_GEMV_Q4_0_R2 && rg == 1 && !env_u1 && nwaves * 2 <= max_units;
+        for (int i = 0; i < count; i++) ok = ok && ws[i]->dims.units % 2 == 0;
+        return ok;
     };
     // A launch shape: `wgs_per_cu` workgroups of `waves` waves per CU, every one resident at once, each with the same
     // number of (tile, unit) items (a segment with a longer K gets fewer row tiles per workgroup), LDS split between
@@ -306,12 +319,27 @@ static int launch_gemv(const void *const *xs, int xk, const rlx_qweight *const *
         // the RMSNorm prologue (GEMV_LDS_TAIL in kernels/gemv.hip)
         constexpr size_t LDS_TAIL = 384;
         while (sh.kcu > 1 && part_bytes + stage_bytes(sh.kcu) + LDS_TAIL > budget) sh.kcu--;
-        // Where the staging of a chunk is even over the waves (8 f32 or 16 sixteen-bit rows on sixteen of them, 16 f32 rows on eight), so are
-        // its units: 17 units leave fifteen waves waiting for one, chunk after chunk. us, Q4_0 / Q8_0 / Q4_K / Q5_K: [4096, 14336], 8 f32
-        // rows 22.2 / 24.8 / 24.7 / 27.4 -> 20.3 / 23.8 / 22.4 / 25.0, [8192, 28672] 47.1 / 57.4 / 55.2 / 65.8 -> 43.2 / 55.1 / 51.0 / 59.5; 16 f32 rows
-        // 91 / 97 -> 79 / 84 there (Q4_0, Q8_0). With other row counts the waves' shares of the staging differ, which uneven units happen to make up for:
-        // 5 - 7 and 10 f32 rows 3 - 20 % slower, 12 16-bit rows 8 %.
-        if ((rv == 16 || (xk == 0 && m == 16)) && sh.kcu < max_units && sh.kcu > kw) sh.kcu -= sh.kcu % kw;
+        // A chunk of 17 units leaves fifteen of sixteen waves waiting for one, chunk after chunk: it is cut to whole rounds of a tile's waves
+        // (of their two-unit items, or at least of units) where that takes at most a fifth of it and no chunk more, or a sixteenth and
+        // at most a quarter more chunks. 2650 launches of more than one chunk (six schemes, twenty matrices of 7168 - 28672 columns,
+        // 1 - 16 f32 and 1 - 32 bf16 rows): 1150 change, 1.04 times as fast on average, 0.967 at worst, 1.25 at best; cut wherever that
+        // takes more chunks, 0.96 on average and 0.74 at worst. us, as many as fit / cut: [4096, 14336] Q4_0, 8 f32 rows, 34 -> 32
+        // units 22.2 / 20.3; 5 rows, 57 -> 48, a third chunk, 15.0 / 16.2; [8192, 28672] Q4_0, 16 rows, 17 -> 16 91 / 79.
+        if (sh.kcu < max_units) {
+            auto chunks = [&](int kcu) {
+                int c = 0;
+                for (int i = 0; i < count; i++) c += ((int)ws[i]->dims.units + kcu - 1) / kcu;
+                return c;
+            };
+            for (int step : {two_units(sh.nwaves) ? 2 * kw : kw, kw}) {
+                const int cut = sh.kcu % step;
+                if (cut == sh.kcu) continue;
+                const int now = chunks(sh.kcu), more = chunks(sh.kcu - cut) - now;
+                if (cut * (more > 0 ? 16 : 5) > sh.kcu || more * 4 > now) continue;
+                sh.kcu -= cut;
+                break;
+            }
+        }
         sh.fits = part_bytes + stage_bytes(sh.kcu) + LDS_TAIL <= budget;
         sh.lds = part_bytes + stage_bytes(sh.kcu) + LDS_TAIL;
         sh.a.nseg = count;
@@ -369,21 +397,22 @@ static int launch_gemv(const void *const *xs, int xk, const rlx_qweight *const *
         set_error("gemv: one K unit of %d activation rows does not fit LDS", rv);
         return RLX_ERR_INVALID;
     }
-    // Two K units per loop item halve the per-item bookkeeping; every chunk of every segment must then hold an even
-    // number of units, and every wave still needs an item.
-    static const bool env_u1 = getenv("RLX_GEMV_UPI") && atoi(getenv("RLX_GEMV_UPI")) == 1;
-    if (family == K_GEMV_Q4_0_R2 && rg == 1 && !env_u1 && sh.kcu % 2 == 0 && sh.nwaves * 2 <= max_units) {
-        bool even = true;
-        for (int i = 0; i < count; i++) even = even && ws[i]->dims.units % 2 == 0;
-        if (even) id = (KernelId)(K_GEMV_Q4_0_U2_R2 + variant);
-    }
+    if (two_units(sh.nwaves) && sh.kcu % 2 == 0) id = (KernelId)(K_GEMV_Q4_0_U2_R2 + variant);
     if (argmax_key && sh.wg > ARGMAX_MAX_WGS) {
         set_error("gemv: %d workgroups are more than the argmax key scratch holds (%d)", sh.wg, ARGMAX_MAX_WGS);
         return RLX_ERR_UNSUPPORTED;
     }
-    if (wgs_out) *wgs_out = sh.wg;
-    void *params[] = {&sh.a};
-    return launch(id, (unsigned)sh.wg, 1, (unsigned)sh.nwaves * 64, (unsigned)sh.lds, stream, params);
+    out = GemvLaunch{id, sh.a, sh.wg, sh.nwaves, sh.lds};
+    return RLX_OK;
+}
+static int launch_gemv(const void *const *xs, int xk, const rlx_qweight *const *ws, float *const *outs, int count, int m,
+                       hipStream_t stream, const float *expert_idx = nullptr, unsigned long long *argmax_key = nullptr,
+                       const rlx_qweight *const *pairs = nullptr, const RmsNorm *norm = nullptr, int *wgs_out = nullptr) {
+    GemvLaunch g;
+    RLX_TRY(plan_gemv(xs, xk, ws, outs, count, m, expert_idx, argmax_key, pairs, norm, g));
+    if (wgs_out) *wgs_out = g.wgs;
+    void *params[] = {&g.a};
+    return launch(g.kernel, (unsigned)g.wgs, 1, (unsigned)g.waves * 64, (unsigned)g.lds, stream, params);
 }
 
 // How K is cut across workgroups when the output tiles alone would leave most of the chip idle: `split` slices of
@@ -936,6 +965,33 @@ int rlx_mi355x_gguf_matmul_plan(int scheme, int x_dtype, int64_t m, int64_t k, c
         i += c;
     }
     return launches;
+}
+
+int rlx_mi355x_gguf_decode_plan(int scheme, int x_dtype, int64_t m, int64_t k, const int64_t *ns, int count, char *buf, size_t cap) {
+    using namespace rlx;
+    const int xk = x_kind(x_dtype);
+    bool ok = ns && count > 0 && count <= GEMV_MAX_SEG && xk >= 0 && m > 0 && k > 0 && layout_of(scheme).unit_k != 0 && m <= decode_rows(xk);
+    for (int i = 0; ok && i < count; i++) ok = ns[i] > 0;
+    if (!ok) {
+        set_error("gguf_decode_plan: needs a claimed scheme, F32 / BF16 / F16 activations, sizes above zero, up to %d matrices and a decode batch", GEMV_MAX_SEG);
+        return RLX_ERR_INVALID;
+    }
+    rlx_qweight w[GEMV_MAX_SEG];
+    const rlx_qweight *ws[GEMV_MAX_SEG];
+    const void *xs[GEMV_MAX_SEG] = {};
+    float *outs[GEMV_MAX_SEG] = {};
+    const int kernels = kernel_scheme(scheme);  // as a weight of this scheme is kept
+    for (int i = 0; i < count; i++) {
+        w[i] = rlx_qweight{kernels, layout_of(scheme), weight_dims(scheme, ns[i], k), nullptr, false, 1, 0};
+        ws[i] = &w[i];
+    }
+    GemvLaunch g;
+    RLX_TRY(plan_gemv(xs, xk, ws, outs, count, (int)m, nullptr, nullptr, nullptr, nullptr, g));
+    if (buf && cap) {
+        snprintf(buf, cap, "%s: %d workgroups, %d waves, %d on a tile, up to %d tiles, chunks of %d units", kernel_name(g.kernel), g.wgs, g.waves, g.a.kw,
+                 g.a.max_tiles_per_wg, g.a.kc_units);
+    }
+    return RLX_OK;
 }
 
 int rlx_mi355x_gguf_matmul_bt_batch(const void *const *xs_dev, int x_dtype, const rlx_qweight *const *ws,

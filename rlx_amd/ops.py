@@ -176,6 +176,13 @@ def matmul_plan(scheme, x_dtype, m, k, ns, workspace_bytes=None):
     return want.value, text.value.decode().splitlines()
 
 
+def decode_plan(scheme, x_dtype, m, k, ns):
+    """One decode launch of up to eight [n, k] matrices on x[m, k], as a line of text (kernel, workgroups, waves, tiles, chunks of K)."""
+    text, arr = C.create_string_buffer(256), (C.c_int64 * len(ns))(*ns)
+    _lib.check(_lib.lib().rlx_mi355x_gguf_decode_plan(int(scheme), int(x_dtype), m, k, arr, len(ns), text, len(text)))
+    return text.value.decode()
+
+
 def gguf_matmul_bt_device(x_dev, x_dtype, w: QWeight, out_dev, m, stream=None, workspace=None):
     """out_dev[m, n] = x_dev[m, k] . W^T on `stream`. `workspace`: DeviceBuffer of matmul_workspace_bytes() (prefill only)."""
     need = matmul_workspace_bytes(w, x_dtype, m)

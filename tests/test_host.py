@@ -284,6 +284,32 @@ def test_plan_takes_the_way_that_was_measured_faster(scheme, x_dtype, m, k, ns, 
     assert ops.matmul_plan(scheme, x_dtype, m, k, ns)[1][0].startswith(faster)
 
 
+@pytest.mark.parametrize("scheme,x_dtype,m,k,ns,plan", [
+    # cut to whole rounds of the waves on a tile: 34 units fit, 57, 17, 98; of their two-unit items, where 34 are even already
+    (QuantScheme.GgufQ4_0, DType.F32, 8, 14336, [4096], "rlx_gemv_q4_0_u2_r4: 256 workgroups, 16 waves, 16 on a tile, up to 1 tiles, chunks of 32 units"),
+    (QuantScheme.GgufQ4_0, DType.F32, 5, 28672, [8192], "rlx_gemv_q4_0_u2_r4: 256 workgroups, 16 waves, 8 on a tile, up to 2 tiles, chunks of 56 units"),
+    (QuantScheme.GgufQ8_0, DType.F32, 16, 28672, [8192], "rlx_gemv_q8_0_g2: 256 workgroups, 8 waves, 4 on a tile, up to 2 tiles, chunks of 16 units"),
+    (QuantScheme.GgufQ4_0, DType.BF16, 6, 14336, [4096], "rlx_gemv_q4_0_u2_r4: 256 workgroups, 16 waves, 16 on a tile, up to 1 tiles, chunks of 96 units"),
+    (QuantScheme.GgufQ4_0, DType.BF16, 16, 8192, [28672], "rlx_gemv_q4_0_u2_r4: 224 workgroups, 16 waves, 2 on a tile, up to 8 tiles, chunks of 32 units"),
+    (QuantScheme.GgufQ4_0, DType.F32, 16, 25344, [542], "rlx_gemv_q4_0_g2: 34 workgroups, 8 waves, 8 on a tile, up to 1 tiles, chunks of 16 units"),
+    # as many as fit where there would be many more chunks (4 -> 7, 2 -> 4), or a chunk would lose more than a fifth (28 -> 16)
+    (QuantScheme.GgufQ4_0, DType.F32, 8, 14336, [6144], "rlx_gemv_q4_0_u2_r4: 192 workgroups, 16 waves, 16 on a tile, up to 2 tiles, chunks of 30 units"),
+    (QuantScheme.GgufQ4K, DType.F32, 5, 14336, [4096], "rlx_gemv_q4_k_r4: 256 workgroups, 16 waves, 16 on a tile, up to 1 tiles, chunks of 28 units"),
+    (QuantScheme.GgufQ4K, DType.F32, 5, 8192, [4096], "rlx_gemv_q4_k_r4: 256 workgroups, 16 waves, 16 on a tile, up to 1 tiles, chunks of 28 units"),
+    # one chunk: nothing to cut
+    (QuantScheme.GgufQ4K, DType.F32, 1, 4096, [4096, 1024, 1024], "rlx_gemv_q4_k_r2: 384 workgroups, 8 waves, 8 on a tile, up to 1 tiles, chunks of 16 units"),
+])
+def test_decode_chunks_hold_whole_rounds(scheme, x_dtype, m, k, ns, plan):
+    assert ops.decode_plan(scheme, x_dtype, m, k, ns) == plan
+
+
+def test_decode_plan_refuses_what_has_no_decode_launch():
+    for args in [(QuantScheme.GgufQ4_0, DType.F32, 17, 256, [16]), (QuantScheme.GgufQ4_0, DType.F32, 1, 256, [0]), (QuantScheme.GgufQ4_0, DType.F32, 1, 256, []),
+                 (QuantScheme.GgufQ4_0, DType.F32, 1, 256, [16] * 9), (QuantScheme.GgufQ4_0, DType.U8, 1, 256, [16])]:
+        with pytest.raises(rlx_amd.RlxError):
+            ops.decode_plan(*args)
+
+
 def test_matmul_plan_refuses_what_has_no_launch():
     for args in [(QuantScheme.GgufQ4_0, DType.F32, 0, 256, [16]), (QuantScheme.GgufQ4_0, DType.F32, 64, 256, [0]), (QuantScheme.GgufQ4_0, DType.F32, 64, 256, []),
                  (QuantScheme.GgufQ4K, DType.I8, 64, 256, [16]), (QuantScheme.GgufQ4_0, DType.U8, 64, 256, [16])]:

@@ -497,3 +497,25 @@ def test_chunks_of_whole_rounds(scheme, m, dtype, k, n):
     # code and min terms are each up to four times their difference.
     assert np.max(np.abs(got - want)) <= (7.2e-6 if scheme == Q4K else 1.8e-6) * np.max(np.abs(want))
     w.free()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("scheme", [Q4_0, Q8_0, Q4K])
+def test_chunks_of_several_tiles(scheme):
+    """Several chunks of K where a workgroup has several tiles and few of its waves share one: whole rounds, and as many units as fit."""
+    n, k = 7000, 6144
+    rng = np.random.default_rng(9)
+    p = ops.quantize(QuantScheme(scheme), (rng.standard_normal(n * k) * 0.02).astype(np.float32))
+    weight = oracle.dequant(scheme, p, n * k).reshape(n, k).astype(np.float64)
+    w = ops.QWeight(QuantScheme(scheme), p, n, k)
+    for m, dtype in ((7, DType.F32), (8, DType.F32), (13, DType.F32), (16, DType.F32), (12, DType.BF16), (16, DType.BF16), (31, DType.BF16)):
+        plan = ops.decode_plan(scheme, dtype, m, k, [n])
+        assert int(plan.split("up to ")[1].split()[0]) > 1 and " 16 on a tile" not in plan and int(plan.split("chunks of ")[1].split()[0]) < k // (256 if scheme == Q4K else 128), plan
+        x = rng.standard_normal((m, k)).astype(np.float32)
+        if dtype == DType.BF16:
+            x = (x.view(np.uint32) & np.uint32(0xFFFF0000)).view(np.float32)
+        got = ops.gguf_matmul_bt((x.view(np.uint32) >> 16).astype(np.uint16) if dtype == DType.BF16 else x, w, m, dtype)
+        want = x.astype(np.float64) @ weight.T
+        # as above, with k / 32 = 192 block sums
+        assert np.max(np.abs(got - want)) <= (3.4e-6 if scheme == Q4K else 0.85e-6) * np.max(np.abs(want)), (m, dtype)
+    w.free()
