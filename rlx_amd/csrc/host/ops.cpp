@@ -1265,11 +1265,15 @@ int rlx_mi355x_rms_norm(const float *x_dev, const float *gamma_dev, const float 
     RowOpArgs a{x_dev, gamma_dev, beta_dev, out_dev, rows, h, eps, 0, 0};
     a.vec4 = h % 4 == 0 && ((uintptr_t)x_dev | (uintptr_t)gamma_dev | (uintptr_t)beta_dev | (uintptr_t)out_dev) % 16 == 0;
     void *params[] = {&a};
-    // Rows that up to 1024 threads can hold, four 16-byte groups each (ROW_KEEP in kernels/rowops.hip): as few threads as do, so that the
-    // rows of a prompt are on the chip at once. us, read twice against kept: 1111 rows of 4096 9.3 / 6.8, 4096 rows of 4096 26.0 / 21.0,
-    // 2000 of 16384 54 / 48; 8192 rows of 2048 22.0 / 21.9, 1111 of 1024 4.0 / 4.3 (most of the four groups past the end).
-    const bool keep = a.vec4 && h > 2048 && h <= 16384;
-    const unsigned bx = keep ? (h <= 4096 ? 256 : h <= 8192 ? 512 : 1024) : h >= 4096 ? 1024 : 256;
+    // Rows that up to 1024 threads can hold, four 16-byte groups each (ROW_KEEP in kernels/rowops.hip), on as few threads as do, so that
+    // the rows of a prompt are on the chip at once. us, read twice / kept, three buffers in turn: 1111 rows of 4096 10.5 / 8.4, 4096 rows
+    // of 4096 33.8 / 27.3, 1500 of 2052 7.5 / 7.0 (on 256 threads 7.9), 2000 of 16384 63.7 / 58.8; rows of 2048 and less are no faster
+    // kept. Between 8192 and 16384 columns 1024 threads hold more than there is, and with 85 registers a CU has room for one such
+    // workgroup: kept pays where a row has a CU to itself (64 rows of 10240 4.6 / 4.3; 300 rows 8.1 / 9.4) and, the fuller the
+    // threads, the earlier again where there are many rows (12288: 1111 rows 27.0 / 28.2, 1500 34.8 / 32.6; 15360: 700 rows 20.2 / 20.4, 1024 32.4 / 30.3).
+    const int64_t kept_from = h <= 8192 || h >= 16000 ? 0 : h >= 15000 ? 900 : h >= 12000 ? 1400 : INT64_MAX;
+    const bool keep = a.vec4 && h > 2048 && h <= 16384 && (rows <= 256 || rows >= kept_from);
+    const unsigned bx = keep ? (h <= 3072 ? 192 : h <= 4096 ? 256 : h <= 8192 ? 512 : 1024) : h >= 4096 ? 1024 : 256;
     return launch(keep ? K_RMSNORM_ROWS_KEEP : K_RMSNORM_ROWS, (unsigned)std::min<int64_t>(rows, 1 << 20), 1, bx, 0, (hipStream_t)stream, params);
 }
 

@@ -172,3 +172,15 @@ def test_rms_norm_rows_kept_in_registers(h, rows, with_beta):
     want = x64 / np.sqrt((x64 ** 2).mean(axis=1, keepdims=True) + 1e-5) * gamma + (0 if beta is None else beta)
     # per thread at most 64 additions of squares, then a tree: the factor is good to 32 ulp, the element itself adds four roundings
     assert np.max(np.abs(got - want) / np.maximum(np.abs(want), 1.0)) <= 36 * 2.0 ** -24
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows,h", [(300, 3072), (300, 3076), (256, 10240), (257, 10240), (1400, 11996), (1399, 12000), (1400, 12000), (900, 14996), (899, 15000), (900, 15000), (257, 15996), (257, 16000)])
+def test_rms_norm_rows_around_the_dispatch(rows, h):
+    """Both sides of the lines between rows kept in registers, on three sizes of workgroup, and rows read twice."""
+    rng = np.random.default_rng(h + rows)
+    x = (rng.standard_normal((rows, h), dtype=np.float32) * 3)
+    gamma = rng.standard_normal(h).astype(np.float32)
+    got = ops.rms_norm(x, gamma, None, 1e-5)
+    want = x / np.sqrt((x.astype(np.float64) ** 2).mean(axis=1, keepdims=True) + 1e-5) * gamma
+    assert np.max(np.abs(got - want) / np.maximum(np.abs(want), 1.0)) <= 36 * 2.0 ** -24  # as above
