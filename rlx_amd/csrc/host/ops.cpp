@@ -477,12 +477,14 @@ static GemmSplit wide_split(const Layout &L, const WeightDims &D, int64_t m, siz
 // The 256 x 256 tiles of kernels/gemm_big.hip (Q4_0, Q8_0, code images) against the 256 x 128 tiles of kernels/gemm.hip, and how the
 // former are handed out: a tile per workgroup, or the whole line of (tile, 128 columns of K) items in equal runs, one per CU, with
 // the pieces of shared tiles added by a launch of their own. `groups` = 0: the 256 x 128 tiles. Estimated times decide. Their constants,
-// in us, are fitted to 1740 random shapes (130 - 8192 image rows, K 512 - 28672, one to four matrices), each timed all three ways, for
-// f32 rows, 16-bit rows and code images apart: these differ in the bytes of a piece and in what a tile's columns cost (no decode on
-// code images). The whole call is 1.06, 1.03 and 1.13 times as fast there as with the smaller tiles on average (1.4 at best, 0.94 at
-// worst) and within 1 % of the fastest of the three on average; against the constants fitted to an epilogue that was twice as long
-// 1.013, 1.008 and 1.005 (1.2 at best, 0.96 at worst). Some of them, smaller / whole / shared: f32 [528, 6944] x 3426 102 / 186 / 94 (the estimate
-// stays with the smaller ones here); bf16 [1424, 8416] x 2794 126 / 230 / 116; codes [3763, 6432] x 2598 276 / 203 / 274, [3138, 6720] x 5014 364 / 362 / 302.
+// in us, are free parameters of a fit: what they are named after is what they stand for, not what it measures alone. Fitted to 1180, 1140
+// and 1080 random launches of f32 rows, 16-bit rows and code images whose rows are whole groups of four columns and half as many of
+// other lengths (97 - 8192 rows, K 256 - 28672, one to four matrices), each timed all three ways. On 330, 320 and 345 others of the
+// former kind, which the fit has not seen, the whole call takes 1.001, 1.003 and 1.003 times the fastest of the three ways on
+// average (1.05, 1.11 and 1.11 at worst) and is 1.02, 1.01 and 1.04 times as fast as with the smaller tiles alone; on 167, 162 and 136 of
+// the latter 1.002, 1.001 and 1.009 (1.06, 1.08, 1.38) and 1.02, 1.08, 1.08. Some, smaller / whole / shared: f32 [528, 6944] x 3426
+// 107 / 188 / 101, [1111, 4096] x 28672 551 / 519 / 529, [417, 256] x 288 14.6 / 23.4 / -; bf16 [1424, 8416] x 2794 129 / 224 / 121; codes
+// [3763, 6432] x 2598 212 / 163 / 219, [3138, 6720] x 5014 323 / 301 / 246.
 // Shared tiles of one row of A are at the same K at the same time, and read A together, where their workgroups, 256 / tiles_n apart, are
 // a whole number apart: gcd(tiles_n, 256) at a time. Alone, each reads A by itself: the kernel on code images of 22 x 12 tiles of 6912
 // columns 212 us, of 24 x 11 tiles 305. Packed weights, whose bytes are a quarter or half, feel it less.
@@ -495,16 +497,18 @@ struct BigCosts {
     double half_idle;                  // share of it that a last round takes however few its tiles are
     double split_start, split_byte;    // a split of K on top: its reduce launch, its partial results per byte
     double whole_start, whole_quad;    // a round of whole 256 x 256 tiles
-    double shared_start, shared_quad;  // shared tiles: two ways in and out of a tile and the reduce launch; every 128 columns of a run
+    double shared_start, shared_quad;  // shared tiles: the pieces, written and added by the reduce launch; every 128 columns of a run (each whole tile in it starts too)
     double alone, pairs;               // added share of the latter where A is read by one workgroup or two at a time
     double sparse_margin;              // shared tiles against a grid that is not full: the estimate's error there
+    double half_word;                  // a result that the 256 x 128 tiles store as a single word (rows that are no multiple of four long)
 };
-constexpr BigCosts BIG_COSTS_F32{0, 1.64, 0.96, 6.5, 7e-8, 1.48, 3.024, 37.4, 2.792, 0.148, 0.14, 0.998};
-constexpr BigCosts BIG_COSTS_16{0.8, 1.83, 0.85, 6.3, 3.4e-7, 6.51, 3.285, 45.3, 3.455, 0.085, 0.021, 0.999};
-constexpr BigCosts BIG_COSTS_CODES{3.8, 1.485, 0.737, 4.5, 1.2e-7, 9.822, 1.734, 27.032, 2.271, 0.502, 0.192, 0.985};
-constexpr double IMG_START = 5.5, IMG_QUAD = 2.3;  // a round of rlx_gemm_img_f16w, every 128 columns of it
+constexpr BigCosts BIG_COSTS_F32{0, 1.64, 0.96, 4.91, 0, 4.09, 2.929, 28.2, 2.838, 0.024, 0.016, 0.917, 8.7e-7};
+constexpr BigCosts BIG_COSTS_16{0.8, 1.83, 0.85, 4.17, 3e-7, 6.17, 3.143, 53, 3.022, 0.073, 0.042, 0.99, 1.35e-6};
+constexpr BigCosts BIG_COSTS_CODES{3.8, 1.485, 0.737, 5.13, 1.7e-7, 9.54, 1.815, 36.6, 2.056, 0.8, 0.21, 0.943, 1.25e-6};
+constexpr double IMG_START = 4.31, IMG_QUAD = 2.49;  // a round of rlx_gemm_img_f16w, every 128 columns of it
 constexpr int64_t IMG_MAX_K = 2304;              // up to here rlx_gemm_img_f16w instead of rlx_gemm_big_f16w: its way in and out of a tile is shorter (kernels/gemm.hip)
-static BigPlan big_plan(int scheme, int xk, int64_t m, int64_t m_rows, int64_t tiles_n, int64_t half_tiles_n, int64_t n_sum, int64_t quads, size_t part_room) {
+static BigPlan big_plan(int scheme, int xk, int64_t m, int64_t m_rows, int64_t tiles_n, int64_t half_tiles_n, int64_t n_sum, int64_t n_words, int64_t quads,
+                        const GemmSplit &sp, int64_t slice_quads, size_t part_room) {
     BigPlan none{0, 0};
     if (scheme != SCHEME_Q4_0 && scheme != SCHEME_Q8_0) return none;
     const bool codes = xk == XK_CODES;
@@ -515,23 +519,22 @@ static BigPlan big_plan(int scheme, int xk, int64_t m, int64_t m_rows, int64_t t
     // code images run whole tiles from two rounds on in any case ([8192, 4096] x [4096, 4096] 310 -> 282 us; half tiles 14 % slower at K = 1024)
     if (codes && tiles >= 2 * cus) return BigPlan{(int)tiles, 0};
     const bool sparse = half * 5 < cus * 4;  // where gemm_split cuts K if two slices or more find a CU each
-    const long long split = sparse ? std::min<long long>(quads, cus / half) : 1;
     double t_half;
-    if (split > 1) {
-        t_half = c.half_start + (double)((quads + split - 1) / split) * c.half_quad + c.split_start + c.split_byte * 4.0 * (double)split * (double)m * (double)n_sum;
+    if (sp.split > 1) {
+        t_half = c.half_start + (double)slice_quads * c.half_quad + c.split_start + c.split_byte * 4.0 * (double)sp.split * (double)m * (double)n_sum;
     } else {
         const double last = (double)(half - cus * (rounds(half) - 1)) / (double)cus;
-        t_half = ((double)(rounds(half) - 1) + c.half_idle + (1 - c.half_idle) * last) * (c.half_start + (double)quads * c.half_quad);
+        t_half = ((double)(rounds(half) - 1) + c.half_idle + (1 - c.half_idle) * last) * (c.half_start + (double)quads * c.half_quad) +
+                 c.half_word * (double)m * (double)n_words;
     }
     const double t_whole = (double)rounds(tiles) * (codes && quads * 128 <= IMG_MAX_K ? IMG_START + (double)quads * IMG_QUAD : c.whole_start + (double)quads * c.whole_quad);
     const bool whole = t_whole < t_half;
     const size_t part = (size_t)cus * 2 * (size_t)(xk == 0 ? 128 : 256) * 1024;  // a workgroup leaves at most two pieces
     if (part <= part_room && tiles * quads >= cus) {
         const double quad = c.shared_quad * (1 + (tiles_n % 2 ? c.alone : tiles_n % 4 ? c.pairs : 0));
-        // From three rounds of whole tiles on there is little left to fill, and the estimates are within a few percent of each other:
-        // f32 [1111, 4096] x 28672, 3.94 rounds, layer 1059 us shared, 1052 whole.
-        const double margin = sparse ? c.sparse_margin : whole && rounds(tiles) > 2 ? 0.97 : 1;
-        if (c.shared_start + (double)rounds(tiles * quads) * quad < margin * (whole ? t_whole : t_half)) return BigPlan{(int)cus, part};
+        const double margin = sparse ? c.sparse_margin : 1;
+        const double t_shared = c.shared_start + (double)tiles / (double)cus * c.whole_start + (double)rounds(tiles * quads) * quad;
+        if (t_shared < margin * (whole ? t_whole : t_half)) return BigPlan{(int)cus, part};
     }
     return whole ? BigPlan{(int)tiles, 0} : none;
 }
@@ -550,9 +553,10 @@ static GemmLaunch launch_plan(int scheme, int xk, int64_t m, int64_t k, const in
     const bool codes = xk == XK_CODES, skinny = gemm_skinny(xk, m);
     const Layout L = codes ? Layout{64, 0, 0, 0, 0} : layout_of(scheme);
     const int64_t rv = xk == 0 ? 2 * m : m, m_rows = (rv + 255) / 256 * 256, k_pad = (k + 255) / 256 * 256;
-    int64_t n_sum = 0, tiles_n = 0, half_tiles_n = 0;
+    int64_t n_sum = 0, n_words = 0, tiles_n = 0, half_tiles_n = 0;
     for (int i = 0; i < count; i++) {
         n_sum += ns[i];
+        n_words += ns[i] % 4 ? ns[i] : 0;
         tiles_n += (ns[i] + 255) / 256;
         half_tiles_n += (ns[i] + 127) / 128;
     }
@@ -574,7 +578,10 @@ static GemmLaunch launch_plan(int scheme, int xk, int64_t m, int64_t k, const in
     }
     if (!skinny) {
         const int64_t quads = codes ? k_pad / 128 : (k + L.unit_k - 1) / L.unit_k;
-        const BigPlan bp = big_plan(scheme, xk, m, m_rows, tiles_n, half_tiles_n, n_sum, quads, part_room);
+        // the 256 x 128 tiles' slices of K, were there room for all of them
+        const GemmSplit sp = gemm_split(half_tiles_n, m_rows / 256, codes ? k_pad / 64 : quads, L.unit_k / 64, false);
+        const int64_t slice_quads = std::min<int64_t>(quads, (int64_t)sp.units_per_split * L.unit_k / 128);
+        const BigPlan bp = big_plan(scheme, xk, m, m_rows, tiles_n, half_tiles_n, n_sum, n_words, quads, sp, slice_quads, part_room);
         if (bp.groups) {
             g.shared = bp.part_bytes > 0;
             g.groups = bp.groups;

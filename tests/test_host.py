@@ -271,14 +271,17 @@ def test_plan_step_workspace_follows_the_launches(scheme, m, k, ns):
 
 @pytest.mark.parametrize("scheme,x_dtype,m,k,ns,faster", [
     # whole calls in us: 256 x 128 tiles / whole 256 x 256 tiles / shared ones
-    (QuantScheme.GgufQ8_0, DType.F32, 2565, 3488, [3155, 3174], "rlx_gemm_q8_0"),               # 305 / 340 / 323
-    (QuantScheme.GgufQ4_0, DType.F32, 1357, 2848, [8523, 5712, 9088, 488], "rlx_gemm_q4_0"),    # 436 / 464 / 455
-    (QuantScheme.GgufQ4_0, DType.F32, 528, 6944, [3426], "rlx_gemm_q4_0"),                      # 102 / 190 / 112, K split
-    (QuantScheme.GgufQ4_0, DType.F32, 1111, 14336, [4096], "rlx_gemm_big_q4_0"),                # 386 / 385 / 272
-    (QuantScheme.GgufQ4_0, DType.BF16, 361, 3904, [2604, 3163, 290, 11691], "rlx_gemm_q4_0"),   # 120 / 126 / 132
-    (QuantScheme.GgufQ8_0, DType.BF16, 1792, 7584, [11351], "rlx_gemm_q8_0"),                   # 376 / 452 / 394
-    (QuantScheme.GgufQ8_0, DType.I8, 1588, 7360, [6223], "rlx_gemm_big_f16w: 1 matrix, whole"),  # 301 / 222 / 309
-    (QuantScheme.GgufQ4_0, DType.I8, 7766, 1856, [6338], "rlx_gemm_img_f16w"),                  # 332 on rlx_gemm_big_f16w, 308 on this
+    (QuantScheme.GgufQ8_0, DType.F32, 2565, 3488, [3155, 3174], "rlx_gemm_big_q8_0: 2 matrices, shared"),              # 314 / 338 / 299
+    (QuantScheme.GgufQ4_0, DType.F32, 1357, 2848, [8523, 5712, 9088, 488], "rlx_gemm_big_q4_0: 4 matrices, shared"),   # 452 / 460 / 422
+    (QuantScheme.GgufQ4_0, DType.F32, 528, 6944, [3426], "rlx_gemm_big_q4_0: 1 matrix, shared"),                       # 107 / 188 / 101, K split on the smaller tiles
+    (QuantScheme.GgufQ4_0, DType.F32, 1111, 14336, [4096], "rlx_gemm_big_q4_0: 1 matrix, shared"),                     # 424 / 407 / 290
+    (QuantScheme.GgufQ4_0, DType.F32, 1111, 4096, [28672], "rlx_gemm_big_q4_0: 1 matrix, whole"),                      # 551 / 519 / 529
+    (QuantScheme.GgufQ4_0, DType.F32, 417, 256, [288], "rlx_gemm_q4_0"),                                               # 14.6 / 23.4, two slices of K would be one
+    (QuantScheme.GgufQ4_0, DType.BF16, 361, 3904, [2604, 3163, 290, 11691], "rlx_gemm_big_q4_0: 4 matrices, whole"),   # 127 / 120 / 115: 4 % from the fastest
+    (QuantScheme.GgufQ8_0, DType.BF16, 1792, 7584, [11351], "rlx_gemm_big_q8_0: 1 matrix, shared"),                    # 386 / 452 / 374
+    (QuantScheme.GgufQ8_0, DType.BF16, 1638, 256, [436, 844], "rlx_gemm_q8_0"),                                        # 18.5 / 27.0
+    (QuantScheme.GgufQ8_0, DType.I8, 1588, 7360, [6223], "rlx_gemm_big_f16w: 1 matrix, whole"),                        # 252 / 194 / 269
+    (QuantScheme.GgufQ4_0, DType.I8, 7766, 1856, [6338], "rlx_gemm_img_f16w"),                                         # 332 on rlx_gemm_big_f16w, 308 on this
 ])
 def test_plan_takes_the_way_that_was_measured_faster(scheme, x_dtype, m, k, ns, faster):
     assert ops.matmul_plan(scheme, x_dtype, m, k, ns)[1][0].startswith(faster)
