@@ -460,7 +460,7 @@ def extra_configs(rlx_amd, stream):
 
         ms_t = time_launches(ops, stream, fn_topk, 200, 20)
         out[f"q4_k_tied_lm_top{cap}_128256x4096"] = {"us": round(ms_t * 1e3, 2), "GB/s": round(b / ms_t / 1e6, 1),
-                                                    "launches": "gemv (logits into scratch) + two (cap 8) or three (cap 40) selection passes, one wave per 1024 candidates"}
+                                                    "launches": "gemv (logits into scratch) + two selection passes: one wave per 1024 candidates, then one wave (cap 8) or workgroup (cap 40)"}
     for q in qws:
         q.free()
     out.update(moe_config(rlx_amd, stream))

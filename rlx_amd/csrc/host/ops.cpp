@@ -497,7 +497,8 @@ struct BigCosts {
     double half_idle;                  // share of it that a last round takes however few its tiles are
     double split_start, split_byte;    // a split of K on top: its reduce launch, its partial results per byte
     double whole_start, whole_quad;    // a round of whole 256 x 256 tiles
-    double shared_start, shared_quad;  // shared tiles: the pieces, written and added by the reduce launch; every 128 columns of a run (each whole tile in it starts too)
+    double shared_start, shared_quad;  // shared tiles: the pieces, written and added by the reduce launch; every 128 columns of a run
+                                       // (whose tiles each take whole_start, too)
     double alone, pairs;               // added share of the latter where A is read by one workgroup or two at a time
     double sparse_margin;              // shared tiles against a grid that is not full: the estimate's error there
     double half_word;                  // a result that the 256 x 128 tiles store as a single word (rows that are no multiple of four long)
@@ -506,7 +507,8 @@ constexpr BigCosts BIG_COSTS_F32{0, 1.64, 0.96, 4.91, 0, 4.09, 2.929, 28.2, 2.83
 constexpr BigCosts BIG_COSTS_16{0.8, 1.83, 0.85, 4.17, 3e-7, 6.17, 3.143, 53, 3.022, 0.073, 0.042, 0.99, 1.35e-6};
 constexpr BigCosts BIG_COSTS_CODES{3.8, 1.485, 0.737, 5.13, 1.7e-7, 9.54, 1.815, 36.6, 2.056, 0.8, 0.21, 0.943, 1.25e-6};
 constexpr double IMG_START = 4.31, IMG_QUAD = 2.49;  // a round of rlx_gemm_img_f16w, every 128 columns of it
-constexpr int64_t IMG_MAX_K = 2304;              // up to here rlx_gemm_img_f16w instead of rlx_gemm_big_f16w: its way in and out of a tile is shorter (kernels/gemm.hip)
+// up to here rlx_gemm_img_f16w instead of rlx_gemm_big_f16w: its way in and out of a tile is shorter (kernels/gemm.hip)
+constexpr int64_t IMG_MAX_K = 2304;
 static BigPlan big_plan(int scheme, int xk, int64_t m, int64_t m_rows, int64_t tiles_n, int64_t half_tiles_n, int64_t n_sum, int64_t n_words, int64_t quads,
                         const GemmSplit &sp, int64_t slice_quads, size_t part_room) {
     BigPlan none{0, 0};

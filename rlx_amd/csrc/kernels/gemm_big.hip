@@ -8,10 +8,12 @@
 //
 // Four waves, one per SIMD, own 128 x 128 of the 256 x 256 tile each (256 accumulator registers): sixteen fragment reads feed 64
 // matrix instructions. K advances in 32-column quanta through a ring of LDS slots that buffer loads fill directly; one barrier per
-// quantum. What bounds it is power: on [8192, 4096] x [4096, 4096] ready images the loop takes 160 K clocks a tile, 19.5 per matrix instruction
-// (16 and a bubble of 2 at best), at the 1.5 - 1.6 GHz that sustained products of drawn data leave of 2.4; 1.0 - 1.1 PFLOP/s. With packed weights decoded in
-// it 26.6 clocks at 1.8 - 2.0 GHz, as much. 16 x 16 x 32 instructions read and write half the accumulator bits per product of 32 x 32 x 16 ones: 210 us
-// against 229 (and 232 for eight waves of 128 x 64 on 32 x 32 x 16, the kernel before).
+// quantum. What bounds it: on [8192, 4096] x [4096, 4096] ready images the loop takes 160 K clocks a tile, 19.5 per matrix instruction (16
+// and a bubble of 2 at best), and the way in and out 20 K: 159 us at the 2.3 GHz it runs at on zeros, 1.73 PFLOP/s. On drawn data the
+// chip draws more and clocks lower: 206 us for one launch after a pause (1.33 PFLOP/s), 199 in a row of a thousand (1.38), 205 - 270
+// for those of a row of sixteen or sixty-four, while the clock settles. With packed weights decoded in it the loop issues for 26.6
+// clocks per matrix instruction, which is what bounds it then. 16 x 16 x 32 instructions read and write half the accumulator bits per
+// product of 32 x 32 x 16 ones: 210 us against 229 (and 232 for eight waves of 128 x 64 on 32 x 32 x 16, the kernel before).
 // An XCD-wise tile order and a ring without address arithmetic (four slots, depth two) measured the same or 2 % slower.
 //
 // Decoding packed weights here costs what writing them out as images first would (about 10 % of the kernel), without 2 bytes per weight
@@ -268,8 +270,8 @@ __device__ __forceinline__ void gemm_big_body(const GemmBigArgs &a) {
         // Epilogue. W is the first operand of the products, so register r of tile (i, j) is row 16 i + lr, column 16 j + 4 lg + r of the
         // wave's quarter: a lane holds four neighbouring columns and stores them as they are, four lanes 64 bytes of a row. With
         // the rows in the registers the wave had to turn its quarter around in LDS first: 41 K clocks of the 205 K of a tile of
-        // [8192, 4096] x [4096, 4096], 17 K now; f32 rows 30 K and 12.5 K (no stores at all: 4 K). The clock that power allows takes
-        // some of it back: 277 -> 262 us, 519 -> 506 on [2222 image rows, 4096] x [28672, 4096]. The rows' factors come through LDS.
+        // [8192, 4096] x [4096, 4096], 17 K now; f32 rows 30 K and 12.5 K (no stores at all: 4 K). A lower clock takes some of it back:
+        // 277 -> 262 us in a row of a few dozen launches, 519 -> 506 on [2222 image rows, 4096] x [28672, 4096]. The rows' factors come through LDS.
         const int rows = a.pair_rows ? 128 : 256;
         float *fac_s = (float *)smem;
         if (tid < rows) {

@@ -128,10 +128,10 @@ extern "C" __global__ __launch_bounds__(64) void rlx_topk_serial(rlx::TopkArgs a
 }
 
 // The bound comes first: the cap-th largest of the 64 lanes' own maxima, one ballot a step. At least cap keys reach it, and few more do
-// (about 62 of 1024 at cap 40 where the values lie in no particular order), so the search for the cap-th largest key counts four keys
-// per lane instead of sixteen: the whole LM-head call at [128256, 4096] Q4_K, cap 40, 67.1 -> 63.2 us with loads
-// that do not wait for each other. Where more survive (long runs of
-// values in descending order) it counts all sixteen.
+// (about 62 of 1024 at cap 40 where the values lie in no particular order, exactly 40 where they rise or fall), so the search for the
+// cap-th largest key counts four keys per lane instead of sixteen: the whole LM-head call at [128256, 4096] Q4_K, cap 40, 67.1 -> 63.2 us
+// with loads that do not wait for each other. Where more than 256 survive (many equal values, or the best ones in fewer lanes than
+// cap: every 64th value belongs to a lane) it counts all sixteen.
 extern "C" __global__ __launch_bounds__(64) void rlx_topk_select(rlx::TopkArgs a) {
     using namespace rlx;
     __shared__ unsigned long long few[TOPK_FEW];
