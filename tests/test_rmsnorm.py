@@ -151,6 +151,25 @@ def test_rmsnorm_swiglu_and_argmax():
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("scheme,m", [(Q4_0, 1), (Q4K, 6)])
+def test_rmsnorm_swiglu_and_argmax_take_rows_of_any_size(scheme, m):
+    """As test_rmsnorm_launch_takes_rows_of_any_size, through the other two epilogues."""
+    rng = np.random.default_rng(8)
+    k, n = 2048, 700
+    x = rng.standard_normal((m, k)).astype(np.float32)
+    gamma = (1.0 + 0.1 * rng.standard_normal(k)).astype(np.float32)
+    up, gate = (ops.QWeight(QuantScheme(scheme), weights(scheme, n, k, 23 + i), n, k) for i in range(2))
+    first = ops.rmsnorm_gguf_matmul_swiglu(x, gamma, None, 0.0, up, gate, m)
+    best = ops.rmsnorm_gguf_tied_lm_argmax(x[0], gamma, None, 0.0, up)
+    for p in (-40, -12, 15, 30):
+        scaled = x * np.float32(2.0 ** p)
+        assert np.array_equal(ops.rmsnorm_gguf_matmul_swiglu(scaled, gamma, None, 0.0, up, gate, m), first), p
+        assert ops.rmsnorm_gguf_tied_lm_argmax(scaled[0], gamma, None, 0.0, up) == best, p
+    up.free()
+    gate.free()
+
+
+@pytest.mark.gpu
 def test_rmsnorm_argument_errors():
     w = ops.QWeight(QuantScheme.GgufQ4_0, weights(Q4_0, 32, 256, 1), 32, 256)
     with pytest.raises(rlx_amd.RlxError, match="decode path"):
