@@ -442,7 +442,7 @@ __device__ __forceinline__ void compute_unit(const UnitRegs<SCHEME> &w, const ha
 // The power of two, from the row's first four columns (norm_prescale), does for the range what the normalization would: x gamma itself
 // is outside what binary16 carries well in rows of small or large activations, and a launch with one such row ran the common and
 // the slow pass, 1.3 to 2 times as long (us, rows of 2^-12: gate / up [14336, 4096] Q4_K, six rows, 44.8; q / k / v of 4096 columns,
-// Q4_0, one row, 16.3; normalized in the staging 25.2 and 11.5; now 22.5 and 8.8). It costs a launch 0.05 - 0.1 us. What is left to
+// Q4_0, one row, 16.3; normalized in the staging 25.2 and 11.5; now 22.1 and 9.0). It costs a launch 0.1 - 0.2 us. What is left to
 // the slow pass: rows whose largest x gamma is 2^15 times those columns or more, or all below 2^-8 of them. It knows the sums and
 // stages the normalized values.
 // A beta (null in most models) has to be added to the normalized value: then the squares are summed first.
