@@ -1,5 +1,7 @@
 """Op::RmsNorm (rlx-cpu/src/thunk.rs:8839-8869) fused into the decode GEMV's activation staging, alone and in front of
 the SwiGLU and LM-head epilogues."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -167,6 +169,38 @@ def test_rmsnorm_swiglu_and_argmax_take_rows_of_any_size(scheme, m):
         assert ops.rmsnorm_gguf_tied_lm_argmax(scaled[0], gamma, None, 0.0, up) == best, p
     up.free()
     gate.free()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,k", [(1, 4096), (6, 2048)])
+def test_rmsnorm_follows_what_the_launch_before_wrote(m, k):
+    """The row's power of two is read through the scalar cache. Launches stand one behind the other on one buffer that
+    a copy on the stream rewrites in between with rows of very different sizes, and nothing is waited for."""
+    rng = np.random.default_rng(9)
+    n = 512
+    gamma = (1.0 + 0.1 * rng.standard_normal(k)).astype(np.float32)
+    w = ops.QWeight(QuantScheme.GgufQ4_0, weights(Q4_0, n, k, 25), n, k)
+    rows = [rng.standard_normal((m, k)).astype(np.float32) for _ in range(3)]
+    want = [ops.rmsnorm_gguf_matmul_bt_batch(x, gamma, None, 0.0, [w], m)[0] for x in rows]
+    L, check = rlx_amd._lib.lib(), rlx_amd._lib.check
+    stream = C.c_void_p()
+    check(L.rlx_mi355x_stream_create(C.byref(stream)))
+    sizes = (0, -30, 25, -12, 40, 14)
+    inputs = {(i, p): ops.DeviceBuffer.from_numpy(x * np.float32(2.0 ** p)) for i, x in enumerate(rows) for p in sizes}
+    slot, gd = ops.DeviceBuffer(m * k * 4), ops.DeviceBuffer.from_numpy(gamma)
+    order = [(int(rng.integers(3)), sizes[int(rng.integers(len(sizes)))]) for _ in range(150)]
+    outs = [ops.DeviceBuffer(m * n * 4) for _ in order]
+    wp = (C.c_void_p * 1)(w.ptr)
+    ops.sync()
+    for key, out in zip(order, outs):
+        check(L.rlx_mi355x_memcpy_d2d(slot.ptr, inputs[key].ptr, m * k * 4, stream))
+        check(L.rlx_mi355x_rmsnorm_gguf_matmul_bt_batch(slot.ptr, gd.ptr, None, 0.0, wp, (C.c_void_p * 1)(out.ptr), 1, m,
+                                                        stream))
+    check(L.rlx_mi355x_stream_sync(stream))
+    for key, out in zip(order, outs):
+        assert np.array_equal(out.to_numpy(np.float32).reshape(m, n), want[key[0]]), key
+    check(L.rlx_mi355x_stream_destroy(stream))
+    w.free()
 
 
 @pytest.mark.gpu
